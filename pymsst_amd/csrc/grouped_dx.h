@@ -27,7 +27,8 @@ template <typename T>
 int launch_uniform_dw(const void* dy, const void* x, void* dw, void* db, int64_t groups, int64_t in_features,
                       int64_t out_features, int64_t rows, hipStream_t stream);
 
-// Whether launch_mask_dz takes this shape (16-bit, H a multiple of 128 or 192, aligned pointers).
+// Whether launch_mask_dz takes this shape (16-bit, H a multiple of 128 or 192, aligned pointers); the
+// caller checks that every band width is a multiple of 4.
 bool mask_dz_supported(int64_t H, int64_t rows, size_t elem, const void* dpre, const void* w, const void* x,
                        const void* dx, int64_t total);
 

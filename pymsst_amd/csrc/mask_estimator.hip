@@ -1146,7 +1146,9 @@ int launch_me_bwd(const void* gout, const void* x, const void* pre, const void* 
     if (rc != PMSST_OK) return rc;
     bool dx_done = false;
     if constexpr (sizeof(T) == 2) {
-      if (mask_dz_supported(H, M, sizeof(T), dpre, weight, x, dx, hm.F)) {
+      // a.vec4: me_dz_kernel moves and masks dpre in whole 8-value K units, so every 2 I_b must be a
+      // multiple of 8 (a mono model's 258-wide last band is not)
+      if (a.vec4 && mask_dz_supported(H, M, sizeof(T), dpre, weight, x, dx, hm.F)) {
         rc = launch_mask_dz<T>(dpre, weight, x, dx, offsets, dim_inputs, hm.NB, M, H, hm.F,
                                input_act == PMSST_ACT_TANH, stream);
         if (rc != PMSST_OK) return rc;

@@ -185,6 +185,28 @@ def test_mask_final_backward_with_tanh_input(hip_ext, dtype):
     assert torch.allclose((dx0.float() * (1 - h.float() ** 2)), dz.float(), rtol=2e-2, atol=2e-2 * dz.abs().max().item())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hidden", [128, 192])
+@pytest.mark.parametrize("dims", [(4, 8, 258, 6), (3, 5, 2, 7, 33)])
+def test_mask_final_tanh_backward_at_widths_not_in_fours(hip_ext, dtype, hidden, dims):
+    """A mono model's widths (2 x 129 bins) and odd ones, at hidden sizes the 16-bit input-gradient
+    kernel takes: its K units of 8 must not reach into the next band's columns."""
+    dn = dt_name(dtype)
+    m, nb = 77, len(dims)
+    g = torch.Generator().manual_seed(31)
+    h = torch.tanh(torch.randn(m, nb, hidden, generator=g)).to(dtype).cuda()
+    ws = [(torch.randn(2 * d, hidden, generator=g) / hidden**0.5).to(dtype) for d in dims]
+    w_all = torch.cat([w.reshape(-1) for w in ws]).cuda()
+    pre = torch.randn(m, 2 * sum(dims), generator=g).to(dtype).cuda()
+    gout = torch.randn(m, sum(dims), generator=g).to(dtype).cuda()
+    dz, db, dw = hip_ext.mask_estimator_final_backward_packed(gout, h, pre, w_all, dims, input_activation="tanh")
+    r_dz, r_db, r_dw = oracle.mask_estimator_final_backward(to_np(gout), to_np(h), to_np(pre), [to_np(w) for w in ws],
+                                                            dims, dn, input_act="tanh", grad_pre_dt=dn)
+    assert_parity(dz, r_dz, dn, "dz", by_index(1))
+    assert_parity(db, r_db, dn, "dbias", by_band(0, [2 * d for d in dims]))
+    assert_parity(dw, np.concatenate([w.reshape(-1) for w in r_dw]), dn, "dW", by_band(0, [2 * d * hidden for d in dims]))
+
+
 @pytest.mark.parametrize("dtype,m,dim", [(torch.float32, 65, 64), (torch.bfloat16, 1032, 192)])
 def test_fused_mask_mlp_autograd_vs_oracle(hip_ext, dtype, m, dim):
     """The whole depth-2 mask MLP through the autograd Function the patch layer uses."""
