@@ -605,7 +605,7 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_kernel(const T* __rest
 // Block = (band, 64-wide input tile, 64-wide output tile); K = the rows, walked in steps of
 // KR = 32 KS rows.  Both operands move as stored (KR rows x 64 columns each
 // per step) into a ring of S LDS stages: x by 4-byte DMA (its rows are only 8-byte aligned), dy
-// by 16-byte DMA; both are read as transposed fragments (ds_read_b64_tr_b16, swz_mn swizzle).
+// by 16-byte DMA; both are read as transposed fragments (ds_read_b64_tr_b16, swz_mn_p swizzle).
 // Wave w moves rows KR/4 w .. + KR/4 - 1 of both tiles.  From the saved input each landed x tile
 // is scaled by inv in LDS (KS 16-byte units per thread, of its own wave's rows; inv of the
 // block's rows sits in LDS in windows of kBdWinRows rows).  Columns past the band or past O are
@@ -707,13 +707,13 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_dma_kernel(
   const int64_t xstride = a.F;
 
   // DMA pieces.  dy instruction t: row kWR wave + 8 t + lane / 8, LDS unit lane % 8 <- unit
-  // (lane % 8) ^ swz_mn(row).  x instruction t: row kWR wave + 2 t + lane / 32, 4-byte word
-  // lane % 32 of the row: LDS unit (lane % 32) / 4 <- unit ((lane % 32) / 4) ^ swz_mn(row).
+  // (lane % 8) ^ swz_mn_p(row).  x instruction t: row kWR wave + 2 t + lane / 32, 4-byte word
+  // lane % 32 of the row: LDS unit (lane % 32) / 4 <- unit ((lane % 32) / 4) ^ swz_mn_p(row).
   uint32_t doff[kDI], doff0[kDI], xoff[kXI], xoff0[kXI];
 #pragma unroll
   for (int t = 0; t < kDI; ++t) {
     const int r = kWR * wave + 8 * t + (lane >> 3);
-    int col = o0 + 8 * ((lane & 7) ^ swz_mn(r));
+    int col = o0 + 8 * ((lane & 7) ^ swz_mn_p<2 * kBdT>(r));
     col = col <= O - 8 ? col : O - 8;
     doff[t] = static_cast<uint32_t>((r * dstride + col) * 2);
     doff0[t] = kbeg + r >= 0 ? doff[t] : static_cast<uint32_t>((-kbeg * dstride + col) * 2);
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_dma_kernel(
 #pragma unroll
   for (int t = 0; t < kXI; ++t) {
     const int r = kWR * wave + 2 * t + (lane >> 5);
-    int i = i0 + 8 * (((lane & 31) >> 2) ^ swz_mn(r)) + 2 * (lane & 3);
+    int i = i0 + 8 * (((lane & 31) >> 2) ^ swz_mn_p<2 * kBdT>(r)) + 2 * (lane & 3);
     i = i <= I - 2 ? i : I - 2;
     xoff[t] = static_cast<uint32_t>((r * xstride + i) * 2);
     xoff0[t] = kbeg + r >= 0 ? xoff[t] : static_cast<uint32_t>((-kbeg * xstride + i) * 2);
@@ -764,8 +764,8 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_dma_kernel(
   uint32_t fa[2], fb[2];
 #pragma unroll
   for (int f = 0; f < 2; ++f) {
-    fa[f] = frag_mn_addr(0, 32 * wr + 16 * f, 2 * kBdT, lane);
-    fb[f] = frag_mn_addr(kTile, 32 * wc + 16 * f, 2 * kBdT, lane);
+    fa[f] = frag_mn_addr_p<2 * kBdT>(0, 32 * wr + 16 * f, lane);
+    fb[f] = frag_mn_addr_p<2 * kBdT>(kTile, 32 * wc + 16 * f, lane);
   }
   f32x4_t acc[2][2], accb[2];
 #pragma unroll

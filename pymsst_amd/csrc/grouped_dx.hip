@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   const int nc = O / 32;
 
   // weight DMA: instruction t (wave t % 4) moves flattened units 64 t + lane of the slab: row
-  // P / kUnits, physical unit P % kUnits <- logical unit (P % kUnits) ^ swz_mn(row) (a permutation
+  // P / kUnits, physical unit P % kUnits <- logical unit (P % kUnits) ^ swz_mn_p(row) (a permutation
   // inside aligned groups of 8 units, so it stays inside the row)
   const int npw = (kInstr - wave + 3) / 4;
   uint32_t gsrc[kMaxPW];
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     const int t = wave + 4 * q;
     const int P = 64 * t + lane;
     const int kr = P / kUnits, pu = P % kUnits;
-    const int u = pu ^ swz_mn(kr);
+    const int u = pu ^ swz_mn_p<2 * I>(kr);
     gsrc[q] = static_cast<uint32_t>((kr * I + 8 * u) * 2);
   }
   const char* wg = reinterpret_cast<const char*>(w + static_cast<int64_t>(g) * O * I);
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
   for (int d = 0; d < DT; ++d) {
     const int col = 16 * d + col0;
-    aoff[d] = static_cast<uint32_t>(kr0 * 2 * I + 16 * ((col >> 3) ^ swz_mn(kr0)) + 2 * (col & 7));
+    aoff[d] = static_cast<uint32_t>(kr0 * 2 * I + 16 * ((col >> 3) ^ swz_mn_p<2 * I>(kr0)) + 2 * (col & 7));
   }
   // B fragment of row tile n: row 16 n + rr of this wave's tile, logical unit gq
   const uint32_t boff = static_cast<uint32_t>(kSlab + wave * NT * 1024 + rr * 64 + 16 * (gq ^ swz_k(rr)));

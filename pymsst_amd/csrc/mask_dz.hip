@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void me_dz_kernel(const T* __restrict__ dpre, 
 
   // weight DMA: instruction t (wave t % 4) moves flattened units 64 t + lane of the slab: row
   // kr = P / kUnits (weight row 32 c + kr, clamped to the band), physical unit P % kUnits <-
-  // logical unit (P % kUnits) ^ swz_mn(kr)
+  // logical unit (P % kUnits) ^ swz_mn_p(kr)
   const int npw = (kInstr - wave + 3) / 4;
   int wrow[kMaxPW], wcol[kMaxPW];
 #pragma unroll
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void me_dz_kernel(const T* __restrict__ dpre, 
     const int P = 64 * t + lane;
     const int kr = P / kUnits, pu = P % kUnits;
     wrow[q] = kr;
-    wcol[q] = h0 + 8 * (pu ^ swz_mn(kr));
+    wcol[q] = h0 + 8 * (pu ^ swz_mn_p<2 * HT>(kr));
   }
   const T* wb = w + static_cast<int64_t>(2) * off * H;
   // dpre DMA: instruction n moves rows wrow0 + 16 n + lane / 4 (clamped), physical unit lane % 4 <-
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void me_dz_kernel(const T* __restrict__ dpre, 
 #pragma unroll
   for (int d = 0; d < DT; ++d) {
     const int col = 16 * d + 4 * (jq & 3);
-    aoff[d] = static_cast<uint32_t>(kr0 * 2 * HT + 16 * ((col >> 3) ^ swz_mn(kr0)) + 2 * (col & 7));
+    aoff[d] = static_cast<uint32_t>(kr0 * 2 * HT + 16 * ((col >> 3) ^ swz_mn_p<2 * HT>(kr0)) + 2 * (col & 7));
   }
   const uint32_t boff = static_cast<uint32_t>(kSlab + wave * NT * 1024 + rr * 64 + 16 * (gq ^ swz_k(rr)));
 

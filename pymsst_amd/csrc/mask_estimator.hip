@@ -609,7 +609,7 @@ __global__ __launch_bounds__(512) void me_bwd_dx_dma_kernel(const T* __restrict_
   const int kbeg = K - nk * kChunkK;  // multiple of 8 (I % 4 == 0)
 
   // DMA pieces of this lane.  Weight instruction t (of 2) of wave w is q = w + NW t: K-rows
-  // (64 / kU) q + lane / kU, unit lane % kU of the row (logical unit ^ swz_mn).  dpre instruction
+  // (64 / kU) q + lane / kU, unit lane % kU of the row (logical unit ^ swz_mn_p).  dpre instruction
   // t (of kDI) is q = w + NW t: rows 16 q + lane / 4, unit (lane % 4) ^ swz_k.
   uint32_t aoff[2], aoff0[2], boff[kDI], boff0[kDI];  // byte offsets from the chunk's bases (full / chunk 0)
   bool aok0[2], bok0;
@@ -880,7 +880,7 @@ __global__ __launch_bounds__(512) void me_bwd_dw_dma_kernel(const T* __restrict_
   const int kbeg = M - nk * kChunkK;
 
   // DMA pieces: piece k < kPX moves flattened units 64 k + lane of the x tile (K-row U / kU,
-  // physical unit U % kU <- logical unit (U % kU) ^ swz_mn(K-row)); piece k >= kPX the same of the
+  // physical unit U % kU <- logical unit (U % kU) ^ swz_mn_p(K-row)); piece k >= kPX the same of the
   // dpre tile with kJU units per K-row (columns past 2 I clamped to the band's last 8).  Wave w
   // issues pieces w, w + NW, ... < kPT.
   const int npw = kEven ? kMaxPW : (kPT - wave + NW - 1) / NW;
@@ -893,7 +893,7 @@ __global__ __launch_bounds__(512) void me_bwd_dw_dma_kernel(const T* __restrict_
     const int units = isx[t] ? kU : kJU;
     const int U = 64 * (isx[t] ? k : k - kPX) + lane;
     const int kr = U / units;
-    const int u = (U % units) ^ swz_mn(kr);
+    const int u = (U % units) ^ (isx[t] ? swz_mn_p<2 * HT>(kr) : swz_mn_p<2 * JT>(kr));
     ok0[t] = kbeg + kr >= 0;
     if (isx[t]) {
       goff[t] = static_cast<uint32_t>((kr * xstride + 8 * u) * 2);
@@ -923,8 +923,8 @@ __global__ __launch_bounds__(512) void me_bwd_dw_dma_kernel(const T* __restrict_
   uint32_t fa[4], fb[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    fa[i] = frag_mn_addr(lds0, 64 * wr + 16 * i, 2 * HT, lane);
-    fb[i] = frag_mn_addr(lds0 + kXTile, 64 * wc + 16 * i, 2 * JT, lane);
+    fa[i] = frag_mn_addr_p<2 * HT>(lds0, 64 * wr + 16 * i, lane);
+    fb[i] = frag_mn_addr_p<2 * JT>(lds0 + kXTile, 64 * wc + 16 * i, lane);
   }
   f32x4_t acc[4][4];
 #pragma unroll

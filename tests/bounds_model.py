@@ -74,26 +74,22 @@ def cdiv(a: int, b: int) -> int:
 
 
 def swz_k(r):  # dma_gemm.h
-    return ((r >> 1) ^ (r >> 3)) & 3
-
-
-def swz_mn(k):  # dma_gemm.h
-    return 2 * (k & 3)
+    return -(r >> 2) & 3
 
 
 def swz_mn_p(pitch: int, k):  # dma_gemm.h swz_mn_p<PITCH>
-    if pitch == 512:
-        return 2 * ((k & 3) | (((k >> 3) & 3) << 2))
-    return swz_mn(k)
+    assert pitch % 128 == 0
+    if pitch % 256 == 0:
+        return 2 * ((k & 3) | (((k >> 3) & 1) << 2))
+    return 2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1))
 
 
-def frag_mn_addr(region, c0, pitch, lane, p512=False):  # dma_gemm.h frag_mn_addr / frag_mn_addr_p
+def frag_mn_addr(region, c0, pitch, lane):  # dma_gemm.h frag_mn_addr_p
     j, g = lane & 15, lane >> 4
     k = 8 * g + (j >> 2)
     col = c0 + 4 * (j & 3)
     unit = col >> 3
-    sw = swz_mn_p(pitch, k) if p512 else swz_mn(k)
-    return region + k * pitch + 16 * (unit ^ sw) + 2 * (col & 7)
+    return region + k * pitch + 16 * (unit ^ swz_mn_p(pitch, k)) + 2 * (col & 7)
 
 
 def frag_k_addr(region, r0, lane):  # dma_gemm.h
@@ -732,7 +728,7 @@ def _replay_glin_dx(bnd, G, I, O, M, rb=None):
                 t = wave + 4 * q
                 P = 64 * t + lane
                 kr, pu = P // kUnits, P % kUnits
-                u = pu ^ swz_mn(kr)
+                u = pu ^ swz_mn_p(2 * I, kr)
                 if np.any(u >= kUnits):
                     bnd.fail("glin_dx: swizzled unit leaves its row")
                 for c in steps(nc):
@@ -757,7 +753,7 @@ def _replay_glin_dx(bnd, G, I, O, M, rb=None):
                 base = stage * kStage
                 for d in range(DT):
                     col = 16 * d + 4 * (jq & 3)
-                    off = kr0 * 2 * I + 16 * ((col >> 3) ^ swz_mn(kr0)) + 2 * (col & 7)
+                    off = kr0 * 2 * I + 16 * ((col >> 3) ^ swz_mn_p(2 * I, kr0)) + 2 * (col & 7)
                     bnd.touch("lds_gdx", base + off, 8)
                     bnd.touch("lds_gdx", base + off + 4 * 2 * I, 8)
                 for n in range(NT):
@@ -822,14 +818,14 @@ def _replay_bs_dw_dma(bnd, widths, offs, M, O, esz, has_bias):
             stage = (c % S) * kStage
             for t in range(kDI):
                 r = kWR * wave + 8 * t + (lane >> 3)
-                col = np.minimum(o0 + 8 * ((lane & 7) ^ swz_mn(r)), O - 8)
+                col = np.minimum(o0 + 8 * ((lane & 7) ^ swz_mn_p(2 * 64, r)), O - 8)
                 row = kbeg + c * KR + r
                 row = np.where((c == 0) & (row < 0), 0, row)
                 bnd.touch("dy", (row * dstride + band * O + col) * esz, 16)
                 bnd.touch("lds", stage + kTile + 128 * (kWR * wave + 8 * t) + 16 * lane, 16)
             for t in range(kXI):
                 r = kWR * wave + 2 * t + (lane >> 5)
-                i = np.minimum(i0 + 8 * (((lane & 31) >> 2) ^ swz_mn(r)) + 2 * (lane & 3), I - 2)
+                i = np.minimum(i0 + 8 * (((lane & 31) >> 2) ^ swz_mn_p(2 * 64, r)) + 2 * (lane & 3), I - 2)
                 row = kbeg + c * KR + r
                 row = np.where((c == 0) & (row < 0), 0, row)
                 bnd.touch("x", (row * F + off + i) * esz, 4)
@@ -1059,7 +1055,7 @@ def _replay_me_dw_dma(bnd, widths, offs, M, H, esz, HT, dpre_buf, x_buf, dw_buf,
                 units = np.where(isx, kU2, kJU)
                 U = 64 * np.where(isx, k, k - PX) + lane
                 kr = U // units
-                uu = (U % units) ^ swz_mn(kr)
+                uu = (U % units) ^ np.where(isx, swz_mn_p(2 * HT, kr), swz_mn_p(2 * JT, kr))
                 row = kbeg + c * CHUNK_K + kr
                 row = np.where((c == 0) & (row < 0), 0, row)
                 bnd.touch(x_buf, (row * xstride + band * H + h0 + 8 * uu) * esz, 16, valid & isx)
@@ -1127,8 +1123,8 @@ def _replay_me_dz(bnd, widths, offs, M, H, esz, tanh_in):
                 t = wave + 4 * q
                 P = 64 * t + lane
                 kr, pu = P // kUnits, P % kUnits
-                col = h0 + 8 * (pu ^ swz_mn(kr))
-                if np.any(pu ^ swz_mn(kr) >= kUnits):
+                col = h0 + 8 * (pu ^ swz_mn_p(2 * HT, kr))
+                if np.any(pu ^ swz_mn_p(2 * HT, kr) >= kUnits):
                     bnd.fail("me_dz: swizzled unit leaves its row")
                 for c in steps(nc):
                     j = np.minimum(32 * c + kr, K - 1)
@@ -1151,7 +1147,7 @@ def _replay_me_dz(bnd, widths, offs, M, H, esz, tanh_in):
                 base = stage * kStage
                 for d in range(DT):
                     col = 16 * d + 4 * (jq & 3)
-                    o = kr0 * 2 * HT + 16 * ((col >> 3) ^ swz_mn(kr0)) + 2 * (col & 7)
+                    o = kr0 * 2 * HT + 16 * ((col >> 3) ^ swz_mn_p(2 * HT, kr0)) + 2 * (col & 7)
                     bnd.touch("lds_dz", base + o, 8)
                     bnd.touch("lds_dz", base + o + 4 * 2 * HT, 8)
                 for n in range(NT):
@@ -1276,7 +1272,7 @@ def replay_mask_final_backward(widths, M, H, esz, *, tanh_in=False):
                 bnd.touch("workspace", ((m0 + mrc) * 2 * F + 2 * off + col) * esz, 16)
                 bnd.touch("lds", st + kWTile + (wave + NW * t) * 1024 + 16 * lane, 16)
             for i in range(4):
-                fa = frag_mn_addr(0, 64 * wr + 16 * i, 2 * HC, lane, p512=True) + st
+                fa = frag_mn_addr(0, 64 * wr + 16 * i, 2 * HC, lane) + st
                 bnd.touch("lds", fa, 8)
                 bnd.touch("lds", fa + 4 * 2 * HC, 8)
             fb = frag_k_addr(kWTile, 64 * wc, lane) + st
