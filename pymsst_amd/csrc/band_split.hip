@@ -1362,7 +1362,12 @@ int launch_grouped_bwd(const void* dy, const void* x, const void* weight, const 
   const T* pdy = static_cast<const T*>(dy);
   const T* px = static_cast<const T*>(x);
   const T* pw = static_cast<const T*>(weight);
-  if (M > 0 && grouped_dx_supported(hb.NB, hb.max_width, O, M, sizeof(T), dy, weight, dx)) {
+  if (wide_dx_supported(hb.NB, hb.max_width, O, M, sizeof(T), dy, weight, dx)) {
+    if constexpr (sizeof(T) == 2) {
+      const int rc = launch_wide_dx<T>(dy, weight, dx, hb.NB, hb.max_width, O, M, stream);
+      if (rc != PMSST_OK) return rc;
+    }
+  } else if (M > 0 && grouped_dx_supported(hb.NB, hb.max_width, O, M, sizeof(T), dy, weight, dx)) {
     if constexpr (sizeof(T) == 2) {
       const int rc = launch_grouped_dx<T>(dy, weight, dx, hb.NB, hb.max_width, O, M, stream);
       if (rc != PMSST_OK) return rc;
@@ -1383,7 +1388,12 @@ int launch_grouped_bwd(const void* dy, const void* x, const void* weight, const 
     int rc = check_launch("bs_bwd_dx_kernel");
     if (rc != PMSST_OK) return rc;
   }
-  if (uniform_dw_supported(hb.NB, hb.max_width, O, M, sizeof(T), dy, x, dw)) {
+  if (wide_dw_supported(hb.NB, hb.max_width, O, M, sizeof(T), dy, x, dw)) {
+    if constexpr (sizeof(T) == 2) {
+      const int rc = launch_wide_dw<T>(dy, x, dw, db, hb.NB, hb.max_width, O, M, stream);
+      if (rc != PMSST_OK) return rc;
+    }
+  } else if (uniform_dw_supported(hb.NB, hb.max_width, O, M, sizeof(T), dy, x, dw)) {
     if constexpr (sizeof(T) == 2) {
       const int rc = launch_uniform_dw<T>(dy, x, dw, db, hb.NB, hb.max_width, O, M, stream);
       if (rc != PMSST_OK) return rc;

@@ -27,6 +27,20 @@ template <typename T>
 int launch_uniform_dw(const void* dy, const void* x, void* dw, void* db, int64_t groups, int64_t in_features,
                       int64_t out_features, int64_t rows, hipStream_t stream);
 
+// Whether the same two products run on grouped_gemm.hip's 256-wide tiles, which are taken first: 16-bit
+// layers of at least 192 inputs (dx at 192 and 256: where the grid fills its rounds), widths in whole
+// eights (dx: out_features in whole 32s), 16-byte aligned pointers.
+bool wide_dx_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
+                       const void* dy, const void* w, const void* dx);
+template <typename T>
+int launch_wide_dx(const void* dy, const void* w, void* dx, int64_t groups, int64_t in_features, int64_t out_features,
+                   int64_t rows, hipStream_t stream);
+bool wide_dw_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
+                       const void* dy, const void* x, const void* dw);
+template <typename T>
+int launch_wide_dw(const void* dy, const void* x, void* dw, void* db, int64_t groups, int64_t in_features,
+                   int64_t out_features, int64_t rows, hipStream_t stream);
+
 // Whether launch_mask_dz takes this shape (16-bit, H a multiple of 128 or 192, aligned pointers); the
 // caller checks that every band width is a multiple of 4.
 bool mask_dz_supported(int64_t H, int64_t rows, size_t elem, const void* dpre, const void* w, const void* x,
