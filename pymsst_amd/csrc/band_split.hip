@@ -1612,6 +1612,12 @@ int pmsst_grouped_linear_forward(const void* x, int64_t x_row_stride, const void
   if (rc != PMSST_OK) return rc;
   return with_dtype(dtype, "grouped_linear_forward", [&](auto tag) {
     using T = decltype(tag);
+    if constexpr (sizeof(T) == 2) {
+      if (activation == PMSST_ACT_TANH && x_row_stride == groups * in_features && group_offsets != nullptr &&
+          wide_tanh_supported(groups, in_features, out_features, rows, sizeof(T), x, weight, bias, out))
+        return launch_wide_tanh<T>(x, weight, bias, out, groups, in_features, out_features, rows,
+                                   static_cast<hipStream_t>(stream));
+    }
     return launch_fwd<T>(x, x_row_stride, nullptr, weight, bias, group_offsets, hb, rows, out_features, out, nullptr,
                          nullptr, false, activation, static_cast<hipStream_t>(stream));
   });

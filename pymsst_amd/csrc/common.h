@@ -9,6 +9,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <type_traits>
 
 #include "pymsst_amd.h"
 
@@ -70,6 +71,24 @@ __device__ __forceinline__ void store_pack(T* __restrict__ p, const float (&o)[N
 #pragma unroll
   for (int i = 0; i < N; ++i) pk.v[i] = from_f32<T>(o[i]);
   *reinterpret_cast<Pack<T, N>*>(p) = pk;
+}
+
+// tanh of a value that holds a T (bf16 or fp16), for rounding back to T: equal to the correctly rounded
+// tanh at each of T's 65536 patterns (checked against the table of pmsst_mask_mlp_tanh_table; NaN gives
+// a NaN).  1 - 2 / (exp(2 z) + 1), and where that cancels z itself, which is bf16's rounded tanh below
+// 1/16, or for fp16, below 1/4, the odd series to z^7 (its z^9 term is 62/2835 z^8 < 4e-7 of the value).
+// exp and reciprocal are the hardware's (1 ulp).
+template <typename T>
+__device__ __forceinline__ float tanh16(float z) {
+  const float e = __builtin_amdgcn_exp2f(z * 2.88539008177792681f);
+  const float t = fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f);
+  if constexpr (std::is_same<T, bf16>::value) {
+    return fabsf(z) < 0.0625f ? z : t;
+  } else {
+    const float q = z * z;
+    const float p = fmaf(q, fmaf(q, fmaf(q, -17.f / 315.f, 2.f / 15.f), -1.f / 3.f), 1.f);
+    return fabsf(z) < 0.25f ? z * p : t;
+  }
 }
 
 // Butterfly sum over aligned groups of `width` lanes (width a power of two <= 64).

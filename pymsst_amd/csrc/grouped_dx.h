@@ -41,6 +41,14 @@ template <typename T>
 int launch_wide_dw(const void* dy, const void* x, void* dw, void* db, int64_t groups, int64_t in_features,
                    int64_t out_features, int64_t rows, hipStream_t stream);
 
+// h[m, g, :] = tanh(x[m, g, :] W_g^T + bias_g), z rounded to the storage type before the tanh, on the same
+// file's forward tiles: 16-bit, in_features in whole 32s, out_features in whole eights, a bias.
+bool wide_tanh_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
+                         const void* x, const void* w, const void* bias, const void* out);
+template <typename T>
+int launch_wide_tanh(const void* x, const void* w, const void* bias, void* out, int64_t groups, int64_t in_features,
+                     int64_t out_features, int64_t rows, hipStream_t stream);
+
 // Whether launch_mask_dz takes this shape (16-bit, H a multiple of 128 or 192, aligned pointers); the
 // caller checks that every band width is a multiple of 4.
 bool mask_dz_supported(int64_t H, int64_t rows, size_t elem, const void* dpre, const void* w, const void* x,

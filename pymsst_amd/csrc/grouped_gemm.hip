@@ -1,13 +1,16 @@
 // The grouped linear's products at wide layers, 16-bit storage, fp32 accumulation:
+//   h[m, g, :]   = tanh(x[m, g, :] W_g^T + bias_g)   (K = in_features; rounded before the tanh)
 //   dx[m, g, :]  = dy[m, g, :] W_g            (K = out_features)
 //   dW[g][o][i]  = sum_m dy[m, g, o] x[m, g, i], db[g][o] = sum_m dy[m, g, o]   (K = rows)
 // dy[M, G, O], x and dx[M, G, I], W and dW[G, O, I] row-major.
 //
-// Block = 8 waves on a tile of AR x BR results: A rows run along the result's contiguous axis (a
+// Backward block = 8 waves on a tile of AR x BR results: A rows run along the result's contiguous axis (a
 // lane's 4 accumulators are 4 neighbours of it), B rows along its rows.  Wave (wa, wb) owns
 // 16 TA x 16 TB of it.  32-wide K chunks of both operands move by global -> LDS DMA into a ring of
 // kGgStages stages; K-contiguous operands (dy in dx) as 64-byte rows, the others (W in dx, both in
-// dW) as K-rows of the tile's width, read transposed (ds_read_b64_tr_b16).
+// dW) as K-rows of the tile's width, read transposed (ds_read_b64_tr_b16).  Forward block = 4 waves on a
+// tile half as high with a ring of 3 stages, two blocks per CU: its K loop is short (2 to 16 chunks) and
+// one block's loads and tanh epilogue run beside the other's products.
 //
 // What bounds it: the matrix cores want 32 MFMAs of 16 cycles per wave and chunk on a 256 x 256 tile,
 // two waves to a SIMD, i.e. 1024 cycles a chunk, in which the block's fragment reads take 768 LDS
@@ -24,19 +27,16 @@
 namespace pmsst {
 namespace {
 
-constexpr int kGgStages = 4;
-constexpr int kGgWaves = 8;
-
-enum GgOp { kGgDx, kGgDw };
+enum GgOp { kGgDx, kGgDw, kGgFwd };
 
 struct GgArgs {
-  const void* a;   // dx: W; dw: x
-  const void* b;   // dy
-  void* d;         // dx or dW
-  void* db;        // dw: bias gradient or null
+  const void* a;   // dx, fwd: W; dw: x
+  const void* b;   // dx, dw: dy; fwd: x
+  void* d;         // dx, dW or h
+  void* db;        // dw: bias gradient or null; fwd: bias
   int64_t M;
   int G, O, I;
-  int a_tiles;     // tiles of AR along I
+  int a_tiles;     // tiles of AR along the A rows
 };
 
 // One 16-byte-per-lane global -> LDS DMA from a uniform base plus a 32-bit byte offset per lane (see
@@ -54,12 +54,15 @@ __device__ __forceinline__ void dma16_base(const char* base, uint32_t off, uint3
       : "memory");
 }
 
+constexpr int gg_waves(GgOp op) { return op == kGgFwd ? 4 : 8; }
+
 template <typename T, GgOp OP, int TA, int WA>
-__global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched sc) {
-  constexpr int S = kGgStages;
-  constexpr int NW = kGgWaves, WB = NW / WA, TB = 16 / WB;  // 256 B rows
-  constexpr int AR = 16 * TA * WA, BR = 256;
-  constexpr bool B_KC = OP == kGgDx;                 // B is K-contiguous
+__global__ __launch_bounds__(gg_waves(OP) * 64) __attribute__((amdgpu_waves_per_eu(2))) void gg_kernel(GgArgs a,
+                                                                                                      BandSched sc) {
+  constexpr int NW = gg_waves(OP), S = NW == 8 ? 4 : 3;
+  constexpr int WB = NW / WA, TB = 4;
+  constexpr int AR = 16 * TA * WA, BR = 16 * TB * WB;
+  constexpr bool A_KC = OP == kGgFwd, B_KC = OP != kGgDw;  // K-contiguous operands
   constexpr int kABytes = AR * 64, kStage = kABytes + BR * 64;
   constexpr int kPA = kABytes / 1024, kPT = kStage / 1024;  // 1 KB DMA pieces: A's, then B's
   constexpr int PW = (kPT + NW - 1) / NW;            // per wave; a wave with fewer repeats its first
@@ -75,28 +78,32 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int wa = wave % WA, wb = wave / WA;
   const int64_t dyrow = static_cast<int64_t>(a.G) * a.O, xrow = static_cast<int64_t>(a.G) * a.I;
-  const int K = OP == kGgDx ? a.O : static_cast<int>(a.M);
+  const int K = OP == kGgDx ? a.O : OP == kGgDw ? static_cast<int>(a.M) : a.I;
   const int nk = (K + 31) / 32;
   const int kbeg = K - 32 * nk;  // dw: chunks end at M, so only chunk 0 has K rows to leave out
   const int a0 = static_cast<int>(ta) * AR;
   const int64_t b0 = static_cast<int64_t>(tb) * BR;
-  const int avalid = a.I - a0 < AR ? a.I - a0 : AR;
-  const int64_t bleft = (OP == kGgDx ? a.M : a.O) - b0;
+  const int aleft = (OP == kGgFwd ? a.O : a.I) - a0;
+  const int avalid = aleft < AR ? aleft : AR;
+  const int64_t bleft = (OP == kGgDw ? a.O : a.M) - b0;
   const int bvalid = bleft < BR ? static_cast<int>(bleft) : BR;
 
   // ---- DMA plan: piece k of a stage (k = wave + NW q).  MN operand: flattened 16-byte units
   // 64 k + lane of its 32 K-rows; K-contiguous: rows 16 k + lane / 4.  Columns and rows past the tile's
   // valid part repeat its last (their products are not stored).
-  const int64_t astride = OP == kGgDx ? a.I : xrow;  // elements between A's K-rows
-  const char* abase = static_cast<const char*>(a.a) +
-                      2 * ((OP == kGgDx ? static_cast<int64_t>(g) * a.O * a.I : static_cast<int64_t>(g) * a.I) + a0);
-  const char* bbase = static_cast<const char*>(a.b) +
-                      2 * (static_cast<int64_t>(g) * a.O + (OP == kGgDx ? b0 * dyrow : b0));
+  const int64_t astride = OP == kGgDw ? xrow : a.I;     // elements between A's K-rows (fwd: rows)
+  const int64_t bstride = OP == kGgFwd ? xrow : dyrow;  // elements between B's rows (dw: K-rows)
+  const int64_t wg = static_cast<int64_t>(g) * a.O * a.I;
+  const char* abase = static_cast<const char*>(a.a) + 2 * (OP == kGgDx   ? wg + a0
+                                                           : OP == kGgDw ? static_cast<int64_t>(g) * a.I + a0
+                                                                         : wg + static_cast<int64_t>(a0) * a.I);
+  const char* bbase = static_cast<const char*>(a.b) + 2 * (static_cast<int64_t>(g) * (OP == kGgFwd ? a.I : a.O) +
+                                                           (OP == kGgDw ? b0 : b0 * bstride));
   if (OP == kGgDw) {
     abase += 2 * kbeg * astride;
-    bbase += 2 * kbeg * dyrow;
+    bbase += 2 * kbeg * bstride;
   }
-  const int64_t astep = 64 * astride, bstep = B_KC ? 64 : 64 * dyrow;  // bytes per chunk
+  const int64_t astep = A_KC ? 64 : 64 * astride, bstep = B_KC ? 64 : 64 * bstride;  // bytes per chunk
   uint32_t off[PW], ldst[PW];
   bool isa[PW];
   [[maybe_unused]] int krow[PW];  // K-row of this lane's unit
@@ -106,20 +113,21 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
     k = k < kPT ? k : wave;
     isa[q] = k < kPA;
     ldst[q] = static_cast<uint32_t>(k * 1024);
-    if (isa[q] || !B_KC) {
+    const int64_t stride = isa[q] ? astride : bstride;
+    const int valid = isa[q] ? avalid : bvalid;
+    if (!(isa[q] ? A_KC : B_KC)) {
       const int units = isa[q] ? AR / 8 : BR / 8;
       const int U = 64 * (isa[q] ? k : k - kPA) + lane;
       const int kr = U / units;
       const int u = (U % units) ^ (isa[q] ? swz_mn_p<2 * AR>(kr) : swz_mn_p<2 * BR>(kr));
-      const int valid = isa[q] ? avalid : bvalid;
       const int col = 8 * u < valid ? 8 * u : valid - 8;
       krow[q] = kr;
-      off[q] = static_cast<uint32_t>((kr * (isa[q] ? astride : dyrow) + col) * 2);
+      off[q] = static_cast<uint32_t>((kr * stride + col) * 2);
     } else {
-      const int r = 16 * (k - kPA) + (lane >> 2);
-      const int rc = r < bvalid ? r : bvalid - 1;
+      const int r = 16 * (isa[q] ? k : k - kPA) + (lane >> 2);
+      const int rc = r < valid ? r : valid - 1;
       krow[q] = 0;
-      off[q] = static_cast<uint32_t>((rc * dyrow + 8 * ((lane & 3) ^ swz_k(lane >> 2))) * 2);
+      off[q] = static_cast<uint32_t>((rc * stride + 8 * ((lane & 3) ^ swz_k(lane >> 2))) * 2);
     }
   }
   const uint32_t lds0 = lds_addr(lds);
@@ -137,7 +145,7 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
     for (int q = 0; q < PW; ++q) {
       uint32_t o = off[q];
       if (OP == kGgDw && kbeg + krow[q] < 0)
-        o += static_cast<uint32_t>(-(kbeg + krow[q])) * static_cast<uint32_t>((isa[q] ? astride : dyrow) * 2);
+        o += static_cast<uint32_t>(-(kbeg + krow[q])) * static_cast<uint32_t>((isa[q] ? astride : bstride) * 2);
       dma16_base(isa[q] ? abase : bbase, o, __builtin_amdgcn_readfirstlane(lds0 + ldst[q]));
     }
   }
@@ -150,6 +158,17 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
   for (int i = 0; i < TA; ++i)
 #pragma unroll
     for (int j = 0; j < TB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if constexpr (OP == kGgFwd) {  // the sums start at the bias, as the one-pass MLP's do
+    const T* bias = static_cast<const T*>(a.db) + static_cast<int64_t>(g) * a.O + a0;
+#pragma unroll
+    for (int i = 0; i < TA; ++i) {
+      const int o = 16 * (TA * wa + i) + 4 * gq;
+      float v[4];
+      load_pack<T, 4>(bias + (o < avalid ? o : avalid - 4), v);
+#pragma unroll
+      for (int j = 0; j < TB; ++j) acc[i][j] = f32x4_t{v[0], v[1], v[2], v[3]};
+    }
+  }
   // column sums of B (db): lane's 8 K values of column 16 j + rr, summed per chunk
   const bool do_bias = OP == kGgDw && a.db != nullptr && ta == 0 && wa == 0;
   [[maybe_unused]] float csum[TB];
@@ -159,7 +178,8 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
   // ---- fragment offsets inside a stage
   uint32_t aoff[TA], boff[TB];
 #pragma unroll
-  for (int i = 0; i < TA; ++i) aoff[i] = frag_mn_addr_p<2 * AR>(0, 16 * (TA * wa + i), lane);
+  for (int i = 0; i < TA; ++i)
+    aoff[i] = A_KC ? frag_k_addr(0, 16 * (TA * wa + i), lane) : frag_mn_addr_p<2 * AR>(0, 16 * (TA * wa + i), lane);
 #pragma unroll
   for (int j = 0; j < TB; ++j)
     boff[j] = B_KC ? frag_k_addr(kABytes, 16 * (TB * wb + j), lane)
@@ -172,7 +192,10 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
       else fb[j] = tr_frag(st + boff[j], 4 * 2 * BR);
     }
 #pragma unroll
-    for (int i = 0; i < TA; ++i) fa[i] = tr_frag(st + aoff[i], 4 * 2 * AR);
+    for (int i = 0; i < TA; ++i) {
+      if constexpr (A_KC) fa[i] = *reinterpret_cast<const u32x4_t*>(st + aoff[i]);
+      else fa[i] = tr_frag(st + aoff[i], 4 * 2 * AR);
+    }
   };
   auto mma = [&](const u32x4_t (&fa)[TA], const u32x4_t (&fb)[TB]) {
 #pragma unroll
@@ -204,13 +227,13 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
     asm volatile("" ::: "memory");
   };
   auto wait_chunks = [&](int after) {
-    if (after >= 2) vm_wait<2 * PW>();
-    else if (after == 1) vm_wait<PW>();
+    if (S == 4 && after >= 2) vm_wait<2 * PW>();
+    else if (after >= 1) vm_wait<PW>();
     else vm_wait<0>();
   };
-  static_assert(S == 4, "wait_chunks");
+  static_assert(S == 3 || S == 4, "wait_chunks");
   // a chunk's fragment reads spread between the MFMAs of the chunk before it
-  constexpr int kReads = 2 * TA + (B_KC ? 1 : 2) * TB, kMma = TA * TB;
+  constexpr int kReads = (A_KC ? 1 : 2) * TA + (B_KC ? 1 : 2) * TB, kMma = TA * TB;
   auto interleave = [&]() {
     constexpr int kPer = kMma / (kReads / 2);
 #pragma unroll
@@ -286,16 +309,22 @@ __global__ __launch_bounds__(64 * kGgWaves) void gg_kernel(GgArgs a, BandSched s
     const int r = 16 * (TB * wb + j) + rr;
 #pragma unroll
     for (int i = 0; i < TA; ++i) {
-      const float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+      float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+      if constexpr (OP == kGgFwd) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = tanh16<T>(to_f32(from_f32<T>(v[e])));
+      }
       store_pack<T, 4>(ot + r * kOP + 16 * (TA * wa + i) + 4 * gq, v);
     }
   }
   __syncthreads();
   constexpr int kUnits = AR / 8;
-  const int64_t drow = OP == kGgDx ? xrow : a.I;
-  T* d = static_cast<T*>(a.d) + (OP == kGgDx ? static_cast<int64_t>(g) * a.I + b0 * xrow
-                                             : (static_cast<int64_t>(g) * a.O + b0) * a.I) + a0;
-  const int nu = avalid / 8;  // whole units (I is a multiple of 8)
+  const int64_t drow = OP == kGgDx ? xrow : OP == kGgDw ? a.I : dyrow;
+  const int64_t d0 = OP == kGgDx   ? static_cast<int64_t>(g) * a.I
+                     : OP == kGgDw ? static_cast<int64_t>(g) * a.O * a.I
+                                   : static_cast<int64_t>(g) * a.O;
+  T* d = static_cast<T*>(a.d) + d0 + b0 * drow + a0;
+  const int nu = avalid / 8;  // whole units
 #pragma unroll
   for (int p = 0; p < BR * kUnits / (64 * NW); ++p) {
     const int q = static_cast<int>(threadIdx.x) + 64 * NW * p;
@@ -311,17 +340,18 @@ int launch(const GgArgs& a, hipStream_t stream) {
   uint32_t per_xcd = 0;
   constexpr int AR = 16 * TA * WA;
   GgArgs ar = a;
-  ar.a_tiles = (a.I + AR - 1) / AR;
-  const int64_t b_rows = OP == kGgDx ? a.M : a.O;
-  if (!build_even_sched(a.G, (b_rows + 255) / 256, [&](int) { return static_cast<int64_t>(ar.a_tiles); }, &sc, &per_xcd))
-    return fail(PMSST_EINVAL, "grouped_linear_backward: too many groups or rows for the block schedule");
-  hipLaunchKernelGGL((gg_kernel<T, OP, TA, WA>), dim3(per_xcd * kXcds), dim3(64 * kGgWaves), 0, stream, ar, sc);
+  constexpr int BR = 16 * 4 * gg_waves(OP) / WA;
+  ar.a_tiles = ((OP == kGgFwd ? a.O : a.I) + AR - 1) / AR;
+  const int64_t b_rows = OP == kGgDw ? a.O : a.M;
+  if (!build_even_sched(a.G, (b_rows + BR - 1) / BR, [&](int) { return static_cast<int64_t>(ar.a_tiles); }, &sc, &per_xcd))
+    return fail(PMSST_EINVAL, "grouped linear: too many groups or rows for the block schedule");
+  hipLaunchKernelGGL((gg_kernel<T, OP, TA, WA>), dim3(per_xcd * kXcds), dim3(64 * gg_waves(OP)), 0, stream, ar, sc);
   return check_launch("gg_kernel");
 }
 
 template <typename T, GgOp OP>
 int launch_op(const GgArgs& a, hipStream_t stream) {
-  if (a.I % 256 == 0) return launch<T, OP, 8, 2>(a, stream);
+  if ((OP == kGgFwd ? a.O : a.I) % 256 == 0) return launch<T, OP, 8, 2>(a, stream);
   return launch<T, OP, 6, 2>(a, stream);
 }
 
@@ -371,7 +401,24 @@ int launch_wide_dw(const void* dy, const void* x, void* dw, void* db, int64_t gr
                                     static_cast<int>(in_features), 0}, stream);
 }
 
+bool wide_tanh_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
+                         const void* x, const void* w, const void* bias, const void* out) {
+  return shape_ok(groups, in_features, out_features, rows, elem) && in_features % 32 == 0 && groups > 0 &&
+         x != nullptr && w != nullptr && out != nullptr && in_features > 0 && out_features > 0 &&
+         256 * in_features * 2 < (int64_t{1} << 31) && aligned16(x) && aligned16(w) && aligned16(out) &&
+         bias != nullptr && reinterpret_cast<uintptr_t>(bias) % 8 == 0;
+}
+
+template <typename T>
+int launch_wide_tanh(const void* x, const void* w, const void* bias, void* out, int64_t groups, int64_t in_features,
+                     int64_t out_features, int64_t rows, hipStream_t stream) {
+  return launch_op<T, kGgFwd>(GgArgs{w, x, out, const_cast<void*>(bias), rows, static_cast<int>(groups),
+                                     static_cast<int>(out_features), static_cast<int>(in_features), 0}, stream);
+}
+
 #define PMSST_GG(T)                                                                                                  \
+  template int launch_wide_tanh<T>(const void*, const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, \
+                                   hipStream_t);                                                                    \
   template int launch_wide_dx<T>(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, hipStream_t); \
   template int launch_wide_dw<T>(const void*, const void*, void*, void*, int64_t, int64_t, int64_t, int64_t,        \
                                  hipStream_t);

@@ -27,6 +27,7 @@
 #include "common.h"
 #include "dma_gemm.h"
 #include "gemm.h"
+#include "mask_mlp.h"
 #include "rowgeom.h"
 #include "grouped_dx.h"
 #include "ring.h"
@@ -192,12 +193,12 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(PM
 constexpr int kMefStage = 16384;  // bytes of one LDS stage
 
 
-template <typename T>
+template <typename T, bool APPLY>
 __global__ __launch_bounds__(kGemmThreads) void me_fwd_dma_kernel(const T* __restrict__ x,
                                                                   const T* __restrict__ weight,
                                                                   const T* __restrict__ bias, T* __restrict__ pre,
                                                                   T* __restrict__ out, int max_lchunks, XcdGrid xg,
-                                                                  MaskArgs a, BandSched sc) {
+                                                                  MaskArgs a, BandSched sc, MlpApply ap) {
   constexpr int S = PMSST_MEF_STAGES;
   static_assert(S >= 2 && S <= 8, "stages");
   __shared__ __attribute__((aligned(1024))) char lds[S * kMefStage];
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(kGemmThreads) void me_fwd_dma_kernel(const T* __res
 #pragma unroll
     for (int t = 0; t < 4; ++t)
       if (t < nv)
-        __builtin_amdgcn_global_load_lds(src + soff[t], my_lds + stage * kMefStage + t * 1024, 16, 0, 0);
+        dma_lds16(src + soff[t], my_lds + stage * kMefStage + t * 1024);
   };
 
   // chunk 0 through registers: units with k < 0 are zero (they load k = 0 of the row)
@@ -352,10 +353,26 @@ __global__ __launch_bounds__(kGemmThreads) void me_fwd_dma_kernel(const T* __res
           vl[r] = acc[2 * h][j][r] + bl[r];
           vg[r] = acc[2 * h + 1][j][r] + bgt[r];
           vo[r] = vl[r] * sigmoidf_(vg[r]);
+          // rounded to fp32 before its 16-bit conversion, as in the one-pass MLP's epilogue
+          asm volatile("" : "+v"(vo[r]));
         }
         store_pack<T, 4>(ol + m * kOP + lt, vl);
         store_pack<T, 4>(og + m * kOP + lt, vg);
-        store_pack<T, 4>(oo + m * kOP + lt, vo);
+        if constexpr (APPLY) {
+          // lanes rr = 0 .. 15 hold consecutive frames; the 4 outputs are 2 complex rows
+          const int r0 = (off + l) >> 1;
+          const int64_t row = m0 + m;
+          if (l < I && m < rows_valid) {
+            const uint32_t bb = ap.frames.div(static_cast<uint32_t>(row));
+            const uint32_t tt = static_cast<uint32_t>(row) - bb * ap.frames.d;
+            const float2* sp = ap.spec + (static_cast<int64_t>(bb) * ap.Fbins * ap.C + r0) * ap.frames.d + tt;
+            const float2 s0 = sp[0], s1 = sp[ap.frames.d];
+            store_masked<T>(ap, bb, tt, r0, s0, vo[0], vo[1]);
+            store_masked<T>(ap, bb, tt, r0 + 1, s1, vo[2], vo[3]);
+          }
+        } else {
+          store_pack<T, 4>(oo + m * kOP + lt, vo);
+        }
       }
     }
   }
@@ -370,8 +387,9 @@ __global__ __launch_bounds__(kGemmThreads) void me_fwd_dma_kernel(const T* __res
       T* pl = pre + (m0 + m) * pitch2 + 2 * off + l0 + c4;
       *reinterpret_cast<u32x2_t*>(pl) = *reinterpret_cast<const u32x2_t*>(ol + m * kOP + c4);
       *reinterpret_cast<u32x2_t*>(pl + I) = *reinterpret_cast<const u32x2_t*>(og + m * kOP + c4);
-      *reinterpret_cast<u32x2_t*>(out + (m0 + m) * a.F + off + l0 + c4) =
-          *reinterpret_cast<const u32x2_t*>(oo + m * kOP + c4);
+      if constexpr (!APPLY)
+        *reinterpret_cast<u32x2_t*>(out + (m0 + m) * a.F + off + l0 + c4) =
+            *reinterpret_cast<const u32x2_t*>(oo + m * kOP + c4);
     }
   }
 }
@@ -1060,14 +1078,20 @@ int check_mask(const char* op, const int64_t* dim_inputs, int64_t band_count, in
 
 bool al(const void* p, size_t b) { return p == nullptr || reinterpret_cast<uintptr_t>(p) % b == 0; }
 
+// 32-bit offsets of the DMA-pipelined forward: a band's weight rows, 128 rows of x
+bool me_fwd_dma_offsets_ok(const HostMask& hm, int64_t H) {
+  return (2 * static_cast<int64_t>(hm.max_width) + 1) * H * 2 < (int64_t{1} << 31) &&
+         (static_cast<int64_t>(kFwdBM) * hm.NB + 1) * H * 2 < (int64_t{1} << 31);
+}
+
 template <typename T>
 int launch_me_fwd(const void* x, const void* weight, const void* bias, const int64_t* offsets,
                   const int64_t* dim_inputs, const HostMask& hm, int64_t M, int64_t H, void* pre, void* out,
-                  hipStream_t stream) {
+                  hipStream_t stream, const MlpApply& ap = MlpApply{}) {
   const char* op = "mask_estimator_final_forward";
   PMSST_REQUIRE(M >= 0 && M < (int64_t{1} << 31), "%s: bad row count", op);
   if (M == 0) return PMSST_OK;
-  PMSST_REQUIRE(x && weight && bias && offsets && pre && out, "%s: null pointer", op);
+  PMSST_REQUIRE(x && weight && bias && offsets && pre && (out || ap.est), "%s: null pointer", op);
   MaskArgs a{offsets, M, hm.NB, static_cast<int>(H), hm.F, false};
   a.vec4 = hm.vec4 && al(x, 4 * sizeof(T)) && al(weight, 4 * sizeof(T)) && al(pre, 4 * sizeof(T)) &&
            al(out, 4 * sizeof(T));
@@ -1078,8 +1102,7 @@ int launch_me_fwd(const void* x, const void* weight, const void* bias, const int
   // two K chunks, 16-byte aligned rows: the DMA-pipelined kernel
   if constexpr (sizeof(T) == 2) {
     if (PMSST_ME_FWD_DMA && a.vec4 && H % 8 == 0 && H > kChunkK && al(x, 16) && al(weight, 16) &&
-        al(bias, 4 * sizeof(T)) && (2 * static_cast<int64_t>(hm.max_width) + 1) * H * 2 < (int64_t{1} << 31) &&
-        (static_cast<int64_t>(kFwdBM) * hm.NB + 1) * H * 2 < (int64_t{1} << 31)) {
+        al(bias, 4 * sizeof(T)) && me_fwd_dma_offsets_ok(hm, H)) {
       BandSched sc;
       uint32_t per_xcd = 0;
       const bool sched =
@@ -1087,12 +1110,18 @@ int launch_me_fwd(const void* x, const void* weight, const void* bias, const int
                                     hm.NB, (M + kFwdBM - 1) / kFwdBM,
                                     [&](int b) { return (dim_inputs[b] + 63) / 64; }, &sc, &per_xcd);
       const dim3 g(sched ? per_xcd * kXcds : grid.x);
-      hipLaunchKernelGGL((me_fwd_dma_kernel<T>), g, dim3(kGemmThreads), 0, stream, static_cast<const T*>(x),
-                         static_cast<const T*>(weight), static_cast<const T*>(bias), static_cast<T*>(pre),
-                         static_cast<T*>(out), max_lchunks, xg, a, sc);
+      if (ap.est != nullptr)
+        hipLaunchKernelGGL((me_fwd_dma_kernel<T, true>), g, dim3(kGemmThreads), 0, stream, static_cast<const T*>(x),
+                           static_cast<const T*>(weight), static_cast<const T*>(bias), static_cast<T*>(pre),
+                           static_cast<T*>(out), max_lchunks, xg, a, sc, ap);
+      else
+        hipLaunchKernelGGL((me_fwd_dma_kernel<T, false>), g, dim3(kGemmThreads), 0, stream, static_cast<const T*>(x),
+                           static_cast<const T*>(weight), static_cast<const T*>(bias), static_cast<T*>(pre),
+                           static_cast<T*>(out), max_lchunks, xg, a, sc, ap);
       return check_launch("me_fwd_dma_kernel");
     }
   }
+  PMSST_REQUIRE(ap.est == nullptr, "%s: the mask product needs the DMA-pipelined kernel", op);
   BandSched sc;  // sc.m_tiles = 0 (the XcdGrid, whose blocks past a band's width exit) past 256 bands
   uint32_t per_xcd = 0;
   const dim3 g(build_even_sched(hm.NB, (M + kFwdBM - 1) / kFwdBM, [&](int b) { return (dim_inputs[b] + 63) / 64; },
@@ -1283,6 +1312,10 @@ int launch_uniform_dw_impl(const void* dy, const void* x, void* dw, void* db, in
   return check_launch("me_bwd_dw_dma_kernel");
 }
 
+bool mask_shape(const int64_t* dim_inputs, int64_t band_count, int64_t H, HostMask* hm) {
+  return check_mask("mask_mlp_forward", dim_inputs, band_count, H, hm) == PMSST_OK;
+}
+
 template <typename F>
 int with_dtype(int dtype, const char* op, F&& f) {
   switch (dtype) {
@@ -1294,6 +1327,24 @@ int with_dtype(int dtype, const char* op, F&& f) {
 }
 
 }  // namespace
+
+bool mask_final_supported(const int64_t* dim_inputs, int64_t band_count, int64_t H) {
+  HostMask hm;
+  return mask_shape(dim_inputs, band_count, H, &hm) && hm.vec4 && H % 8 == 0 && H > kChunkK && me_fwd_dma_offsets_ok(hm, H);
+}
+
+template <typename T>
+int launch_mask_final(const void* x, const void* weight, const void* bias, const int64_t* offsets,
+                      const int64_t* dim_inputs, int64_t band_count, int64_t M, int64_t H, void* pre, void* out,
+                      const MlpApply& ap, hipStream_t stream) {
+  HostMask hm;
+  if (!mask_shape(dim_inputs, band_count, H, &hm)) return PMSST_EINVAL;
+  return launch_me_fwd<T>(x, weight, bias, offsets, dim_inputs, hm, M, H, pre, out, stream, ap);
+}
+template int launch_mask_final<bf16>(const void*, const void*, const void*, const int64_t*, const int64_t*, int64_t,
+                                     int64_t, int64_t, void*, void*, const MlpApply&, hipStream_t);
+template int launch_mask_final<f16>(const void*, const void*, const void*, const int64_t*, const int64_t*, int64_t,
+                                    int64_t, int64_t, void*, void*, const MlpApply&, hipStream_t);
 
 bool uniform_dw_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
                           const void* dy, const void* x, const void* dw) {

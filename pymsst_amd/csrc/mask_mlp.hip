@@ -35,6 +35,8 @@
 
 #include "common.h"
 #include "dma_gemm.h"
+#include "grouped_dx.h"
+#include "mask_mlp.h"
 #include "ring.h"
 
 
@@ -49,17 +51,6 @@ constexpr int kTanhBytes = kTanhEntries * 2;
 
 // tanh tables: [bf16 patterns | fp16 patterns], filled once per device from the host
 __device__ __align__(256) uint16_t g_tanh_tables[2 * kTanhEntries];
-
-// Mask application in the epilogue (stem s of S): est[b, s, c, f, t] = spec[b, f C + c, t] x the
-// complex mask (out[m, 2 r], out[m, 2 r + 1]) of row m = b T + t, complex row r = f C + c, in the
-// iSTFT layout [B * S * C, Fbins, T] (complex64); bin 0 zero when zero_dc.  The mask values are
-// rounded to the storage dtype first, as the stored mask the stock product multiplies is.
-struct MlpApply {
-  const float2* spec;  // complex64 [B, Fbins * C, T]
-  float2* est;         // complex64 [B * S * C, Fbins, T]
-  FastDiv frames;      // T
-  int C, Fbins, S, s, zero_dc;
-};
 
 struct MlpArgs {
   const int64_t* offsets;  // device [NB + 1] prefix sums of I_b
@@ -420,16 +411,7 @@ __device__ __forceinline__ void mlp_fwd_block(const T* __restrict__ x, const T* 
         const int r0 = (off + j) >> 1;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-          const int r = r0 + q;
-          const int f = r / ap.C, c = r - f * ap.C;
-          // the mask rounded to the storage dtype, as the stored mask is
-          const float mr = to_f32(from_f32<T>(vo[2 * q])), mi = to_f32(from_f32<T>(vo[2 * q + 1]));
-          const float2 sv = spv[t][n][q];
-          float2 e = make_float2(sv.x * mr - sv.y * mi, sv.x * mi + sv.y * mr);
-          if (ap.zero_dc && f == 0) e = make_float2(0.f, 0.f);
-          ap.est[((static_cast<int64_t>(bbn[n]) * ap.S + ap.s) * ap.C + c) * static_cast<int64_t>(ap.Fbins) *
-                     ap.frames.d +
-                 static_cast<int64_t>(f) * ap.frames.d + ttn[n]] = e;
+          store_masked<T>(ap, bbn[n], ttn[n], r0 + q, spv[t][n][q], vo[2 * q], vo[2 * q + 1]);
         }
       } else {
         store_pack<T, 4>(out + m * a.F + off + j, vo);
@@ -600,6 +582,18 @@ int launch_mlp_fwd(const void* x, const void* w1, const void* b1, const void* w2
   }
 }
 
+// Whether a hidden-layer and a final-layer kernel beat the one pass when the hidden layer is stored anyway.
+// The one pass recomputes GEMM1 for every 64 GLU outputs past a band's first, and from dim 384 on its
+// x fragments leave it 4 waves of 32 rows; the two kernels read the hidden layer once more.  Forward
+// with the hidden layer stored: dim 512, 62 bands, 1896 rows 770 -> 600 us; 60 mel bands (2.5 passes a
+// band), dim 192, 2760 rows 375 -> 346 us; 62 bands (1.6 passes), dim 192, 1032 rows 99 -> 131 us, so
+// there the one pass stays.
+bool two_kernels_better(int64_t dim, const int64_t* dim_inputs, int64_t band_count) {
+  int64_t passes = 0;
+  for (int64_t b = 0; b < band_count; ++b) passes += (dim_inputs[b] + kMlpJ - 1) / kMlpJ;
+  return dim >= 384 || passes > 2 * band_count;
+}
+
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
 }  // namespace
@@ -628,6 +622,17 @@ int mask_mlp_forward_impl(const char* op, const void* x, const void* w1, const v
   int64_t total = 0;
   for (int64_t b = 0; b < band_count; ++b) total += dim_inputs[b];
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (hidden_out != nullptr && two_kernels_better(dim, dim_inputs, band_count) &&
+      wide_tanh_supported(band_count, dim, hidden, rows, 2, x, w1, b1, hidden_out) &&
+      mask_final_supported(dim_inputs, band_count, hidden)) {
+    auto two = [&](auto tag) {
+      using T = decltype(tag);
+      const int rc = launch_wide_tanh<T>(x, w1, b1, hidden_out, band_count, dim, hidden, rows, s);
+      if (rc != PMSST_OK) return rc;
+      return launch_mask_final<T>(hidden_out, w2, b2, dim_offsets, dim_inputs, band_count, rows, hidden, pre, out, ap, s);
+    };
+    return dtype == PMSST_BF16 ? two(bf16{}) : two(f16{});
+  }
   const uint16_t* tabs = nullptr;
   const int rc = tanh_tables(s, &tabs);
   if (rc != PMSST_OK) return rc;
