@@ -68,6 +68,7 @@ struct BandArgs {
 // last valid row in interior chunks (their outputs and sums are discarded).
 template <typename T, bool NORM, bool V4>
 struct XGammaLoader {
+  static constexpr bool kTransposed = false;
   static constexpr int kQuads = kBM * (kChunkK / 4) / kGemmThreads;
   static_assert(kQuads == 2, "two rows per thread");
   struct Regs {
@@ -114,13 +115,14 @@ struct XGammaLoader {
       fetch_edge(k0, g);
     }
   }
+  template <bool SPLIT>
   __device__ __forceinline__ void commit_impl(const Regs& g, T* lds, bool masked) const {
     const int kq = lane_k();
     if constexpr (!NORM) {
       // plain grouped linear: no gamma, no sums of squares
 #pragma unroll
       for (int i = 0; i < kQuads; ++i)
-        commit_quad<T>(lds, tile_row(i), kq, masked ? mask_quad<T>(g.q[i], (g.ok >> i) & 1) : g.q[i]);
+        commit_quad<T, kBM, SPLIT>(lds, tile_row(i), kq, masked ? mask_quad<T>(g.q[i], (g.ok >> i) & 1) : g.q[i]);
       return;
     }
     float gm[4];
@@ -135,15 +137,17 @@ struct XGammaLoader {
         ss[i] += v[j] * v[j];
         pk.v[j] = from_f32<T>(v[j] * gm[j]);
       }
-      commit_quad<T>(lds, tile_row(i), kq, __builtin_bit_cast(quad_t<T>, pk));
+      commit_quad<T, kBM, SPLIT>(lds, tile_row(i), kq, __builtin_bit_cast(quad_t<T>, pk));
     }
   }
-  __device__ __forceinline__ void commit_edge(const Regs& g, T* lds) const { commit_impl(g, lds, true); }
-  __device__ __forceinline__ void commit(const Regs& g, T* lds) const { commit_impl(g, lds, !V4); }
+  template <bool SPLIT>
+  __device__ __forceinline__ void commit_edge(const Regs& g, T* lds) const { commit_impl<SPLIT>(g, lds, true); }
+  template <bool SPLIT>
+  __device__ __forceinline__ void commit(const Regs& g, T* lds) const { commit_impl<SPLIT>(g, lds, !V4); }
 };
 
 template <typename T, int TO, bool WRITE_NORMED, bool NORM, int ACT, bool V4>
-__global__ __launch_bounds__(kGemmThreads) void bs_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1))) void bs_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                               const T* __restrict__ weight,
                                                               const T* __restrict__ bias, T* __restrict__ out,
                                                               T* __restrict__ normed, float* __restrict__ inv_norm,
@@ -312,8 +316,14 @@ __device__ __forceinline__ bool bs_dx_block(const BandSched& sc, const XcdGrid& 
   return true;
 }
 
+// Rows of a block's tile: 64, or 128 for fp32 without the norm (the grouped linear: the weight chunk is
+// read half as often and a wave's fragments serve twice the products; 190 -> 160 us for 62 groups of
+// 192 -> 768 at 1032 rows).  With the norm the partials have 64 rows.
+template <typename T, bool NORM>
+constexpr int bs_dx_rows() { return sizeof(T) == 4 && !NORM ? 128 : 64; }
+
 template <typename T, bool FROM_X, bool NORM, bool V4>
-__global__ __launch_bounds__(kGemmThreads) void bs_bwd_dx_kernel(const T* __restrict__ dy,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void bs_bwd_dx_kernel(const T* __restrict__ dy,
                                                                  const T* __restrict__ nsrc,
                                                                  const float* __restrict__ inv_norm,
                                                                  const T* __restrict__ gamma,
@@ -324,57 +334,65 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dx_kernel(const T* __rest
                                                                  int max_ichunks, XcdGrid xg, BandSched sc,
                                                                  BandArgs a) {
   constexpr int kBI = 64;
-  __shared__ T lds[gemm_lds_elems<T, kBI, kBM>()];
-  __shared__ float sinv[kBM];
-  __shared__ float sdot[4][kBM];
-  using S = TileShape<kBI, kBM, 4, 1>;  // TR = 1, TC = 4
+  constexpr int BM = bs_dx_rows<T, NORM>();
+  __shared__ T lds[gemm_lds_elems<T, kBI, BM>()];
+  __shared__ float sinv[BM];
+  __shared__ float sdot[4][BM];
+  constexpr int WR = BM == 64 ? 4 : 2, WC = 4 / WR;
+  using S = TileShape<kBI, BM, WR, WC>;  // 64 rows: TR = 1, TC = 4; 128: TR = 2, TC = 4
 
   const int O = a.O;
   int band, ichunk;
   uint32_t mt;
   if (!bs_dx_block(sc, xg, max_ichunks, a.NB, blockIdx.x, band, ichunk, mt)) return;
   const int64_t mtile = mt;
-  const int64_t m0 = mtile * kBM;
+  const int64_t m0 = mtile * BM;
   const int off = static_cast<int>(a.offsets[band]);
   const int I = static_cast<int>(a.offsets[band + 1]) - off;
   const int i0 = ichunk * kBI;
   if (i0 >= I) return;  // uniform over the block
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rows_valid = static_cast<int>(a.M - m0 < kBM ? a.M - m0 : kBM);
+  const int rows_valid = static_cast<int>(a.M - m0 < BM ? a.M - m0 : BM);
   const T* wb = weight + static_cast<int64_t>(O) * off;  // [O][I]
   const T* dyb = dy + (m0 * a.NB + band) * O;
   const float root = sqrtf(static_cast<float>(I));
 
   if (NORM) {
-    if (tid < kBM) sinv[tid] = tid < rows_valid ? inv_norm[(m0 + tid) * a.NB + band] : 0.f;
+    if (tid < BM) sinv[tid] = tid < rows_valid ? inv_norm[(m0 + tid) * a.NB + band] : 0.f;
     __syncthreads();
   }
 
   // A[i][o] = W_b[o][i0 + i] (MN-contiguous in i);  B[m][o] = dy[m0 + m][band][o]
   MNLoader<T, kBI, V4> la{wb + i0, I, I - i0, O};
-  KRowLoader<T, kBM, V4> lb{dyb, static_cast<int64_t>(a.NB) * O, rows_valid, O};
+  KRowLoader<T, BM, V4> lb{dyb, static_cast<int64_t>(a.NB) * O, rows_valid, O};
   f32x4_t acc[S::kTR][S::kTC];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc[0][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gemm_mainloop<T, kBI, kBM, 4, 1, PMSST_BS_DX_DEPTH>(la, lb, O, lds, acc);
-
-  // lane holds gs[m = 16 j + (lane & 15)][i = i0 + 16 wave + 4 (lane >> 4) + r]
-  const int il = i0 + wave * 16 + 4 * (lane >> 4);
-  if (!NORM) {
+  for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int m = j * 16 + (lane & 15);
-      if (m >= rows_valid || il >= I) continue;
-      float o[4] = {acc[0][j][0], acc[0][j][1], acc[0][j][2], acc[0][j][3]};
-      T* dp = dx + (m0 + m) * a.F + off + il;
-      if (a.vec4) {
-        store_pack<T, 4>(dp, o);
-      } else {
-        for (int r = 0; r < 4 && il + r < I; ++r) dp[r] = from_f32<T>(o[r]);
+    for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  gemm_mainloop<T, kBI, BM, WR, WC, PMSST_BS_DX_DEPTH>(la, lb, O, lds, acc);
+
+  if constexpr (!NORM) {
+#pragma unroll
+    for (int i = 0; i < S::kTR; ++i) {
+      const int ii = i0 + (wave / WC) * (kBI / WR) + 16 * i + 4 * (lane >> 4);
+#pragma unroll
+      for (int j = 0; j < S::kTC; ++j) {
+        const int m = (wave % WC) * (BM / WC) + j * 16 + (lane & 15);
+        if (m >= rows_valid || ii >= I) continue;
+        float o[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+        T* dp = dx + (m0 + m) * a.F + off + ii;
+        if (a.vec4) {
+          store_pack<T, 4>(dp, o);
+        } else {
+          for (int r = 0; r < 4 && ii + r < I; ++r) dp[r] = from_f32<T>(o[r]);
+        }
       }
     }
     return;
   }
+  // lane holds gs[m = 16 j + (lane & 15)][i = i0 + 16 wave + 4 (lane >> 4) + r]
+  const int il = i0 + wave * 16 + 4 * (lane >> 4);
   float g[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) g[r] = il + r < I ? to_f32(gamma[off + il + r]) : 0.f;
@@ -522,16 +540,20 @@ __global__ __launch_bounds__(256) void bs_dx_finish_kernel(const float* __restri
 // ------------------------------------------------------------------ backward: dW
 
 constexpr int kDwBI = 64;
-constexpr int kDwBO = 64;
+// Output columns of a block: 128 for the fp32 grouped linear (768 of them and K = the rows: the x slab is
+// read half as often, and a wave's fragments serve twice the products), else 64.
+template <typename T, bool NORM>
+constexpr int dw_cols() { return sizeof(T) == 4 && !NORM ? 128 : 64; }
 
 // NORM = false: plain grouped linear, dW_b^T = x_b^T dy_b (no gamma / inv_norm scaling).
 template <typename T, bool FROM_X, bool NORM, bool V4>
-__global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_kernel(const T* __restrict__ dy,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void bs_bwd_dw_kernel(const T* __restrict__ dy,
                                                                  const T* __restrict__ nsrc,
                                                                  const float* __restrict__ inv_norm,
                                                                  const T* __restrict__ gamma, T* __restrict__ dw,
                                                                  T* __restrict__ db, int max_itiles, XcdGrid xg,
                                                                  BandSched sc, BandArgs a) {
+  constexpr int kDwBO = dw_cols<T, NORM>();
   __shared__ T lds[gemm_lds_elems<T, kDwBI, kDwBO>()];
   using S = TileShape<kDwBI, kDwBO, 2, 2>;
   const int O = a.O;
@@ -1125,10 +1147,10 @@ int check_bands(const char* op, const int64_t* dim_inputs, int64_t band_count, H
   return PMSST_OK;
 }
 
-// Grid of bs_bwd_dw_kernel: one block per existing (band, 64-wide input tile, 64-wide output tile)
+// Grid of bs_bwd_dw_kernel: one block per existing (band, 64-wide input tile, `cols`-wide output tile)
 // on an even XCD schedule; past the schedule's band count sc->m_tiles = 0 and the XcdGrid.
-uint32_t dw_grid(const HostBands& hb, int64_t O, const XcdGrid& xg, BandSched* sc) {
-  const int64_t otiles = (O + kDwBO - 1) / kDwBO;
+uint32_t dw_grid(const HostBands& hb, int64_t O, int64_t cols, const XcdGrid& xg, BandSched* sc) {
+  const int64_t otiles = (O + cols - 1) / cols;
   uint32_t per_xcd = 0;
   if (build_even_sched(hb.NB, 1, [&](int b) { return (hb.widths[b] + kDwBI - 1) / kDwBI * otiles; }, sc, &per_xcd))
     return per_xcd * kXcds;
@@ -1323,8 +1345,9 @@ int launch_bwd(const void* dy, const void* nsrc, bool from_x, const float* inv_n
   if (!dw_done) {
     BandSched wsc;
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kDwBO - 1) / kDwBO)};
-    const dim3 grid(dw_grid(hb, O, xg, &wsc));
+    constexpr int kCols = dw_cols<T, true>();
+    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kCols - 1) / kCols)};
+    const dim3 grid(dw_grid(hb, O, kCols, xg, &wsc));
     const bool v4 = a.vec4 && a.ovec4;
 #define PMSST_BDW(FX, V4)                                                                                   \
   hipLaunchKernelGGL((bs_bwd_dw_kernel<T, FX, true, V4>), grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm, \
@@ -1374,7 +1397,8 @@ int launch_grouped_bwd(const void* dy, const void* x, const void* weight, const 
     }
   } else if (M > 0) {
     const int max_ichunks = (hb.max_width + 63) / 64;
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>((M + kBM - 1) / kBM)};
+    constexpr int kRows = bs_dx_rows<T, false>();
+    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>((M + kRows - 1) / kRows)};
     const dim3 grid(xg.blocks());
     const BandSched nosc{};  // groups of one width: every XcdGrid block has a chunk
     if (a.vec4 && a.ovec4)
@@ -1400,9 +1424,10 @@ int launch_grouped_bwd(const void* dy, const void* x, const void* weight, const 
     }
   } else {
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kDwBO - 1) / kDwBO)};
+    constexpr int kCols = dw_cols<T, false>();
+    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kCols - 1) / kCols)};
     BandSched wsc;
-    const dim3 grid(dw_grid(hb, O, xg, &wsc));
+    const dim3 grid(dw_grid(hb, O, kCols, xg, &wsc));
     if (a.vec4 && a.ovec4)
       hipLaunchKernelGGL((bs_bwd_dw_kernel<T, false, false, true>), grid, dim3(kGemmThreads), 0, stream, pdy, px,
                          nullptr, nullptr, static_cast<T*>(dw), static_cast<T*>(db), max_itiles, xg, wsc, a);
@@ -1524,7 +1549,7 @@ int launch_mixed_bwd(const void* dy, const float* x, int64_t x_stride, const voi
   float* partial = reinterpret_cast<float*>(ws + mixed_g_bytes(M, hb.F) + mixed_dot_bytes(M, hb.NB));
   if (M > 0) {
     // g = T(dy W_b): the norm-free dx kernel, one block per existing (band, row tile, 64-wide chunk)
-    const int m_tiles = static_cast<int>((M + kBM - 1) / kBM);
+    const int m_tiles = static_cast<int>((M + bs_dx_rows<T, false>() - 1) / bs_dx_rows<T, false>());
     const int max_ichunks = (hb.max_width + 63) / 64;
     const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>(m_tiles)};
     BandSched sc;
@@ -1554,9 +1579,10 @@ int launch_mixed_bwd(const void* dy, const float* x, int64_t x_stride, const voi
   // runs for M == 0 and then writes zeros)
   {
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kDwBO - 1) / kDwBO)};
+    constexpr int kCols = dw_cols<T, false>();
+    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kCols - 1) / kCols)};
     BandSched wsc;
-    const dim3 grid(dw_grid(hb, O, xg, &wsc));
+    const dim3 grid(dw_grid(hb, O, kCols, xg, &wsc));
     if (a.vec4 && a.ovec4)
       hipLaunchKernelGGL((bs_bwd_dw_kernel<T, false, false, true>), grid, dim3(kGemmThreads), 0, stream, pdy, pu,
                          nullptr, nullptr, static_cast<T*>(dw), static_cast<T*>(db), max_itiles, xg, wsc, a);

@@ -10,7 +10,18 @@
 // i.e. the four 16-byte k-units of a row are XOR-swizzled by the row's 16-row
 // group.  MFMA fragment reads (16 consecutive rows, one unit) stay 16-byte
 // aligned and conflict-free, and the transposed stores of MNLoader (8 bytes to
-// rows 4q..4q+3) spread over all banks.  fp32 tiles use a plain odd pitch.
+// rows 4q..4q+3) spread over all banks.
+//
+// fp32: each value is split on its way into LDS into three bf16 numbers, x = x1 + x2 + x3 (each the
+// rest's round-to-nearest bf16; 8 + 8 + 8 significant bits, so the sum is exact), and a product is the
+// six bf16 MFMAs a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1 with fp32 accumulation; the three left out are
+// below 2^-25 of it.  bf16 products are exact in fp32, so the result's error stays that of the fp32 sums
+// (measured against 64 bits: no larger than with the fp32 MFMAs), at 6 x 16 matrix-core cycles per 16 x 16
+// x 32 instead of 8 x 32, and 3 LDS reads of 16 bytes per fragment instead of 8 of 4.  A tile holds three
+// planes, of 64-byte rows (swz_k)
+// or, from an MNLoader, of 32 K-rows as they are stored (swz_mn_p; read transposed).  A non-finite accumulator (an infinity or a NaN among the inputs, or
+// one above bf16's largest, whose split is not finite; or an overflow) sends the block through the sum
+// again on the fp32 MFMAs, which give such inputs their usual results.
 //
 // Waves are laid out WR x WC over the tile; wave (wr, wc) owns rows
 // [wr * BR/WR, ...) and columns [wc * BC/WC, ...) as TR x TC 16x16 tiles.
@@ -29,6 +40,49 @@
 namespace pmsst {
 
 constexpr int kGemmThreads = 256;
+
+// ---------------------------------------------------------------- LDS swizzles and fragment reads
+// ds_read_b128 serves 16 lanes a cycle: lanes 0-3, 12-15, 20-27, then 4-11, 16-19, 28-31, and the
+// same of the upper half.  In a fragment read those are rows 0-3 and 12-15 of one unit and rows 4-11
+// of the next (or the reverse), and rows 4 apart share a bank quarter at the 64-byte pitch, so the
+// swizzles s(q) of the row quads q must make s(0), s(3), 1 ^ s(1), 1 ^ s(2) distinct: s = 0, 3, 2, 1.
+// (s = 0, 1, 2, 3 and (r / 2) ^ (r / 8) collide two by two.)  GEMM1 of the one-pass MLP reads rows
+// 8 (r / 4) + r % 4 (+ 4), which s = 0, 3, 2, 1 spreads too.
+__device__ __forceinline__ int swz_k(int r) { return -(r >> 2) & 3; }
+// A transpose read takes 8 bytes of each of 32 lanes a cycle: K-rows k, k + 1, k + 2, k + 3 and the
+// same + 8, 32 bytes of each, which must fill the 256 bytes of the 64 banks.  At a pitch of whole
+// 256 bytes every row starts on bank 0, so the 8 rows take 8 different unit pairs; at an odd multiple
+// of 128 bytes odd rows start half way round, and the 4 rows of a parity take the 4 pairs of a half.
+// Rows k and k + 4 keep the same swizzle, as the second read of a fragment needs.  The swizzle stays
+// inside aligned groups of 16 (or 8) units, which the pitch holds whole.
+template <int PITCH>
+__device__ __forceinline__ int swz_mn_p(int k) {
+  static_assert(PITCH % 128 == 0, "rows of whole 128 bytes");
+  if constexpr (PITCH % 256 == 0) return 2 * ((k & 3) | (((k >> 3) & 1) << 2));
+  else return 2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1));
+}
+
+// First of the two transpose reads of an MN-contiguous fragment (columns c0 .. c0 + 15,
+// c0 % 16 == 0, row pitch PITCH bytes); the second is at + 4 * PITCH.
+template <int PITCH>
+__device__ __forceinline__ uint32_t frag_mn_addr_p(uint32_t region, int c0, int lane) {
+  const int j = lane & 15, g = lane >> 4;
+  const int k = 8 * g + (j >> 2);                // K-row of this lane's 4 elements
+  const int col = c0 + 4 * (j & 3);
+  const int unit = col >> 3;
+  return region + static_cast<uint32_t>(k * PITCH + 16 * (unit ^ swz_mn_p<PITCH>(k)) + 2 * (col & 7));
+}
+
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+
+// Transposed fragment (two ds_read_b64_tr_b16 through the compiler's builtin, which it waits for)
+__device__ __forceinline__ u32x4_t tr_frag(const char* p, int step) {
+  typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
+  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
+  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + step));
+  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
+  return u32x4_t{a.x, a.y, b.x, b.y};
+}
 
 template <typename T>
 __device__ __forceinline__ int lds_index(int r, int k) {
@@ -71,6 +125,53 @@ using raw_t = typename std::conditional<sizeof(T) == 2, uint16_t, uint32_t>::typ
 // 4 consecutive elements as raw bits: 8 bytes for 16-bit types, 16 for fp32.
 template <typename T>
 using quad_t = typename std::conditional<sizeof(T) == 2, uint2, uint4>::type;
+
+// LDS floats per tile row of the fp32 path: three bf16 planes of 64 bytes (the fp32 re-run's rows of
+// LdsPitch<float> fit in them).
+constexpr int kSplitRow = 48;
+static_assert(kSplitRow >= LdsPitch<float>::value, "the fp32 re-run's tile fits");
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+// Two fp32 values as three words of two bf16 each, high part first.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&w)[3]) {
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    w[p] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
+    if (p < 2) {
+      a -= __uint_as_float(w[p] << 16);
+      b -= __uint_as_float(w[p] & 0xffff0000u);
+    }
+  }
+}
+
+// Byte offset of element (r, k) inside plane 0 of a split tile; plane p is p * ROWS * 64 bytes on.
+__device__ __forceinline__ int split_offset(int r, int k) {
+  return r * 64 + 16 * ((k >> 3) ^ swz_k(r & 15)) + 2 * (k & 7);
+}
+
+// 4 consecutive k (k % 4 == 0) of row r into the three planes.
+template <int ROWS>
+__device__ __forceinline__ void put_split(float* lds, int r, int k, const float (&v)[4]) {
+  char* dst = reinterpret_cast<char*>(lds) + split_offset(r, k);
+  uint32_t lo[3], hi[3];
+  split_pair(v[0], v[1], lo);
+  split_pair(v[2], v[3], hi);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(dst + p * ROWS * 64) = make_uint2(lo[p], hi[p]);
+}
+
+// 4 consecutive rows mn (mn % 4 == 0) of K-row k into the three planes of a tile that keeps K-rows.
+template <int ROWS>
+__device__ __forceinline__ void put_split_mn(float* lds, int mn, int k, const float (&v)[4]) {
+  char* dst = reinterpret_cast<char*>(lds) + k * 2 * ROWS + 16 * ((mn >> 3) ^ swz_mn_p<2 * ROWS>(k)) + 2 * (mn & 7);
+  uint32_t lo[3], hi[3];
+  split_pair(v[0], v[1], lo);
+  split_pair(v[2], v[3], hi);
+#pragma unroll
+  for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(dst + p * ROWS * 64) = make_uint2(lo[p], hi[p]);
+}
 
 template <typename T>
 __device__ __forceinline__ quad_t<T> raw_quad(const T* p) {
@@ -146,10 +247,13 @@ __device__ __forceinline__ void quad_to_f32(const quad_t<T>& q, float (&o)[4]) {
   }
 }
 
-// Stores a quad of consecutive k (kq % 4 == 0) of LDS row r.
-template <typename T>
+// Stores a quad of consecutive k (kq % 4 == 0) of LDS row r (SPLIT: fp32 as three bf16 planes).
+template <typename T, int ROWS, bool SPLIT>
 __device__ __forceinline__ void commit_quad(T* lds, int r, int kq, const quad_t<T>& q) {
-  if constexpr (sizeof(T) == 2) {
+  if constexpr (SPLIT) {
+    const float v[4] = {__uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z), __uint_as_float(q.w)};
+    put_split<ROWS>(lds, r, kq, v);
+  } else if constexpr (sizeof(T) == 2) {
     *reinterpret_cast<uint2*>(lds + lds_index<T>(r, kq)) = q;
   } else {
     uint32_t* row = reinterpret_cast<uint32_t*>(lds);
@@ -165,6 +269,7 @@ __device__ __forceinline__ void commit_quad(T* lds, int r, int kq, const quad_t<
 // r < rows_valid; prepare_rows() lets a kernel map tile rows to other source rows.
 template <typename T, int ROWS, bool V4>
 struct KRowLoader {
+  static constexpr bool kTransposed = false;  // the split tile's layout: rows
   static constexpr int kQuads = ROWS * (kChunkK / 4) / kGemmThreads;
   static_assert(kQuads >= 1 && ROWS * (kChunkK / 4) % kGemmThreads == 0, "tile too small");
   struct Regs {
@@ -209,9 +314,11 @@ struct KRowLoader {
     for (int i = 0; i < kQuads; ++i)
       g.q[i] = fetch_quad_k<T, V4>(base + src_row[i] * stride + k, base, row_ok(i), k, k_valid, g.ok, i);
   }
+  template <bool SPLIT>
   __device__ __forceinline__ void commit_edge(const Regs& g, T* lds) const {
 #pragma unroll
-    for (int i = 0; i < kQuads; ++i) commit_quad<T>(lds, tile_row(i), lane_k(), mask_quad<T>(g.q[i], (g.ok >> i) & 1));
+    for (int i = 0; i < kQuads; ++i)
+      commit_quad<T, ROWS, SPLIT>(lds, tile_row(i), lane_k(), mask_quad<T>(g.q[i], (g.ok >> i) & 1));
   }
   __device__ __forceinline__ void fetch(int k0, Regs& g) const {
     if constexpr (V4) {
@@ -221,12 +328,13 @@ struct KRowLoader {
       fetch_edge(k0, g);
     }
   }
+  template <bool SPLIT>
   __device__ __forceinline__ void commit(const Regs& g, T* lds) const {
     if constexpr (V4) {
 #pragma unroll
-      for (int i = 0; i < kQuads; ++i) commit_quad<T>(lds, tile_row(i), lane_k(), g.q[i]);
+      for (int i = 0; i < kQuads; ++i) commit_quad<T, ROWS, SPLIT>(lds, tile_row(i), lane_k(), g.q[i]);
     } else {
-      commit_edge(g, lds);
+      commit_edge<SPLIT>(g, lds);
     }
   }
 };
@@ -241,6 +349,7 @@ struct KRowLoader {
 // are transposed as raw bits (byte permutes, no conversions).
 template <typename T, int ROWS, bool V4>
 struct MNLoader {
+  static constexpr bool kTransposed = true;  // the split tile's layout: K-rows
   static constexpr int kQuadsPerK = ROWS / 4;
   static constexpr int KB = ROWS / 32;
   static_assert(KB >= 1 && KB * kQuadsPerK * (kChunkK / KB) == ROWS * kChunkK / 4, "tile shape");
@@ -308,6 +417,7 @@ struct MNLoader {
   }
 
   // Float path: optional masking of k rows (edge), column sums, scales.
+  template <bool SPLIT>
   __device__ __forceinline__ void commit_f32(const Regs& g, T* lds, bool masked) const {
     const int mn = lane_mn();
     const int kb = lane_kb();
@@ -322,6 +432,11 @@ struct MNLoader {
       const float st = rs != nullptr ? g.s[t] * rs_mul : 1.f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[t][j] *= st * c[j];
+    }
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int t = 0; t < KB; ++t) put_split_mn<ROWS>(lds, mn, kb + t, v[t]);
+      return;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -362,18 +477,20 @@ struct MNLoader {
       }
     }
   }
-  __device__ __forceinline__ void commit_edge(const Regs& g, T* lds) const { commit_f32(g, lds, true); }
+  template <bool SPLIT>
+  __device__ __forceinline__ void commit_edge(const Regs& g, T* lds) const { commit_f32<SPLIT>(g, lds, true); }
+  template <bool SPLIT>
   __device__ __forceinline__ void commit(const Regs& g, T* lds) const {
     if constexpr (!V4) {
-      commit_f32(g, lds, true);
+      commit_f32<SPLIT>(g, lds, true);
     } else if constexpr (sizeof(T) == 2) {
       if (cs == nullptr && rs == nullptr && !colsum) {
         commit_raw16(g, lds);
       } else {
-        commit_f32(g, lds, false);
+        commit_f32<false>(g, lds, false);
       }
     } else {
-      commit_f32(g, lds, false);
+      commit_f32<SPLIT>(g, lds, false);
     }
   }
 };
@@ -436,10 +553,137 @@ struct TileShape {
   static_assert(kTR >= 1 && kTC >= 1 && BR % (WR * 16) == 0 && BC % (WC * 16) == 0, "bad tile");
 };
 
-// LDS elements the main loop needs for a BR x BC tile (two buffers).
+// LDS elements the main loop needs for a BR x BC tile (16-bit: two buffers; fp32: one split tile).
 template <typename T, int BR, int BC>
 constexpr int gemm_lds_elems() {
-  return 2 * (BR + BC) * LdsPitch<T>::value;
+  return sizeof(T) == 2 ? 2 * (BR + BC) * LdsPitch<T>::value : (BR + BC) * kSplitRow;
+}
+
+// Register budget of the fp32 kernels with 8 or fewer 16 x 16 tiles a wave, in waves per SIMD: their K
+// steps wait on loads and barriers, which three blocks a CU cover better than two (224 against 228-324
+// us for the mask backward's input gradient).
+constexpr int kSplitWaves = 3;
+
+// The fp32 K loop: one LDS tile, the next chunk's loads in registers while this one is multiplied (the
+// blocks of a CU, two to six of them, cover each other's splits and barriers).  SPLIT: three bf16 planes
+// and six products; else the fp32 MFMAs.
+template <int BR, int BC, int WR, int WC, bool SPLIT, class LA, class LB>
+__device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
+                                              f32x4_t (&acc)[TileShape<BR, BC, WR, WC>::kTR]
+                                                            [TileShape<BR, BC, WR, WC>::kTC]) {
+  using S = TileShape<BR, BC, WR, WC>;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int r0 = (wave / WC) * (BR / WR);
+  const int c0 = (wave % WC) * (BC / WC);
+  const int nk = (K + kChunkK - 1) / kChunkK;
+  const int kbeg = K - nk * kChunkK;  // chunk 0 may be partial
+  float* lds_b = lds + BR * kSplitRow;
+  la.prepare();
+  lb.prepare();
+  typename LA::Regs ra;
+  typename LB::Regs rb;
+  if (kbeg < 0) {
+    la.fetch_edge(kbeg, ra);
+    lb.fetch_edge(kbeg, rb);
+    la.template commit_edge<SPLIT>(ra, lds);
+    lb.template commit_edge<SPLIT>(rb, lds_b);
+  } else {
+    la.fetch(kbeg, ra);
+    lb.fetch(kbeg, rb);
+    la.template commit<SPLIT>(ra, lds);
+    lb.template commit<SPLIT>(rb, lds_b);
+  }
+  // Where the registers allow, the products of the low parts have accumulators of their own, 2^-8 the
+  // size: the matrix cores cut a sum off one-sidedly (column sums of the result, over a thousand rows,
+  // showed it), and so the large accumulators are cut off once a chunk instead of six times.
+  constexpr bool kLow = SPLIT && S::kTR * S::kTC <= 8;
+  f32x4_t low[kLow ? S::kTR : 1][kLow ? S::kTC : 1];
+#pragma unroll
+  for (int i = 0; i < (kLow ? S::kTR : 1); ++i)
+#pragma unroll
+    for (int j = 0; j < (kLow ? S::kTC : 1); ++j) low[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto mma = [&]() {
+    if constexpr (SPLIT) {
+      constexpr int kP[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};  // small parts first
+      auto term = [&](int i, int j, int q, const bf16x8_t (&a)[3], const bf16x8_t (&b)[3]) {
+        f32x4_t& d = kLow && q < 5 ? low[kLow ? i : 0][kLow ? j : 0] : acc[i][j];
+        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kP[q][0]], b[kP[q][1]], d, 0, 0, 0);
+      };
+      auto frag = [&](auto tr, const float* tile, auto rows, int r, int t, bf16x8_t (&f)[3]) {
+        constexpr int ROWS = decltype(rows)::value;
+        const char* base = reinterpret_cast<const char*>(tile);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          if constexpr (decltype(tr)::value)
+            f[p] = __builtin_bit_cast(
+                bf16x8_t, tr_frag(base + p * ROWS * 64 + frag_mn_addr_p<2 * ROWS>(0, r + 16 * t, lane), 4 * 2 * ROWS));
+          else
+            f[p] = *reinterpret_cast<const bf16x8_t*>(base + p * ROWS * 64 +
+                                                      split_offset(r + 16 * t + (lane & 15), 8 * (lane >> 4)));
+        }
+      };
+      using RowsA = std::integral_constant<int, BR>;
+      using RowsB = std::integral_constant<int, BC>;
+      using TrA = std::integral_constant<bool, LA::kTransposed>;
+      using TrB = std::integral_constant<bool, LB::kTransposed>;
+      // the operand with fewer tiles stays in registers, the other's tiles pass by
+      if constexpr (S::kTR <= S::kTC) {
+        bf16x8_t a[S::kTR][3];
+#pragma unroll
+        for (int i = 0; i < S::kTR; ++i) frag(TrA{}, lds, RowsA{}, r0, i, a[i]);
+#pragma unroll
+        for (int j = 0; j < S::kTC; ++j) {
+          bf16x8_t b[3];
+          frag(TrB{}, lds_b, RowsB{}, c0, j, b);
+#pragma unroll
+          for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int i = 0; i < S::kTR; ++i) term(i, j, q, a[i], b);
+        }
+      } else {
+        bf16x8_t b[S::kTC][3];
+#pragma unroll
+        for (int j = 0; j < S::kTC; ++j) frag(TrB{}, lds_b, RowsB{}, c0, j, b[j]);
+#pragma unroll
+        for (int i = 0; i < S::kTR; ++i) {
+          bf16x8_t a[3];
+          frag(TrA{}, lds, RowsA{}, r0, i, a);
+#pragma unroll
+          for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int j = 0; j < S::kTC; ++j) term(i, j, q, a, b[j]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < S::kTR; ++i)
+#pragma unroll
+        for (int j = 0; j < S::kTC; ++j)
+          acc[i][j] = mfma_tile<float>(lds, r0 + i * 16 + (lane & 15), lds_b, c0 + j * 16 + (lane & 15), acc[i][j], lane);
+    }
+  };
+  for (int kc = 0;;) {
+    __syncthreads();
+    const bool more = ++kc < nk;
+    if (more) {
+      la.fetch(kbeg + kc * kChunkK, ra);
+      lb.fetch(kbeg + kc * kChunkK, rb);
+    }
+    mma();
+    __syncthreads();
+    if (!more) break;
+    la.template commit<SPLIT>(ra, lds);
+    lb.template commit<SPLIT>(rb, lds_b);
+  }
+  if constexpr (kLow) {
+#pragma unroll
+    for (int i = 0; i < S::kTR; ++i)
+#pragma unroll
+      for (int j = 0; j < S::kTC; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i][j][r] += low[i][j][r];
+  }
 }
 
 // Runs the K loop; `acc` is accumulated (callers zero it).
@@ -457,6 +701,29 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
                                                             [TileShape<BR, BC, WR, WC>::kTC]) {
   static_assert(DEPTH == 1 || DEPTH == 2, "prefetch depth 1 or 2");
   using S = TileShape<BR, BC, WR, WC>;
+  if constexpr (sizeof(T) == 4) {
+    if (K <= 0) return;
+    const LA la0 = la;  // the loaders' row and column sums start again with a re-run
+    const LB lb0 = lb;
+    gemm_f32_loop<BR, BC, WR, WC, true>(la, lb, K, lds, acc);
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < S::kTR; ++i)
+#pragma unroll
+      for (int j = 0; j < S::kTC; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) finite = finite && fabsf(acc[i][j][r]) <= 3.402823466e38f;
+    if (__syncthreads_or(!finite)) {
+      la = la0;
+      lb = lb0;
+#pragma unroll
+      for (int i = 0; i < S::kTR; ++i)
+#pragma unroll
+        for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      gemm_f32_loop<BR, BC, WR, WC, false>(la, lb, K, lds, acc);
+    }
+    return;
+  } else {
   constexpr int P = LdsPitch<T>::value;
   constexpr int kBuf = (BR + BC) * P;  // elements of one (A, B) buffer pair
   const int lane = threadIdx.x & (kWave - 1);
@@ -497,11 +764,11 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
   }
   auto commit0 = [&]() {
     if (edge0) {
-      la.commit_edge(ra0, lds);
-      lb.commit_edge(rb0, lds + BR * P);
+      la.template commit_edge<false>(ra0, lds);
+      lb.template commit_edge<false>(rb0, lds + BR * P);
     } else {
-      la.commit(ra0, lds);
-      lb.commit(rb0, lds + BR * P);
+      la.template commit<false>(ra0, lds);
+      lb.template commit<false>(rb0, lds + BR * P);
     }
   };
   // The steady-state loops below fetch unconditionally: with every trip issuing the
@@ -517,8 +784,8 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
       la.fetch(kbeg + (kc + 1) * kChunkK, ra0);
       lb.fetch(kbeg + (kc + 1) * kChunkK, rb0);
       mma(cur);
-      la.commit(ra0, lds + kBuf - cur);
-      lb.commit(rb0, lds + kBuf - cur + BR * P);
+      la.template commit<false>(ra0, lds + kBuf - cur);
+      lb.template commit<false>(rb0, lds + kBuf - cur + BR * P);
       __syncthreads();
     }
     mma((kc & 1) * kBuf);
@@ -540,14 +807,14 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
       la.fetch(kbeg + (kc + 2) * kChunkK, ra0);
       lb.fetch(kbeg + (kc + 2) * kChunkK, rb0);
       mma(cur);
-      la.commit(ra1, lds + kBuf - cur);
-      lb.commit(rb1, lds + kBuf - cur + BR * P);
+      la.template commit<false>(ra1, lds + kBuf - cur);
+      lb.template commit<false>(rb1, lds + kBuf - cur + BR * P);
       __syncthreads();
       la.fetch(kbeg + (kc + 3) * kChunkK, ra1);
       lb.fetch(kbeg + (kc + 3) * kChunkK, rb1);
       mma(kBuf - cur);
-      la.commit(ra0, lds + cur);
-      lb.commit(rb0, lds + cur + BR * P);
+      la.template commit<false>(ra0, lds + cur);
+      lb.template commit<false>(rb0, lds + cur + BR * P);
       __syncthreads();
     }
     // 1 to 3 chunks left: kc (in LDS), kc + 1 (set 1, in flight), kc + 2 (not fetched)
@@ -556,24 +823,25 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
       la.fetch(kbeg + (kc + 2) * kChunkK, ra0);
       lb.fetch(kbeg + (kc + 2) * kChunkK, rb0);
       mma(cur);
-      la.commit(ra1, lds + kBuf - cur);
-      lb.commit(rb1, lds + kBuf - cur + BR * P);
+      la.template commit<false>(ra1, lds + kBuf - cur);
+      lb.template commit<false>(rb1, lds + kBuf - cur + BR * P);
       __syncthreads();
       mma(kBuf - cur);
-      la.commit(ra0, lds + cur);
-      lb.commit(rb0, lds + cur + BR * P);
+      la.template commit<false>(ra0, lds + cur);
+      lb.template commit<false>(rb0, lds + cur + BR * P);
       __syncthreads();
       mma(cur);
     } else if (kc + 1 < nk) {
       mma(cur);
-      la.commit(ra1, lds + kBuf - cur);
-      lb.commit(rb1, lds + kBuf - cur + BR * P);
+      la.template commit<false>(ra1, lds + kBuf - cur);
+      lb.template commit<false>(rb1, lds + kBuf - cur + BR * P);
       __syncthreads();
       mma(kBuf - cur);
     } else {
       mma(cur);
     }
     __syncthreads();
+  }
   }
 }
 

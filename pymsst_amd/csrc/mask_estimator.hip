@@ -83,7 +83,7 @@ struct LeftGateLoader : KRowLoader<T, 128, V4> {
 constexpr int kFwdBM = 128;
 
 template <typename T, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(PMSST_ME_FWD_WAVES))) void me_fwd_kernel(const T* __restrict__ x, const T* __restrict__ weight,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? PMSST_ME_FWD_WAVES : 2))) void me_fwd_kernel(const T* __restrict__ x, const T* __restrict__ weight,
                                                               const T* __restrict__ bias, T* __restrict__ pre,
                                                               T* __restrict__ out, int max_lchunks, XcdGrid xg,
                                                               MaskArgs a, BandSched sc) {
@@ -511,7 +511,7 @@ constexpr int kDxBM = 64;
 // TANH_IN: the layer input x is tanh(z) of the previous layer, and the kernel writes
 // dz = (dpre W_b) * (1 - x^2) instead of dx (the hidden activation's backward, fused).
 template <typename T, bool TANH_IN, bool V4>
-__global__ __launch_bounds__(kGemmThreads) void me_bwd_dx_kernel(const T* __restrict__ dpre,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void me_bwd_dx_kernel(const T* __restrict__ dpre,
                                                                  const T* __restrict__ weight,
                                                                  const T* __restrict__ x, T* __restrict__ dx,
                                                                  int hchunks, XcdGrid xg, MaskArgs a) {
@@ -537,9 +537,9 @@ __global__ __launch_bounds__(kGemmThreads) void me_bwd_dx_kernel(const T* __rest
   for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int hr = (wave >> 1) * (kDxBH / 2), mc = (wave & 1) * (kDxBM / 2);
   gemm_mainloop<T, kDxBH, kDxBM, 2, 2>(la, lb, 2 * I, lds, acc);
 
-  const int hr = (wave >> 1) * (kDxBH / 2), mc = (wave & 1) * (kDxBM / 2);
 #pragma unroll
   for (int i = 0; i < S::kTR; ++i) {
     const int h = h0 + hr + i * 16 + 4 * (lane >> 4);
@@ -762,7 +762,7 @@ constexpr int kDwBH = 128;
 constexpr int kDwBJ = 64;
 
 template <typename T, bool V4>
-__global__ __launch_bounds__(kGemmThreads) void me_bwd_dw_kernel(const T* __restrict__ dpre, const T* __restrict__ x,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void me_bwd_dw_kernel(const T* __restrict__ dpre, const T* __restrict__ x,
                                                                  T* __restrict__ dw, T* __restrict__ dbias,
                                                                  int htiles, XcdGrid xg, MaskArgs a, BandSched sc) {
   __shared__ T lds[gemm_lds_elems<T, kDwBH, kDwBJ>()];

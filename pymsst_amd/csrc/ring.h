@@ -1,22 +1,11 @@
-// Helpers of the register-accumulating DMA-ring kernels (grouped_dx.hip, mask_dz.hip): LDS
-// fragment reads the compiler waits for itself, an M0-preserving asm DMA, a runtime vmcnt wait.
+// Helpers of the register-accumulating DMA-ring kernels (grouped_dx.hip, mask_dz.hip): an
+// M0-preserving asm DMA, a runtime vmcnt wait.
 #pragma once
 
 #include "common.h"
 #include "dma_gemm.h"
 
 namespace pmsst {
-
-typedef short s16x4_t __attribute__((ext_vector_type(4)));
-
-// Transposed fragment (two ds_read_b64_tr_b16 through the compiler's builtin, which it waits for)
-__device__ __forceinline__ u32x4_t tr_frag(const char* p, int step) {
-  typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
-  const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-  const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + step));
-  const uint2 a = __builtin_bit_cast(uint2, lo), b = __builtin_bit_cast(uint2, hi);
-  return u32x4_t{a.x, a.y, b.x, b.y};
-}
 
 // One 16-byte-per-lane global -> LDS DMA (lane l writes LDS byte lds + 16 l; lds wave-uniform),
 // from inline asm that saves and restores M0 itself.  The compiler then sees no LDS write and no
