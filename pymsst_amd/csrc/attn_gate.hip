@@ -26,10 +26,15 @@
 // issue order).  The grids hold as many blocks as fit on the device at once, so a block's staging of
 // W is spread over as many tokens as possible.
 //
+// 16-bit, dim a multiple of 64 up to 512: the three products run on the matrix cores (gate_mfma_*_kernel
+// below), on the same 16-bit operands.
+//
 // Any other shape runs the generic kernels (one wave per token, one head at a time).
 #include <algorithm>
 
 #include "common.h"
+#include "dma_gemm.h"
+#include "ring.h"
 #include "rowgeom.h"
 
 namespace pmsst {
@@ -305,6 +310,243 @@ __global__ __launch_bounds__(kGateThreads) void gate_bwd_kernel(
   if (threadIdx.x < H) pb[static_cast<int64_t>(blockIdx.x) * H + threadIdx.x] = red[H * dim + threadIdx.x];
 }
 
+// ------------------------------------------------------------------ 16-bit, matrix cores
+//
+// The kernels above spend their time on the gate products, 2 to 4 x H x dim multiply-adds a token on the
+// vector units with x moved two bytes a lane (dim 512, 8 heads, 117,552 tokens: forward 138 us, 2.6 TB/s,
+// backward 263 us, 2.3 TB/s, where a copy of the bytes takes 74 and 123; the kernels below take 82 and
+// 119 us and the stream of rows bounds them).  H <= 16 heads fill one side of a 16 x 16 x 32 MFMA:
+//   logits   [16 heads x 16 tokens], K = dim:  A = W rows, B = x rows, 16 bytes a lane from memory
+//   grad_x^T [16 i x 16 tokens],     K = heads: A = W^T (registers), B = gpre
+//   grad_W^T [16 i x 16 heads],      K = tokens: A = x^T (LDS tile, transposed reads), B = gpre
+// and the rest is the stream of attn, out, grad_out, grad_attn, x and grad_x in 16-byte packs.
+
+// Forward: a wave takes 16 tokens; every load of theirs is issued before the first product.
+template <typename T, int E, int NT>  // E elements a lane of a token's H * Dh, dim = 64 NT
+__global__ __launch_bounds__(kGateThreads) void gate_mfma_fwd_kernel(const T* __restrict__ attn, GateRows ar,
+                                                                     const T* __restrict__ x,
+                                                                     const T* __restrict__ w,
+                                                                     const T* __restrict__ bias, T* __restrict__ out,
+                                                                     T* __restrict__ gate, int64_t rows, int logh) {
+  constexpr int DIM = 64 * NT, KS = DIM / 32;
+  __shared__ __attribute__((aligned(16))) char wl[KS * 1024];  // W as A fragments: lane l of K step s at 1024 s + 16 l
+  __shared__ float gl[kGateWaves][16][17];                     // a wave's gates [token][head]
+  const int H = 1 << logh;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, gq = lane >> 4, rr = lane & 15;
+  const int head = lane >> (6 - logh), sub = lane & ((64 >> logh) - 1);
+  for (int q = tid; q < KS * 64; q += kGateThreads) {
+    const int l = q & 63, h = l & 15;
+    const u32x4_t v = h < H ? *reinterpret_cast<const u32x4_t*>(w + h * DIM + 32 * (q >> 6) + 8 * (l >> 4))
+                            : u32x4_t{0u, 0u, 0u, 0u};
+    *reinterpret_cast<u32x4_t*>(wl + q * 16) = v;
+  }
+  float bv[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bv[r] = 4 * gq + r < H ? to_f32(bias[4 * gq + r]) : 0.f;
+  const int64_t m0 = (static_cast<int64_t>(blockIdx.x) * kGateWaves + wave) * 16;
+  u32x4_t xf[KS];
+  Pack<T, E> ap[16];
+  if (m0 < rows) {  // tokens past the end load the last one (their results are not stored)
+    const int64_t mx = m0 + rr < rows ? m0 + rr : rows - 1;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) xf[k] = *reinterpret_cast<const u32x4_t*>(x + mx * DIM + 32 * k + 8 * gq);
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      const int64_t m = m0 + t < rows ? m0 + t : rows - 1;
+      ap[t] = *reinterpret_cast<const Pack<T, E>*>(token_base(attn, ar, static_cast<uint32_t>(m)) + head * ar.sh + sub * E);
+    }
+  }
+  __syncthreads();
+  if (m0 >= rows) return;
+  f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int k = 0; k < KS; ++k)
+    acc[k & 1] = mfma_raw<T>(*reinterpret_cast<const u32x4_t*>(wl + k * 1024 + lane * 16), xf[k], acc[k & 1]);
+  // lane: heads 4 gq + r of token rr
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int h = 4 * gq + r;
+    const T gt = from_f32<T>(sigmoidf(acc[0][r] + acc[1][r] + bv[r]));
+    gl[wave][rr][h] = to_f32(gt);
+    if (h < H && m0 + rr < rows) gate[(m0 + rr) * H + h] = gt;
+  }
+  __builtin_amdgcn_wave_barrier();  // the wave's own LDS writes, read back below in order
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    if (m0 + t >= rows) break;
+    const float gf = gl[wave][t][head];
+    float o[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = to_f32(ap[t].v[e]) * gf;
+    store_pack<T, E>(out + (m0 + t) * (64 * E) + lane * E, o);
+  }
+}
+
+// Backward: a block walks 32-token groups blockIdx.x, + gridDim.x, ...  Per group each wave forms gpre of
+// 8 tokens from the packs loaded a group ahead and writes their grad_attn; after the block's one barrier
+// it moves the next group's x tile (DMA, two buffers) and packs, then takes dim / 4 columns of grad_x and
+// of the grad_W accumulators over all 32 tokens.
+template <typename T, int E, int NT>
+__global__ __launch_bounds__(kGateThreads) __attribute__((amdgpu_waves_per_eu(2))) void gate_mfma_bwd_kernel(
+    const T* __restrict__ grad_out, const T* __restrict__ attn, GateRows ar, const T* __restrict__ x,
+    const T* __restrict__ w, const T* __restrict__ gate, T* __restrict__ grad_attn, GateRows gr,
+    T* __restrict__ grad_x, float* __restrict__ pw, float* __restrict__ pb, int64_t rows, int logh) {
+  constexpr int DIM = 64 * NT, PITCH = 2 * DIM;
+  constexpr int kTok = 32, kWT = kTok / kGateWaves;  // tokens of a group, of a wave
+  constexpr int kTile = kTok * PITCH;
+  constexpr int kGxStores = 2 * (NT / 2 + NT % 2);   // grad_x stores of a wave and full group
+  __shared__ __attribute__((aligned(1024))) char xt[2 * kTile];  // x rows, units swizzled by swz_mn_p
+  __shared__ __attribute__((aligned(16))) T gt_tok[2][kTok][16];  // gpre by token, heads past H zero
+  __shared__ __attribute__((aligned(16))) T gt_head[2][16][kTok];
+  __shared__ float red[kGateWaves][16];
+  const int H = 1 << logh;
+  const int tid = threadIdx.x, lane = tid & 63, gq = lane >> 4, rr = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int head = lane >> (6 - logh), lph = 64 >> logh, sub = lane & (lph - 1);
+  const int i0 = 16 * NT * wave;  // this wave's columns
+  for (int q = tid; q < 2 * kTok * 16; q += kGateThreads) {
+    (&gt_tok[0][0][0])[q] = from_f32<T>(0.f);
+    (&gt_head[0][0][0])[q] = from_f32<T>(0.f);
+  }
+  // W^T fragments: K = heads 8 gq + e; tile t's row r is column 32 (t / 2) + 8 (r / 4) + 4 (t % 2) + r % 4
+  // of a pair of tiles, so that a lane's accumulators of the pair are 8 neighbours, or 16 t + r of a last
+  // single tile
+  auto col = [](int t, int r) { return t < NT / 2 * 2 ? 32 * (t / 2) + 8 * (r >> 2) + 4 * (t & 1) + (r & 3) : 16 * t + r; };
+  u32x4_t wf[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    Pack<T, 8> pk;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int h = 8 * gq + e;
+      pk.v[e] = h < H ? w[h * DIM + i0 + col(t, rr)] : from_f32<T>(0.f);
+    }
+    wf[t] = __builtin_bit_cast(u32x4_t, pk);
+  }
+  f32x4_t acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float accb = 0.f;
+
+  const int64_t groups = (rows + kTok - 1) / kTok;
+  // x tile: piece p = wave + 4 q of 4 NT moves flattened 16-byte units 64 p + lane (rows past the end: the
+  // last row, zeroed once it has landed)
+  auto dma = [&](int64_t grp, int buf) {
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      const int p = wave + kGateWaves * q;
+      const int U = 64 * p + lane;
+      const int kr = U / (DIM / 8), u = (U % (DIM / 8)) ^ swz_mn_p<PITCH>(kr);
+      const int64_t m = grp * kTok + kr < rows ? grp * kTok + kr : rows - 1;
+      dma16_m0(x + m * DIM + 8 * u, __builtin_amdgcn_readfirstlane(lds_addr(xt) + buf * kTile + p * 1024));
+    }
+  };
+  Pack<T, E> gp[kWT], ap[kWT];
+  T gtv[kWT];
+  auto load = [&](int64_t grp) {
+#pragma unroll
+    for (int t = 0; t < kWT; ++t) {
+      int64_t m = grp * kTok + wave * kWT + t;
+      m = m < rows ? m : rows - 1;
+      gp[t] = *reinterpret_cast<const Pack<T, E>*>(grad_out + m * (64 * E) + lane * E);
+      ap[t] = *reinterpret_cast<const Pack<T, E>*>(token_base(attn, ar, static_cast<uint32_t>(m)) + head * ar.sh + sub * E);
+      gtv[t] = gate[m * H + head];
+    }
+  };
+  int64_t grp = blockIdx.x;
+  if (grp < groups) {
+    dma(grp, 0);
+    load(grp);
+  }
+  __syncthreads();  // the zeroed gpre tiles
+  for (int it = 0; grp < groups; grp += gridDim.x, ++it) {
+    const int buf = it & 1;
+    // this group's x has landed: it was issued before the packs, of which all but the grad_x stores issued
+    // since (none before the first group) must be back
+    if (it == 0) vm_wait<0>();
+    else vm_wait<kGxStores>();
+    if ((grp + 1) * kTok > rows) {  // rows past the end
+#pragma unroll
+      for (int q = 0; q < NT; ++q) {
+        const int U = 64 * (wave + kGateWaves * q) + lane;
+        if (grp * kTok + U / (DIM / 8) >= rows)
+          *reinterpret_cast<u32x4_t*>(xt + buf * kTile + U * 16) = u32x4_t{0u, 0u, 0u, 0u};
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < kWT; ++t) {
+      const int tok = wave * kWT + t;
+      const int64_t m = grp * kTok + tok;
+      const float gf = to_f32(gtv[t]);
+      float s = 0.f, o[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const float g = to_f32(gp[t].v[e]);
+        s += g * to_f32(ap[t].v[e]);
+        o[e] = g * gf;
+      }
+      for (int d = lph >> 1; d > 0; d >>= 1) s += __shfl_xor(s, d, kWave);
+      T gpre = from_f32<T>(s * gf * (1.0f - gf));
+      if (m < rows) {
+        store_pack<T, E>(token_base(grad_attn, gr, static_cast<uint32_t>(m)) + head * gr.sh + sub * E, o);
+        accb += to_f32(gpre);
+      } else {
+        gpre = from_f32<T>(0.f);
+      }
+      if (sub == 0) {
+        gt_tok[buf][tok][head] = gpre;
+        gt_head[buf][head][tok] = gpre;
+      }
+    }
+    __syncthreads();
+    const int64_t next = grp + gridDim.x;
+    if (next < groups) {
+      dma(next, buf ^ 1);  // its buffer's readers passed the barrier above
+      load(next);
+    }
+    // grad_x of 2 x 16 tokens
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      u32x4_t bf{0u, 0u, 0u, 0u};
+      if (gq < 2) bf = *reinterpret_cast<const u32x4_t*>(&gt_tok[buf][16 * n + rr][8 * gq]);
+      const int64_t m = grp * kTok + 16 * n + rr;
+      f32x4_t d[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) d[t] = mfma_raw<T>(wf[t], bf, f32x4_t{0.f, 0.f, 0.f, 0.f});
+      if (m < rows) {
+        T* dst = grad_x + m * DIM + i0;
+#pragma unroll
+        for (int t = 0; t + 1 < NT; t += 2) {
+          const float v[8] = {d[t][0], d[t][1], d[t][2], d[t][3], d[t + 1][0], d[t + 1][1], d[t + 1][2], d[t + 1][3]};
+          store_pack<T, 8>(dst + 16 * t + 8 * gq, v);
+        }
+        if constexpr (NT % 2 == 1) {
+          const float v[4] = {d[NT - 1][0], d[NT - 1][1], d[NT - 1][2], d[NT - 1][3]};
+          store_pack<T, 4>(dst + 16 * (NT - 1) + 4 * gq, v);
+        }
+      }
+    }
+    // grad_W over the 32 tokens
+    const u32x4_t hf = *reinterpret_cast<const u32x4_t*>(&gt_head[buf][rr][8 * gq]);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      acc[t] = mfma_raw<T>(tr_frag(xt + buf * kTile + frag_mn_addr_p<PITCH>(0, i0 + 16 * t, lane), 4 * PITCH), hf, acc[t]);
+  }
+  vm_wait<0>();  // no DMA may still be writing this block's LDS when its waves end
+
+  // partials: lane holds columns i0 + 16 t + 4 gq + r of head rr; grad_b over the waves in order
+  if (rr < H) {
+    float* dst = pw + static_cast<int64_t>(blockIdx.x) * H * DIM + rr * DIM + i0 + 4 * gq;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      *reinterpret_cast<float4*>(dst + 16 * t) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+  }
+  if (sub == 0) red[wave][head] = accb;
+  __syncthreads();
+  if (tid < H)
+    pb[static_cast<int64_t>(blockIdx.x) * H + tid] = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
+}
+
 // ------------------------------------------------------------------ generic kernels (any shape)
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -510,6 +752,33 @@ inline GateRows gate_rows(const int64_t* st, const GateShape& s) {
   return g;
 }
 
+// Whether the matrix-core kernels take a shape the fast path takes: 16-bit, dim = 64 NT with NT built
+// below, 16-byte aligned rows of x, W and grad_x.
+inline bool gate_mfma_ok(const GateShape& s, size_t esz, const void* x, const void* w, const void* gx) {
+  const bool al = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(gx) % 16 == 0;
+  const int64_t nt = s.dim / 64;
+  return esz == 2 && al && s.dim % 64 == 0 && (nt <= 4 || nt == 6 || nt == 8) && s.rows() < (int64_t{1} << 30);
+}
+
+// f(E, NT) as integral constants.
+template <class F>
+void gate_mfma_dispatch(int e, int64_t dim, F&& f) {
+  auto with_e = [&](auto nt) {
+    if (e == 2) f(std::integral_constant<int, 2>{}, nt);
+    else if (e == 4) f(std::integral_constant<int, 4>{}, nt);
+    else f(std::integral_constant<int, 8>{}, nt);
+  };
+  switch (dim / 64) {
+    case 1: with_e(std::integral_constant<int, 1>{}); break;
+    case 2: with_e(std::integral_constant<int, 2>{}); break;
+    case 3: with_e(std::integral_constant<int, 3>{}); break;
+    case 4: with_e(std::integral_constant<int, 4>{}); break;
+    case 6: with_e(std::integral_constant<int, 6>{}); break;
+    default: with_e(std::integral_constant<int, 8>{}); break;
+  }
+}
+
 template <typename T>
 int launch_gate_fwd(const void* attn, const int64_t* attn_strides, const void* x, const void* weight,
                     const void* bias, void* out, void* gate, const GateShape& s, hipStream_t stream) {
@@ -537,6 +806,16 @@ int launch_gate_fwd(const void* attn, const int64_t* attn_strides, const void* x
                        stream, pa, ar, px, pw, pb, po, pg, rows, static_cast<int>(s.heads), static_cast<int>(s.dh),
                        dim);
     return check_launch("gate_fwd_generic_kernel");
+  }
+  if constexpr (sizeof(T) == 2) {
+    if (gate_mfma_ok(s, sizeof(T), x, weight, nullptr)) {
+      const dim3 grid(static_cast<unsigned>((rows + 16 * kGateWaves - 1) / (16 * kGateWaves)));
+      gate_mfma_dispatch(e, s.dim, [&](auto ec, auto nt) {
+        hipLaunchKernelGGL((gate_mfma_fwd_kernel<T, decltype(ec)::value, decltype(nt)::value>), grid,
+                           dim3(kGateThreads), 0, stream, pa, ar, px, pw, pb, po, pg, rows, gate_log2(s.heads));
+      });
+      return check_launch("gate_mfma_fwd_kernel");
+    }
   }
   const int blocks = gate_blocks(rows, kGateRows, kGateMaxBlocks);
   const int jx = gate_jx(s.dim);
@@ -633,6 +912,21 @@ int launch_gate_bwd(const void* grad_out, const void* attn, const int64_t* attn_
                          stream, gpre, px, pw, pbias, rows, heads, dim, static_cast<int>(gate_dw_chunk_rows(rows)));
       rc = check_launch("gate_dw_generic_kernel");
       if (rc != PMSST_OK) return rc;
+    } else if (gate_mfma_ok(s, sizeof(T), x, weight, grad_x)) {
+      if constexpr (sizeof(T) == 2) {
+        // the groups of 32 tokens in equal turns of at most two blocks per CU
+        const int64_t groups = (rows + 31) / 32;
+        const int64_t slots = std::min<int64_t>(2 * static_cast<int64_t>(num_cus()), kGateBwdMaxBlocks);
+        const int64_t turns = (groups + slots - 1) / slots;
+        nparts = static_cast<int>((groups + turns - 1) / turns);
+        gate_mfma_dispatch(e, s.dim, [&](auto ec, auto nt) {
+          hipLaunchKernelGGL((gate_mfma_bwd_kernel<T, decltype(ec)::value, decltype(nt)::value>), dim3(nparts),
+                             dim3(kGateThreads), 0, stream, pgo, pa, ar, px, pw_, pg, pga, gr, pgx, pw, pbias, rows,
+                             gate_log2(s.heads));
+        });
+        rc = check_launch("gate_mfma_bwd_kernel");
+        if (rc != PMSST_OK) return rc;
+      }
     } else {
       nparts = gate_blocks(rows, kGateRows, kGateBwdMaxBlocks);
       const int jx = gate_jx(s.dim);
