@@ -635,6 +635,12 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
 // are read from its first row and zeroed.  dbias: the two top waves of input tile 0 also
 // multiply their dy fragments by an all-ones A fragment (every row of that product is the
 // column sum).  The tile leaves through LDS as rows o of dW_b.
+//
+// The fp32-input band split takes it too (gamma null: the features hold it already; dgamma in fp32).
+// What bounds it there is the serial walk over the rows, 64 of them a step with two steps in flight: 60
+// mel bands at 2760 rows, O = 192: 54.6 us with dgamma, where bs_bwd_dw_kernel (32 rows a step, one in
+// flight) and a dgamma launch took 82; 62 bands at 1032 rows 15.5 against 27.6.  32-row steps with four
+// in flight measure 56.9 and 18.8.
 constexpr int kBdT = 64;
 // 1024 rows (4 KB) keep the kernel at 52 KB of LDS, three blocks per CU, so the dx finish and
 // dgamma tail blocks run beside the dW blocks' row loops (2048 rows: 56 KB, two per CU)
@@ -672,11 +678,11 @@ __device__ __forceinline__ void vm_wait_steps(int nd) {  // at most N nd DMAs ou
   }
 }
 
-template <typename T, bool FROM_X>
+template <typename T, typename TG, bool FROM_X>
 __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_dma_kernel(
     const T* __restrict__ dy, const T* __restrict__ nsrc, const float* __restrict__ inv_norm,
     const T* __restrict__ gamma, T* __restrict__ dw, T* __restrict__ db, BandSched sc, BandArgs a, int otiles,
-    const float* __restrict__ dg_partial, int dg_parts, T* __restrict__ dgamma, uint32_t main_blocks,
+    const float* __restrict__ dg_partial, int dg_parts, TG* __restrict__ dgamma, uint32_t main_blocks,
     const float* __restrict__ tbuf, const float* __restrict__ pdot, T* __restrict__ dx, int pitch, BandSched fsc,
     uint32_t fin_blocks) {
   constexpr int S = PMSST_BS_DWD_STAGES;
@@ -698,7 +704,7 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_dma_kernel(
   // of kXcds, so each keeps its XCD), then dgamma = the column sums of the dx kernel's partials in
   // col_sum_kernel's order.  Neither gets a launch of its own.
   if (blockIdx.x >= main_blocks + fin_blocks) {
-    col_sum_tile<T, kGemmThreads>(dg_partial, dg_parts, a.F, dgamma,
+    col_sum_tile<TG, kGemmThreads>(dg_partial, dg_parts, a.F, dgamma,
                                   static_cast<int>(blockIdx.x - main_blocks - fin_blocks),
                                   reinterpret_cast<float*>(lds));
     return;
@@ -875,7 +881,7 @@ __global__ __launch_bounds__(kGemmThreads) void bs_bwd_dw_dma_kernel(
     const int i = i0 + 32 * wr + 16 * f + 4 * (lane >> 4);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {  // clamped loads outside any branch: issued together
-      const float gv = to_f32(gamma[off + (i + r < I ? i + r : I - 1)]);
+      const float gv = gamma != nullptr ? to_f32(gamma[off + (i + r < I ? i + r : I - 1)]) : 1.f;
       gsc[f][r] = i + r < I ? gv * sb : 0.f;
     }
   }
@@ -1242,6 +1248,19 @@ size_t bwd_workspace(int64_t M, int F, int NB) {
   return M == 0 ? 0 : dg_partial_bytes(M, F) + pdot_bytes(M, F, NB) + tbuf_bytes(M, F);
 }
 
+// Whether bs_bwd_dw_dma_kernel takes a dW, and its schedule: 16-bit, 4-aligned widths and pointers,
+// O % 8 == 0 with 16-byte aligned dy rows, at least one step of rows.
+template <typename T>
+bool dma_dw_sched(const BandArgs& a, const HostBands& hb, int64_t M, int64_t O, const void* dy, BandSched* sc,
+                  uint32_t* per_xcd) {
+  constexpr int KR = PMSST_BS_DWD_KS * kChunkK;
+  const int otiles = static_cast<int>((O + kBdT - 1) / kBdT);
+  return sizeof(T) == 2 && PMSST_BS_DW_DMA && M >= KR && a.vec4 && O % 8 == 0 && aligned_to(dy, 16) &&
+         (static_cast<int64_t>(KR) * hb.F + hb.F) * 2 < (int64_t{1} << 31) &&
+         (static_cast<int64_t>(KR) * hb.NB * O + O) * 2 < (int64_t{1} << 31) &&
+         build_band_sched(hb.NB, 1, [&](int b) { return (hb.widths[b] + kBdT - 1) / kBdT * otiles; }, sc, per_xcd);
+}
+
 template <typename T>
 int launch_bwd(const void* dy, const void* nsrc, bool from_x, const float* inv_norm, const void* gamma,
                const void* weight, const int64_t* offsets, const int64_t* dim_inputs, const HostBands& hb,
@@ -1273,15 +1292,10 @@ int launch_bwd(const void* dy, const void* nsrc, bool from_x, const float* inv_n
   const int pitch = pdot_pitch(hb.F, hb.NB);
   const int m_tiles = static_cast<int>((M + kBM - 1) / kBM);
   // DMA-ring dW: 16-bit, 4-aligned widths and pointers, O % 8 == 0 with 16-byte aligned dy rows
-  constexpr int KR = PMSST_BS_DWD_KS * kChunkK;
   const int otiles = static_cast<int>((O + kBdT - 1) / kBdT);
   BandSched wsc;
   uint32_t w_per_xcd = 0;
-  const bool dma_dw = sizeof(T) == 2 && PMSST_BS_DW_DMA && M >= KR && a.vec4 && O % 8 == 0 && aligned_to(dy, 16) &&
-                      (static_cast<int64_t>(KR) * hb.F + hb.F) * 2 < (int64_t{1} << 31) &&
-                      (static_cast<int64_t>(KR) * hb.NB * O + O) * 2 < (int64_t{1} << 31) &&
-                      build_band_sched(hb.NB, 1, [&](int b) { return (dim_inputs[b] + kBdT - 1) / kBdT * otiles; },
-                                       &wsc, &w_per_xcd);
+  const bool dma_dw = dma_dw_sched<T>(a, hb, M, O, dy, &wsc, &w_per_xcd);
   BandSched sc;  // dx and finish: one block per existing (band, row tile, chunk); sc.m_tiles = 0 without
   uint32_t per_xcd = 0;
   const bool dx_sched =
@@ -1330,11 +1344,11 @@ int launch_bwd(const void* dy, const void* nsrc, bool from_x, const float* inv_n
       T* pdg = static_cast<T*>(dgamma);
       T* pdx = static_cast<T*>(dx);
       if (from_x)
-        hipLaunchKernelGGL((bs_bwd_dw_dma_kernel<T, true>), grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm,
+        hipLaunchKernelGGL((bs_bwd_dw_dma_kernel<T, T, true>), grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm,
                            pg, static_cast<T*>(dw), static_cast<T*>(db), wsc, a, otiles, partial, m_tiles, pdg,
                            main_blocks, tbuf, pdot, pdx, pitch, fsc, fin_blocks);
       else
-        hipLaunchKernelGGL((bs_bwd_dw_dma_kernel<T, false>), grid, dim3(kGemmThreads), 0, stream, pdy, pn,
+        hipLaunchKernelGGL((bs_bwd_dw_dma_kernel<T, T, false>), grid, dim3(kGemmThreads), 0, stream, pdy, pn,
                            inv_norm, pg, static_cast<T*>(dw), static_cast<T*>(db), wsc, a, otiles, partial, m_tiles,
                            pdg, main_blocks, tbuf, pdot, pdx, pitch, fsc, fin_blocks);
       const int rc = check_launch("bs_bwd_dw_dma_kernel");
@@ -1575,8 +1589,23 @@ int launch_mixed_bwd(const void* dy, const float* x, int64_t x_stride, const voi
                               stream);
     if (rc != PMSST_OK) return rc;
   }
-  // dW_b = T(dy_b^T u_b), dbias = T(sum_m dy_b): the norm-free register-staged dW kernel (it also
-  // runs for M == 0 and then writes zeros)
+  const int parts = static_cast<int>((M + kColRows - 1) / kColRows);
+  // dW_b = T(dy_b^T u_b), dbias = T(sum_m dy_b), and in tail blocks dgamma = the column sums of the
+  // partials
+  BandSched dsc;
+  uint32_t d_per_xcd = 0;
+  if (dma_dw_sched<T>(a, hb, M, O, dy, &dsc, &d_per_xcd)) {
+    if constexpr (sizeof(T) == 2) {
+      const uint32_t main_blocks = d_per_xcd * kXcds;
+      const dim3 grid(main_blocks + static_cast<uint32_t>((hb.F + kColSumCols - 1) / kColSumCols));
+      hipLaunchKernelGGL((bs_bwd_dw_dma_kernel<T, float, false>), grid, dim3(kGemmThreads), 0, stream, pdy, pu, nullptr,
+                         nullptr, static_cast<T*>(dw), static_cast<T*>(db), dsc, a,
+                         static_cast<int>((O + kBdT - 1) / kBdT), partial, parts, dgamma, main_blocks, nullptr, nullptr,
+                         nullptr, 0, dsc, 0u);
+      return check_launch("bs_bwd_dw_dma_kernel");
+    }
+  }
+  // other shapes: the norm-free register-staged dW kernel (it also runs for M == 0 and then writes zeros)
   {
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
     constexpr int kCols = dw_cols<T, false>();
@@ -1593,7 +1622,6 @@ int launch_mixed_bwd(const void* dy, const float* x, int64_t x_stride, const voi
     if (rc != PMSST_OK) return rc;
   }
   // dgamma = the column sums of the partials (parts == 0 writes zeros)
-  const int parts = static_cast<int>((M + kColRows - 1) / kColRows);
   return launch_col_sum(partial, parts, hb.F, dgamma, PMSST_F32, stream);
 }
 

@@ -516,7 +516,7 @@ def replay_band_split_backward(widths, M, O, esz, *, has_bias=True, grouped=Fals
                                     bnd.touch("x", (e + q) * esz, esz, okq)
                                     bnd.touch("dx", (e + q) * esz, esz, okq)
     # -- dW
-    dma = (not grouped) and esz == 2 and M >= 64 and vec4 and O % 8 == 0
+    dma = (not grouped or even_dx) and esz == 2 and M >= 64 and vec4 and O % 8 == 0
     uniform_dw = grouped and esz == 2 and M >= CHUNK_K and len(set(widths)) == 1 and widths[0] % 64 == 0 \
         and O % 8 == 0
     if dma:
@@ -666,8 +666,8 @@ def replay_band_split_mixed(widths, M, O, *, x_stride=None):
     _replay_band_colpass(bwd, widths, offs, M, x_stride, 1)
     _replay_col_sum(bwd, "partial", cdiv(M, 16), F, "dgamma", 4)
     yield "band_split_mixed_bwd_norm", bwd
-    # g = T(dy W) on the norm-free dx kernel and dW / dbias on the norm-free register dW kernel: the
-    # grouped-linear replay of those two kernels (dx = g here, x = the features)
+    # g = T(dy W) on the norm-free dx kernel (dx = g here, x = the features) and dW / dbias on the DMA dW
+    # kernel, or where that does not fit on the norm-free register dW kernel
     yield "band_split_mixed_bwd_gemm", replay_band_split_backward(widths, M, O, 2, grouped=True, even_dx=True)
 
 

@@ -86,6 +86,14 @@ def test_mixed_odd_widths_and_pitch(hip_ext, dtype):
     _case(hip_ext, (8, 64, 132, 4), 300, 64, dtype, 34, pitch_extra=12)
 
 
+@pytest.mark.parametrize("m", [63, 64, 65, 191, 1100])
+def test_mixed_dw_row_steps(hip_ext, m):
+    # dW walks 64-row steps of the features (from 64 rows; a partial first step) over 64 x 64 tiles:
+    # one narrow band, a tile's remainders on both sides, and O short of a tile
+    _case(hip_ext, (4, 60, 68, 132), m, 72, torch.bfloat16, 100 + m)
+    _case(hip_ext, (8, 124), m, 8, torch.float16, 200 + m)
+
+
 def test_mixed_empty_batch(hip_ext):
     dims = (8, 16)
     x = torch.empty(0, 24, device="cuda")
