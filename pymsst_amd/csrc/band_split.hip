@@ -322,7 +322,7 @@ __device__ __forceinline__ bool bs_dx_block(const BandSched& sc, const XcdGrid& 
 template <typename T, bool NORM>
 constexpr int bs_dx_rows() { return sizeof(T) == 4 && !NORM ? 128 : 64; }
 
-template <typename T, bool FROM_X, bool NORM, bool V4>
+template <typename T, bool FROM_X, bool NORM, bool V4, int BM = bs_dx_rows<T, NORM>()>
 __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void bs_bwd_dx_kernel(const T* __restrict__ dy,
                                                                  const T* __restrict__ nsrc,
                                                                  const float* __restrict__ inv_norm,
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
                                                                  int max_ichunks, XcdGrid xg, BandSched sc,
                                                                  BandArgs a) {
   constexpr int kBI = 64;
-  constexpr int BM = bs_dx_rows<T, NORM>();
+  static_assert(BM == 64 || (BM == 128 && !NORM), "tile rows");
   __shared__ T lds[gemm_lds_elems<T, kBI, BM>()];
   __shared__ float sinv[BM];
   __shared__ float sdot[4][BM];
@@ -1562,22 +1562,33 @@ int launch_mixed_bwd(const void* dy, const float* x, int64_t x_stride, const voi
   float* dot = reinterpret_cast<float*>(ws + mixed_g_bytes(M, hb.F));
   float* partial = reinterpret_cast<float*>(ws + mixed_g_bytes(M, hb.F) + mixed_dot_bytes(M, hb.NB));
   if (M > 0) {
-    // g = T(dy W_b): the norm-free dx kernel, one block per existing (band, row tile, 64-wide chunk)
-    const int m_tiles = static_cast<int>((M + bs_dx_rows<T, false>() - 1) / bs_dx_rows<T, false>());
+    // g = T(dy W_b): the norm-free dx kernel, one block per existing (band, row tile, 64-wide chunk).
+    // Its blocks are short (K = O) and read as much weight as dy, so 128-row tiles, which halve the
+    // weight's share, where the grid keeps them: from two rounds of 64-row blocks at the 7 a CU holds
+    // (60 mel bands, 2760 rows, O = 192: 55.1 -> 49.1 us; 62 bands, 1032 rows, 0.9 of a round: 15.3
+    // and 15.4).
+    int64_t chunks = 0;
+    for (int b = 0; b < hb.NB; ++b) chunks += (hb.widths[b] + 63) / 64;
     const int max_ichunks = (hb.max_width + 63) / 64;
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>(m_tiles)};
-    BandSched sc;
-    uint32_t per_xcd = 0;
-    const bool sched =
-        build_even_sched(hb.NB, m_tiles, [&](int b) { return (hb.widths[b] + 63) / 64; }, &sc, &per_xcd);
-    const dim3 grid(sched ? per_xcd * kXcds : xg.blocks());
     const bool gv4 = a.vec4 && a.ovec4;
-    if (gv4)
-      hipLaunchKernelGGL((bs_bwd_dx_kernel<T, false, false, true>), grid, dim3(kGemmThreads), 0, stream, pdy, pu,
-                         nullptr, nullptr, pw, g, nullptr, nullptr, nullptr, 0, max_ichunks, xg, sc, a);
-    else
-      hipLaunchKernelGGL((bs_bwd_dx_kernel<T, false, false, false>), grid, dim3(kGemmThreads), 0, stream, pdy, pu,
-                         nullptr, nullptr, pw, g, nullptr, nullptr, nullptr, 0, max_ichunks, xg, sc, a);
+    auto launch_g = [&](auto bm) {
+      constexpr int kRows = decltype(bm)::value;
+      const int m_tiles = static_cast<int>((M + kRows - 1) / kRows);
+      const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>(m_tiles)};
+      BandSched sc;
+      uint32_t per_xcd = 0;
+      const bool sched =
+          build_even_sched(hb.NB, m_tiles, [&](int b) { return (hb.widths[b] + 63) / 64; }, &sc, &per_xcd);
+      const dim3 grid(sched ? per_xcd * kXcds : xg.blocks());
+      if (gv4)
+        hipLaunchKernelGGL((bs_bwd_dx_kernel<T, false, false, true, kRows>), grid, dim3(kGemmThreads), 0, stream, pdy,
+                           pu, nullptr, nullptr, pw, g, nullptr, nullptr, nullptr, 0, max_ichunks, xg, sc, a);
+      else
+        hipLaunchKernelGGL((bs_bwd_dx_kernel<T, false, false, false, kRows>), grid, dim3(kGemmThreads), 0, stream, pdy,
+                           pu, nullptr, nullptr, pw, g, nullptr, nullptr, nullptr, 0, max_ichunks, xg, sc, a);
+    };
+    if ((M + 63) / 64 * chunks >= int64_t{2} * 7 * num_cus()) launch_g(std::integral_constant<int, 128>{});
+    else launch_g(std::integral_constant<int, 64>{});
     int rc = check_launch("bs_bwd_dx_kernel");
     if (rc != PMSST_OK) return rc;
     // fp32 RMSNorm backward: dot = sum g gamma x per (row, band), then dx and the dgamma partials
