@@ -146,8 +146,18 @@ struct XGammaLoader {
   __device__ __forceinline__ void commit(const Regs& g, T* lds) const { commit_impl<SPLIT>(g, lds, !V4); }
 };
 
+// Waves per SIMD of a forward kernel's registers.  The blocks are short (K = I_b, a few 32-wide chunks) and
+// wait on their loads, so it is the blocks of a CU that hide them.  The 192-output tile of the projection
+// under autocast fits 168 registers without spills when asked to, three blocks per CU instead of two: 60
+// mel bands at 2760 rows 53.4 -> 44.5 us, 62 bands at 1032 rows 17.8 -> 15.6.  (One chunk in flight instead
+// of two: 42.2 and 19.1.  Four blocks with two in flight, or three at 256 outputs, spill: 92 and 30.4 us.)
+template <typename T, int TO, bool NORM, int ACT, bool V4>
+constexpr int bs_fwd_waves() {
+  return sizeof(T) == 4 ? 2 : !NORM && ACT == PMSST_ACT_NONE && TO == 3 && V4 ? 3 : 1;
+}
+
 template <typename T, int TO, bool WRITE_NORMED, bool NORM, int ACT, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1))) void bs_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(bs_fwd_waves<T, TO, NORM, ACT, V4>()))) void bs_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                               const T* __restrict__ weight,
                                                               const T* __restrict__ bias, T* __restrict__ out,
                                                               T* __restrict__ normed, float* __restrict__ inv_norm,
@@ -178,19 +188,25 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   gemm_mainloop<T, OT, kBM, 4, 1, PMSST_BS_FWD_DEPTH>(la, lb, I, lds, acc);
 
-  const float root = sqrtf(static_cast<float>(I));
-  const float ss0 = group_sum(lb.ss[0], 8);
-  const float ss1 = group_sum(lb.ss[1], 8);
-  if ((tid & 7) == 0) {
+  if constexpr (NORM) {
+    const float root = sqrtf(static_cast<float>(I));
+    const float ss0 = group_sum(lb.ss[0], 8);
+    const float ss1 = group_sum(lb.ss[1], 8);
+    if ((tid & 7) == 0) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int r = (tid >> 3) + 32 * p;
-      const float inv = 1.0f / fmaxf(sqrtf(p == 0 ? ss0 : ss1), 1.0e-12f);
-      sscale[r] = NORM ? inv * root : 1.0f;
-      if (NORM && blockIdx.z == 0 && r < rows_valid) inv_norm[(m0 + r) * a.NB + band] = inv;
+      for (int p = 0; p < 2; ++p) {
+        const int r = (tid >> 3) + 32 * p;
+        const float inv = 1.0f / fmaxf(sqrtf(p == 0 ? ss0 : ss1), 1.0e-12f);
+        sscale[r] = inv * root;
+        if (blockIdx.z == 0 && r < rows_valid) inv_norm[(m0 + r) * a.NB + band] = inv;
+      }
     }
+    __syncthreads();
   }
-  __syncthreads();
+  auto row_scale = [&](int m) {
+    if constexpr (NORM) return sscale[m];
+    else return 1.0f;
+  };
 
   if (a.ovec8) {
     // epilogue through LDS: lane holds 4 consecutive outputs of one row (8-byte runs of 16 rows
@@ -208,7 +224,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
 #pragma unroll
       for (int j = 0; j < S::kTC; ++j) {
         const int m = j * 16 + (lane & 15);
-        const float s = sscale[m];
+        const float s = row_scale(m);
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
       for (int j = 0; j < S::kTC; ++j) {
         const int m = j * 16 + (lane & 15);
         if (m >= rows_valid) continue;
-        const float s = sscale[m];
+        const float s = row_scale(m);
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -270,7 +286,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
       const int r = q / nq;
       const int k = (q - r * nq) * 4;
       if (r >= rows_valid) continue;
-      const float s = sscale[r];
+      const float s = row_scale(r);
       T* dst = normed + (m0 + r) * a.F + off + k;
       const T* srcp = xb + r * a.x_stride + k;
       if (a.vec4) {
