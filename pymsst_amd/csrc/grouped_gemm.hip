@@ -388,10 +388,18 @@ int launch_wide_dx(const void* dy, const void* w, void* dx, int64_t groups, int6
 
 bool wide_dw_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
                        const void* dy, const void* x, const void* dw) {
-  // from 192 inputs on (192 -> 768, 60 groups, 2760 rows: 90 us against me_bwd_dw_dma_kernel's 98; 62
-  // groups, 1032 rows: 36 against 37); narrower layers leave columns of the tile empty
-  return shape_ok(groups, in_features, out_features, rows, elem) && in_features >= 192 && rows >= 32 && aligned16(dy) &&
-         aligned16(x) && aligned16(dw);
+  if (!shape_ok(groups, in_features, out_features, rows, elem) || in_features < 192 || rows < 32 || !aligned16(dy) ||
+      !aligned16(x) || !aligned16(dw))
+    return false;  // below 192 inputs columns of the tile stay empty
+  if (in_features > 256 || in_features % 64 != 0) return true;
+  // At 192 and 256 inputs me_bwd_dw_dma_kernel's smaller blocks win while the loop over the rows is short
+  // or the 256-row tiles leave CUs idle: 192 -> 768, 62 groups (186 blocks): 64 rows 8.8 us against 10.0,
+  // 320 rows 15.4 against 16.4, 600 rows 24.2 each, 1032 rows 37 against 36; 60 groups, 2760 rows 98
+  // against 90; 192 -> 384 (124 blocks): 162 rows 8.9 against 11.6, 600 rows 16.4 against 21.4.
+  const int64_t a_cols = in_features % 256 == 0 ? 256 : 192;
+  const int64_t blocks = groups * ((out_features + 255) / 256) * ((in_features + a_cols - 1) / a_cols);
+  const int64_t cus = num_cus(), rounds = (blocks + cus - 1) / cus;
+  return rows >= 1024 && 3 * blocks >= 2 * rounds * cus;
 }
 
 template <typename T>
