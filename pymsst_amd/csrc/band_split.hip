@@ -151,19 +151,19 @@ struct XGammaLoader {
 // under autocast fits 168 registers without spills when asked to, three blocks per CU instead of two: 60
 // mel bands at 2760 rows 53.4 -> 44.5 us, 62 bands at 1032 rows 17.8 -> 15.6.  (One chunk in flight instead
 // of two: 42.2 and 19.1.  Four blocks with two in flight, or three at 256 outputs, spill: 92 and 30.4 us.)
-template <typename T, int TO, bool NORM, int ACT, bool V4>
+template <typename T, int TO, bool NORM, int ACT, bool V4, bool SPLIT>
 constexpr int bs_fwd_waves() {
-  return sizeof(T) == 4 ? 2 : !NORM && ACT == PMSST_ACT_NONE && TO == 3 && V4 ? 3 : 1;
+  return SPLIT ? 2 : sizeof(T) == 2 && !NORM && ACT == PMSST_ACT_NONE && TO == 3 && V4 ? 3 : 1;
 }
 
-template <typename T, int TO, bool WRITE_NORMED, bool NORM, int ACT, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(bs_fwd_waves<T, TO, NORM, ACT, V4>()))) void bs_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
+template <typename T, int TO, bool WRITE_NORMED, bool NORM, int ACT, bool V4, bool SPLIT>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(bs_fwd_waves<T, TO, NORM, ACT, V4, SPLIT>()))) void bs_fwd_kernel(const T* __restrict__ x, const T* __restrict__ gamma,
                                                               const T* __restrict__ weight,
                                                               const T* __restrict__ bias, T* __restrict__ out,
                                                               T* __restrict__ normed, float* __restrict__ inv_norm,
                                                               BandArgs a) {
   constexpr int OT = 64 * TO;
-  __shared__ T lds[gemm_lds_elems<T, OT, kBM>()];
+  __shared__ T lds[gemm_lds_elems<T, OT, kBM, SPLIT>()];
   __shared__ float sscale[kBM];
   using S = TileShape<OT, kBM, 4, 1>;  // TR = TO, TC = 4
 
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(bs
   for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gemm_mainloop<T, OT, kBM, 4, 1, PMSST_BS_FWD_DEPTH>(la, lb, I, lds, acc);
+  gemm_mainloop<T, OT, kBM, 4, 1, PMSST_BS_FWD_DEPTH, SPLIT>(la, lb, I, lds, acc);
 
   if constexpr (NORM) {
     const float root = sqrtf(static_cast<float>(I));
@@ -332,14 +332,11 @@ __device__ __forceinline__ bool bs_dx_block(const BandSched& sc, const XcdGrid& 
   return true;
 }
 
-// Rows of a block's tile: 64, or 128 for fp32 without the norm (the grouped linear: the weight chunk is
-// read half as often and a wave's fragments serve twice the products; 190 -> 160 us for 62 groups of
-// 192 -> 768 at 1032 rows).  With the norm the partials have 64 rows.
-template <typename T, bool NORM>
-constexpr int bs_dx_rows() { return sizeof(T) == 4 && !NORM ? 128 : 64; }
-
-template <typename T, bool FROM_X, bool NORM, bool V4, int BM = bs_dx_rows<T, NORM>()>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void bs_bwd_dx_kernel(const T* __restrict__ dy,
+// SPLIT takes 128 rows a tile without the norm (the grouped linear: the weight chunk is read half as often
+// and a wave's fragments serve twice the products; 190 -> 160 us for 62 groups of 192 -> 768 at 1032
+// rows).  With the norm the partials have 64 rows.
+template <typename T, bool FROM_X, bool NORM, bool V4, int BM = 64, bool SPLIT = false>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(SPLIT ? kSplitWaves : 1))) void bs_bwd_dx_kernel(const T* __restrict__ dy,
                                                                  const T* __restrict__ nsrc,
                                                                  const float* __restrict__ inv_norm,
                                                                  const T* __restrict__ gamma,
@@ -351,7 +348,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
                                                                  BandArgs a) {
   constexpr int kBI = 64;
   static_assert(BM == 64 || (BM == 128 && !NORM), "tile rows");
-  __shared__ T lds[gemm_lds_elems<T, kBI, BM>()];
+  __shared__ T lds[gemm_lds_elems<T, kBI, BM, SPLIT>()];
   __shared__ float sinv[BM];
   __shared__ float sdot[4][BM];
   constexpr int WR = BM == 64 ? 4 : 2, WC = 4 / WR;
@@ -386,7 +383,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
   for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gemm_mainloop<T, kBI, BM, WR, WC, PMSST_BS_DX_DEPTH>(la, lb, O, lds, acc);
+  gemm_mainloop<T, kBI, BM, WR, WC, PMSST_BS_DX_DEPTH, SPLIT>(la, lb, O, lds, acc);
 
   if constexpr (!NORM) {
 #pragma unroll
@@ -556,21 +553,20 @@ __global__ __launch_bounds__(256) void bs_dx_finish_kernel(const float* __restri
 // ------------------------------------------------------------------ backward: dW
 
 constexpr int kDwBI = 64;
-// Output columns of a block: 128 for the fp32 grouped linear (768 of them and K = the rows: the x slab is
+// Output columns of a block: 128 for the split grouped linear (768 of them and K = the rows: the x slab is
 // read half as often, and a wave's fragments serve twice the products), else 64.
-template <typename T, bool NORM>
-constexpr int dw_cols() { return sizeof(T) == 4 && !NORM ? 128 : 64; }
+constexpr int dw_cols(bool norm, bool split) { return split && !norm ? 128 : 64; }
 
 // NORM = false: plain grouped linear, dW_b^T = x_b^T dy_b (no gamma / inv_norm scaling).
-template <typename T, bool FROM_X, bool NORM, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void bs_bwd_dw_kernel(const T* __restrict__ dy,
+template <typename T, bool FROM_X, bool NORM, bool V4, bool SPLIT = false>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(SPLIT ? kSplitWaves : 1))) void bs_bwd_dw_kernel(const T* __restrict__ dy,
                                                                  const T* __restrict__ nsrc,
                                                                  const float* __restrict__ inv_norm,
                                                                  const T* __restrict__ gamma, T* __restrict__ dw,
                                                                  T* __restrict__ db, int max_itiles, XcdGrid xg,
                                                                  BandSched sc, BandArgs a) {
-  constexpr int kDwBO = dw_cols<T, NORM>();
-  __shared__ T lds[gemm_lds_elems<T, kDwBI, kDwBO>()];
+  constexpr int kDwBO = dw_cols(NORM, SPLIT);
+  __shared__ T lds[gemm_lds_elems<T, kDwBI, kDwBO, SPLIT>()];
   using S = TileShape<kDwBI, kDwBO, 2, 2>;
   const int O = a.O;
   int band, i0, o0;
@@ -612,7 +608,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
   for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gemm_mainloop<T, kDwBI, kDwBO, 2, 2, PMSST_BS_DW_DEPTH>(la, lb, static_cast<int>(a.M), lds, acc);
+  gemm_mainloop<T, kDwBI, kDwBO, 2, 2, PMSST_BS_DW_DEPTH, SPLIT>(la, lb, static_cast<int>(a.M), lds, acc);
   if (lb.colsum) reduce_colsum<T, kDwBO, V4>(lb, lds, db + static_cast<int64_t>(band) * O + o0);
 
   T* dwb = dw + static_cast<int64_t>(O) * off;  // [O][I]
@@ -1179,6 +1175,17 @@ uint32_t dw_grid(const HostBands& hb, int64_t O, int64_t cols, const XcdGrid& xg
   return xg.blocks();
 }
 
+// Whether the fp32 dW takes the split: with fewer blocks than CUs a block's walk over the rows is the time,
+// and the split's, with one LDS tile, is the longer one (62 groups of 64 -> 256, 124 blocks: 1032 rows 35
+// against 50 us, 192 -> 768, 1116 blocks: 203 against 158).  Widths in whole fours only: masked loads cost
+// it more (mono bands, O = 192, 1896 rows: 84 against 121 us).
+bool split_dw(const HostBands& hb, int64_t M, int64_t O, bool norm) {
+  const int64_t otiles = (O + dw_cols(norm, true) - 1) / dw_cols(norm, true);
+  int64_t blocks = 0;
+  for (int b = 0; b < hb.NB; ++b) blocks += (hb.widths[b] + kDwBI - 1) / kDwBI * otiles;
+  return split_macs(M, hb.F, O) && blocks >= num_cus();
+}
+
 // 64-wide output tiles per forward block (capacity 64 * TO >= min(O, 256)).
 int tile_capacity(int64_t O) {
   const int64_t t = (O + 63) / 64;
@@ -1215,33 +1222,38 @@ int launch_fwd(const void* x, int64_t x_stride, const void* gamma, const void* w
   const T* pb = static_cast<const T*>(bias);
   T* po = static_cast<T*>(out);
   T* pn = static_cast<T*>(normed);
-#define PMSST_BSF(TO, V4)                                                                                           \
-  do {                                                                                                              \
-    if (!norm && act == PMSST_ACT_TANH)                                                                             \
-      hipLaunchKernelGGL((bs_fwd_kernel<T, TO, false, false, PMSST_ACT_TANH, V4>), grid, dim3(kGemmThreads), 0,      \
-                         stream, px, pg, pw, pb, po, pn, inv_norm, a);                                              \
-    else if (!norm)                                                                                                 \
-      hipLaunchKernelGGL((bs_fwd_kernel<T, TO, false, false, PMSST_ACT_NONE, V4>), grid, dim3(kGemmThreads), 0,      \
-                         stream, px, pg, pw, pb, po, pn, inv_norm, a);                                              \
-    else if (pn != nullptr)                                                                                         \
-      hipLaunchKernelGGL((bs_fwd_kernel<T, TO, true, true, PMSST_ACT_NONE, V4>), grid, dim3(kGemmThreads), 0, stream, \
-                         px, pg, pw, pb, po, pn, inv_norm, a);                                                      \
-    else                                                                                                            \
-      hipLaunchKernelGGL((bs_fwd_kernel<T, TO, false, true, PMSST_ACT_NONE, V4>), grid, dim3(kGemmThreads), 0,       \
-                         stream, px, pg, pw, pb, po, pn, inv_norm, a);                                              \
-  } while (0)
+  auto with_tile = [&](auto to, auto v4, auto split) {
+    constexpr int TO = decltype(to)::value;
+    constexpr bool V4 = decltype(v4)::value, SPLIT = decltype(split)::value;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, px, pg, pw, pb, po, pn, inv_norm, a);
+    };
+    if (!norm && act == PMSST_ACT_TANH) go(bs_fwd_kernel<T, TO, false, false, PMSST_ACT_TANH, V4, SPLIT>);
+    else if (!norm) go(bs_fwd_kernel<T, TO, false, false, PMSST_ACT_NONE, V4, SPLIT>);
+    else if (pn != nullptr) go(bs_fwd_kernel<T, TO, true, true, PMSST_ACT_NONE, V4, SPLIT>);
+    else go(bs_fwd_kernel<T, TO, false, true, PMSST_ACT_NONE, V4, SPLIT>);
+  };
   // Unaligned shapes (odd band widths) take one scalar-load variant with the widest tile.
-  if (!a.vec4) {
-    PMSST_BSF(4, false);
-  } else {
-    switch (tile_capacity(O)) {
-      case 1: PMSST_BSF(1, true); break;
-      case 2: PMSST_BSF(2, true); break;
-      case 3: PMSST_BSF(3, true); break;
-      default: PMSST_BSF(4, true); break;
+  auto launch = [&](auto split) {
+    if (!a.vec4) {
+      with_tile(std::integral_constant<int, 4>{}, std::false_type{}, split);
+    } else {
+      switch (tile_capacity(O)) {
+        case 1: with_tile(std::integral_constant<int, 1>{}, std::true_type{}, split); break;
+        case 2: with_tile(std::integral_constant<int, 2>{}, std::true_type{}, split); break;
+        case 3: with_tile(std::integral_constant<int, 3>{}, std::true_type{}, split); break;
+        default: with_tile(std::integral_constant<int, 4>{}, std::true_type{}, split); break;
+      }
     }
+  };
+  // Masked loads take the split from twice the products (O = 192, mono bands at 1032 rows, 0.41 G: 78 against
+  // 86 us; mono mel bands at 1032 rows, 0.78 G: 100 against 80).
+  if constexpr (sizeof(T) == 4) {
+    if (split_macs(a.vec4 ? M : M / 2, hb.F, O)) launch(std::true_type{});
+    else launch(std::false_type{});
+  } else {
+    launch(std::false_type{});
   }
-#undef PMSST_BSF
   return check_launch("bs_fwd_kernel");
 }
 
@@ -1323,15 +1335,22 @@ int launch_bwd(const void* dy, const void* nsrc, bool from_x, const float* inv_n
     const int max_ichunks = (hb.max_width + 63) / 64;
     const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>(m_tiles)};
     const dim3 grid(dx_sched ? per_xcd * kXcds : xg.blocks());
-#define PMSST_BDX(FX, V4)                                                                                          \
-  hipLaunchKernelGGL((bs_bwd_dx_kernel<T, FX, true, V4>), grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm, pg, \
-                     pw, static_cast<T*>(dx), tbuf, partial, pdot, pitch, max_ichunks, xg, sc, a)
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm, pg, pw, static_cast<T*>(dx),
+                         tbuf, partial, pdot, pitch, max_ichunks, xg, sc, a);
+    };
+    // fp32: the split where the widths are whole fours (mono bands, O = 192: 55 against 54 us, no gain)
+    constexpr bool kF32 = sizeof(T) == 4;
+    const bool split = kF32 && v4 && split_macs(M, hb.F, O);
     if (from_x) {
-      if (v4) PMSST_BDX(true, true); else PMSST_BDX(true, false);
+      if (split) go(bs_bwd_dx_kernel<T, true, true, true, 64, kF32>);
+      else if (v4) go(bs_bwd_dx_kernel<T, true, true, true>);
+      else go(bs_bwd_dx_kernel<T, true, true, false>);
     } else {
-      if (v4) PMSST_BDX(false, true); else PMSST_BDX(false, false);
+      if (split) go(bs_bwd_dx_kernel<T, false, true, true, 64, kF32>);
+      else if (v4) go(bs_bwd_dx_kernel<T, false, true, true>);
+      else go(bs_bwd_dx_kernel<T, false, true, false>);
     }
-#undef PMSST_BDX
     int rc = check_launch("bs_bwd_dx_kernel");
     if (rc != PMSST_OK) return rc;
     if (!fold_finish) {  // else the DMA dW kernel's tail blocks finish dx
@@ -1375,19 +1394,25 @@ int launch_bwd(const void* dy, const void* nsrc, bool from_x, const float* inv_n
   if (!dw_done) {
     BandSched wsc;
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
-    constexpr int kCols = dw_cols<T, true>();
+    constexpr int kCols = dw_cols(true, false);  // the split's too
     const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kCols - 1) / kCols)};
     const dim3 grid(dw_grid(hb, O, kCols, xg, &wsc));
     const bool v4 = a.vec4 && a.ovec4;
-#define PMSST_BDW(FX, V4)                                                                                   \
-  hipLaunchKernelGGL((bs_bwd_dw_kernel<T, FX, true, V4>), grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm, \
-                     pg, static_cast<T*>(dw), static_cast<T*>(db), max_itiles, xg, wsc, a)
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, pdy, pn, inv_norm, pg, static_cast<T*>(dw),
+                         static_cast<T*>(db), max_itiles, xg, wsc, a);
+    };
+    constexpr bool kF32 = sizeof(T) == 4;
+    const bool split = kF32 && v4 && split_dw(hb, M, O, true);
     if (from_x) {
-      if (v4) PMSST_BDW(true, true); else PMSST_BDW(true, false);
+      if (split) go(bs_bwd_dw_kernel<T, true, true, true, kF32>);
+      else if (v4) go(bs_bwd_dw_kernel<T, true, true, true>);
+      else go(bs_bwd_dw_kernel<T, true, true, false>);
     } else {
-      if (v4) PMSST_BDW(false, true); else PMSST_BDW(false, false);
+      if (split) go(bs_bwd_dw_kernel<T, false, true, true, kF32>);
+      else if (v4) go(bs_bwd_dw_kernel<T, false, true, true>);
+      else go(bs_bwd_dw_kernel<T, false, true, false>);
     }
-#undef PMSST_BDW
     int rc = check_launch("bs_bwd_dw_kernel");
     if (rc != PMSST_OK) return rc;
   }
@@ -1427,18 +1452,25 @@ int launch_grouped_bwd(const void* dy, const void* x, const void* weight, const 
     }
   } else if (M > 0) {
     const int max_ichunks = (hb.max_width + 63) / 64;
-    constexpr int kRows = bs_dx_rows<T, false>();
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>((M + kRows - 1) / kRows)};
+    const bool v4 = a.vec4 && a.ovec4;
+    constexpr bool kF32 = sizeof(T) == 4;
+    // The split's 128-row tiles pay where they are full and every CU has more than one: 62 groups of 192 ->
+    // 768: 64 rows 26 against 34 us, 130 rows (372 blocks) 52 against 46; 32 groups, 320 rows (288) 39
+    // against 44, 600 rows (480) 68 against 49; 62 groups of 64 -> 256, 1032 rows (558) 34 against 28.
+    const int64_t split_blocks = hb.NB * max_ichunks * ((M + 127) / 128);
+    const bool split =
+        kF32 && v4 && split_macs(M, hb.F, O) && M > 64 && 5 * split_blocks >= int64_t{6} * num_cus();
+    const int rows = split ? 128 : 64;
+    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_ichunks), static_cast<uint32_t>((M + rows - 1) / rows)};
     const dim3 grid(xg.blocks());
     const BandSched nosc{};  // groups of one width: every XcdGrid block has a chunk
-    if (a.vec4 && a.ovec4)
-      hipLaunchKernelGGL((bs_bwd_dx_kernel<T, false, false, true>), grid, dim3(kGemmThreads), 0, stream, pdy, px,
-                         nullptr, nullptr, pw, static_cast<T*>(dx), nullptr, nullptr, nullptr, 0, max_ichunks, xg, nosc,
-                         a);
-    else
-      hipLaunchKernelGGL((bs_bwd_dx_kernel<T, false, false, false>), grid, dim3(kGemmThreads), 0, stream, pdy, px,
-                         nullptr, nullptr, pw, static_cast<T*>(dx), nullptr, nullptr, nullptr, 0, max_ichunks, xg, nosc,
-                         a);
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, pdy, px, nullptr, nullptr, pw,
+                         static_cast<T*>(dx), nullptr, nullptr, nullptr, 0, max_ichunks, xg, nosc, a);
+    };
+    if (split) go(bs_bwd_dx_kernel<T, false, false, true, kF32 ? 128 : 64, kF32>);
+    else if (v4) go(bs_bwd_dx_kernel<T, false, false, true>);
+    else go(bs_bwd_dx_kernel<T, false, false, false>);
     int rc = check_launch("bs_bwd_dx_kernel");
     if (rc != PMSST_OK) return rc;
   }
@@ -1454,16 +1486,20 @@ int launch_grouped_bwd(const void* dy, const void* x, const void* weight, const 
     }
   } else {
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
-    constexpr int kCols = dw_cols<T, false>();
-    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kCols - 1) / kCols)};
+    const bool v4 = a.vec4 && a.ovec4;
+    constexpr bool kF32 = sizeof(T) == 4;
+    const bool split = kF32 && v4 && split_dw(hb, M, O, false);
+    const int cols = dw_cols(false, split);
+    const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + cols - 1) / cols)};
     BandSched wsc;
-    const dim3 grid(dw_grid(hb, O, kCols, xg, &wsc));
-    if (a.vec4 && a.ovec4)
-      hipLaunchKernelGGL((bs_bwd_dw_kernel<T, false, false, true>), grid, dim3(kGemmThreads), 0, stream, pdy, px,
-                         nullptr, nullptr, static_cast<T*>(dw), static_cast<T*>(db), max_itiles, xg, wsc, a);
-    else
-      hipLaunchKernelGGL((bs_bwd_dw_kernel<T, false, false, false>), grid, dim3(kGemmThreads), 0, stream, pdy, px,
-                         nullptr, nullptr, static_cast<T*>(dw), static_cast<T*>(db), max_itiles, xg, wsc, a);
+    const dim3 grid(dw_grid(hb, O, cols, xg, &wsc));
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(kGemmThreads), 0, stream, pdy, px, nullptr, nullptr, static_cast<T*>(dw),
+                         static_cast<T*>(db), max_itiles, xg, wsc, a);
+    };
+    if (split) go(bs_bwd_dw_kernel<T, false, false, true, kF32>);
+    else if (v4) go(bs_bwd_dw_kernel<T, false, false, true>);
+    else go(bs_bwd_dw_kernel<T, false, false, false>);
     int rc = check_launch("bs_bwd_dw_kernel");
     if (rc != PMSST_OK) return rc;
   }
@@ -1635,7 +1671,7 @@ int launch_mixed_bwd(const void* dy, const float* x, int64_t x_stride, const voi
   // other shapes: the norm-free register-staged dW kernel (it also runs for M == 0 and then writes zeros)
   {
     const int max_itiles = (hb.max_width + kDwBI - 1) / kDwBI;
-    constexpr int kCols = dw_cols<T, false>();
+    constexpr int kCols = dw_cols(false, false);
     const XcdGrid xg{static_cast<uint32_t>(hb.NB * max_itiles), static_cast<uint32_t>((O + kCols - 1) / kCols)};
     BandSched wsc;
     const dim3 grid(dw_grid(hb, O, kCols, xg, &wsc));

@@ -12,16 +12,18 @@
 // aligned and conflict-free, and the transposed stores of MNLoader (8 bytes to
 // rows 4q..4q+3) spread over all banks.
 //
-// fp32: each value is split on its way into LDS into three bf16 numbers, x = x1 + x2 + x3 (each the
-// rest's round-to-nearest bf16; 8 + 8 + 8 significant bits, so the sum is exact), and a product is the
-// six bf16 MFMAs a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1 with fp32 accumulation; the three left out are
-// below 2^-25 of it.  bf16 products are exact in fp32, so the result's error stays that of the fp32 sums
-// (measured against 64 bits: no larger than with the fp32 MFMAs), at 6 x 16 matrix-core cycles per 16 x 16
-// x 32 instead of 8 x 32, and 3 LDS reads of 16 bytes per fragment instead of 8 of 4.  A tile holds three
-// planes, of 64-byte rows (swz_k)
-// or, from an MNLoader, of 32 K-rows as they are stored (swz_mn_p; read transposed).  A non-finite accumulator (an infinity or a NaN among the inputs, or
-// one above bf16's largest, whose split is not finite; or an overflow) sends the block through the sum
-// again on the fp32 MFMAs, which give such inputs their usual results.
+// fp32 tiles use a plain odd pitch and the fp32 MFMAs, whose sum of a result is the chain of fused
+// multiply-adds over k, bit for bit.  Large fp32 products (split_macs) take SPLIT instead: each value is
+// split on its way into LDS into three bf16 numbers, x = x1 + x2 + x3 (each the rest's round-to-nearest
+// bf16; 8 + 8 + 8 significant bits, so the sum is exact), and a product is the six bf16 MFMAs a1 b1, a1 b2,
+// a2 b1, a2 b2, a1 b3, a3 b1 with fp32 accumulation; the three left out are below 2^-25 of it.  bf16
+// products are exact in fp32, so the result's error stays that of the fp32 sums (measured against 64 bits:
+// no larger than with the fp32 MFMAs), at 6 x 16 matrix-core cycles per 16 x 16 x 32 instead of 8 x 32, and
+// 3 LDS reads of 16 bytes per fragment instead of 8 of 4.  A tile holds three planes, of 64-byte rows
+// (swz_k) or, from an MNLoader, of 32 K-rows as they are stored (swz_mn_p; read transposed).  A non-finite
+// accumulator (an infinity or a NaN among the inputs, or one above bf16's largest, whose split is not
+// finite; or an overflow) sends the block through the sum again on the fp32 MFMAs, which give such inputs
+// their usual results.
 //
 // Waves are laid out WR x WC over the tile; wave (wr, wc) owns rows
 // [wr * BR/WR, ...) and columns [wc * BC/WC, ...) as TR x TC 16x16 tiles.
@@ -126,7 +128,7 @@ using raw_t = typename std::conditional<sizeof(T) == 2, uint16_t, uint32_t>::typ
 template <typename T>
 using quad_t = typename std::conditional<sizeof(T) == 2, uint2, uint4>::type;
 
-// LDS floats per tile row of the fp32 path: three bf16 planes of 64 bytes (the fp32 re-run's rows of
+// LDS floats per tile row of a split tile: three bf16 planes of 64 bytes (the fp32 re-run's rows of
 // LdsPitch<float> fit in them).
 constexpr int kSplitRow = 48;
 static_assert(kSplitRow >= LdsPitch<float>::value, "the fp32 re-run's tile fits");
@@ -553,18 +555,30 @@ struct TileShape {
   static_assert(kTR >= 1 && kTC >= 1 && BR % (WR * 16) == 0 && BC % (WC * 16) == 0, "bad tile");
 };
 
-// LDS elements the main loop needs for a BR x BC tile (16-bit: two buffers; fp32: one split tile).
-template <typename T, int BR, int BC>
+// LDS elements the main loop needs for a BR x BC tile (two buffers; SPLIT: one split tile).
+template <typename T, int BR, int BC, bool SPLIT = false>
 constexpr int gemm_lds_elems() {
-  return sizeof(T) == 2 ? 2 * (BR + BC) * LdsPitch<T>::value : (BR + BC) * kSplitRow;
+  return SPLIT ? (BR + BC) * kSplitRow : 2 * (BR + BC) * LdsPitch<T>::value;
 }
 
-// Register budget of the fp32 kernels with 8 or fewer 16 x 16 tiles a wave, in waves per SIMD: their K
+// Register budget of the split kernels with 8 or fewer 16 x 16 tiles a wave, in waves per SIMD: their K
 // steps wait on loads and barriers, which three blocks a CU cover better than two (224 against 228-324
 // us for the mask backward's input gradient).
 constexpr int kSplitWaves = 3;
 
-// The fp32 K loop: one LDS tile, the next chunk's loads in registers while this one is multiplied (the
+// Multiply-adds of a launch from which an fp32 product takes the split.  Below them the fp32 MFMAs need
+// less than 4 us for the products themselves; launches, loads and barriers are the time, and the split
+// gains little or loses: the tiny model's mask MLP (130 rows, 64 -> 256, 0.27 G at most a launch) 148
+// against 138 us, its band split 45.5 against 44.6, 32 bands of odd widths 128 against 131 and 64.2
+// against 64.9.  What it would cost there is the sums' exact bits: a loss that takes absolute values (an
+// L1 on spectra) turns the sign of one element of half a million, and so all gradients by 2e-3, when the
+// estimate moves by 1e-7 of its size.  At 0.3 to 0.6 G (62 bands, 192 -> 768, 64 rows) 226 against 197 us.
+constexpr int64_t kSplitMacs = 300'000'000;
+inline bool split_macs(int64_t rows, int64_t in_features, int64_t out_features) {
+  return rows * in_features >= (kSplitMacs + out_features - 1) / out_features;
+}
+
+// The K loop of a SPLIT kernel: one LDS tile, the next chunk's loads in registers while this one is multiplied (the
 // blocks of a CU, two to six of them, cover each other's splits and barriers).  SPLIT: three bf16 planes
 // and six products; else the fp32 MFMAs.
 template <int BR, int BC, int WR, int WC, bool SPLIT, class LA, class LB>
@@ -695,13 +709,16 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
 // loop is unrolled by two so the sets stay fixed registers).  Buffer offsets are
 // computed from the __shared__ base (no pointer tables), so every LDS access stays
 // a ds_* instruction and waits only on the LDS counter.
-template <typename T, int BR, int BC, int WR, int WC, int DEPTH = 1, class LA, class LB>
+//
+// SPLIT (fp32): gemm_f32_loop on the three bf16 planes, and again on the fp32 MFMAs if a sum is not finite.
+template <typename T, int BR, int BC, int WR, int WC, int DEPTH = 1, bool SPLIT = false, class LA, class LB>
 __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
                                               f32x4_t (&acc)[TileShape<BR, BC, WR, WC>::kTR]
                                                             [TileShape<BR, BC, WR, WC>::kTC]) {
   static_assert(DEPTH == 1 || DEPTH == 2, "prefetch depth 1 or 2");
+  static_assert(!SPLIT || sizeof(T) == 4, "fp32 only");
   using S = TileShape<BR, BC, WR, WC>;
-  if constexpr (sizeof(T) == 4) {
+  if constexpr (SPLIT) {
     if (K <= 0) return;
     const LA la0 = la;  // the loaders' row and column sums start again with a re-run
     const LB lb0 = lb;

@@ -82,12 +82,12 @@ struct LeftGateLoader : KRowLoader<T, 128, V4> {
 #endif
 constexpr int kFwdBM = 128;
 
-template <typename T, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 ? PMSST_ME_FWD_WAVES : 2))) void me_fwd_kernel(const T* __restrict__ x, const T* __restrict__ weight,
+template <typename T, bool V4, bool SPLIT = false>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(SPLIT ? 2 : PMSST_ME_FWD_WAVES))) void me_fwd_kernel(const T* __restrict__ x, const T* __restrict__ weight,
                                                               const T* __restrict__ bias, T* __restrict__ pre,
                                                               T* __restrict__ out, int max_lchunks, XcdGrid xg,
                                                               MaskArgs a, BandSched sc) {
-  __shared__ T lds[gemm_lds_elems<T, 128, kFwdBM>()];
+  __shared__ T lds[gemm_lds_elems<T, 128, kFwdBM, SPLIT>()];
   using S = TileShape<128, kFwdBM, 1, 4>;  // TR = 8 (4 left + 4 gate), TC = 2
   int band, l0;
   uint32_t mt;
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
   for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gemm_mainloop<T, 128, kFwdBM, 1, 4, PMSST_ME_FWD_DEPTH>(la, lb, H, lds, acc);
+  gemm_mainloop<T, 128, kFwdBM, 1, 4, PMSST_ME_FWD_DEPTH, SPLIT>(la, lb, H, lds, acc);
 
   const int64_t pitch2 = 2 * static_cast<int64_t>(a.F);
 #pragma unroll
@@ -510,12 +510,12 @@ constexpr int kDxBM = 64;
 
 // TANH_IN: the layer input x is tanh(z) of the previous layer, and the kernel writes
 // dz = (dpre W_b) * (1 - x^2) instead of dx (the hidden activation's backward, fused).
-template <typename T, bool TANH_IN, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void me_bwd_dx_kernel(const T* __restrict__ dpre,
+template <typename T, bool TANH_IN, bool V4, bool SPLIT = false>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(SPLIT ? kSplitWaves : 1))) void me_bwd_dx_kernel(const T* __restrict__ dpre,
                                                                  const T* __restrict__ weight,
                                                                  const T* __restrict__ x, T* __restrict__ dx,
                                                                  int hchunks, XcdGrid xg, MaskArgs a) {
-  __shared__ T lds[gemm_lds_elems<T, kDxBH, kDxBM>()];
+  __shared__ T lds[gemm_lds_elems<T, kDxBH, kDxBM, SPLIT>()];
   using S = TileShape<kDxBH, kDxBM, 2, 2>;
   uint32_t grp, mt;  // group = (band, hidden chunk), member = row tile: weight chunk shared in L2
   if (!xcd_block(xg, grp, mt)) return;
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int hr = (wave >> 1) * (kDxBH / 2), mc = (wave & 1) * (kDxBM / 2);
-  gemm_mainloop<T, kDxBH, kDxBM, 2, 2>(la, lb, 2 * I, lds, acc);
+  gemm_mainloop<T, kDxBH, kDxBM, 2, 2, 1, SPLIT>(la, lb, 2 * I, lds, acc);
 
 #pragma unroll
   for (int i = 0; i < S::kTR; ++i) {
@@ -761,11 +761,11 @@ __global__ __launch_bounds__(512) void me_bwd_dx_dma_kernel(const T* __restrict_
 constexpr int kDwBH = 128;
 constexpr int kDwBJ = 64;
 
-template <typename T, bool V4>
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (V4 ? kSplitWaves : 2) : 1))) void me_bwd_dw_kernel(const T* __restrict__ dpre, const T* __restrict__ x,
+template <typename T, bool V4, bool SPLIT = false>
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(SPLIT ? kSplitWaves : 1))) void me_bwd_dw_kernel(const T* __restrict__ dpre, const T* __restrict__ x,
                                                                  T* __restrict__ dw, T* __restrict__ dbias,
                                                                  int htiles, XcdGrid xg, MaskArgs a, BandSched sc) {
-  __shared__ T lds[gemm_lds_elems<T, kDwBH, kDwBJ>()];
+  __shared__ T lds[gemm_lds_elems<T, kDwBH, kDwBJ, SPLIT>()];
   using S = TileShape<kDwBH, kDwBJ, 2, 2>;
   int band, h0, j0, off, I;
   if (sc.m_tiles != 0) {
@@ -804,7 +804,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(si
   for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
     for (int j = 0; j < S::kTC; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gemm_mainloop<T, kDwBH, kDwBJ, 2, 2>(la, lb, static_cast<int>(a.M), lds, acc);
+  gemm_mainloop<T, kDwBH, kDwBJ, 2, 2, 1, SPLIT>(la, lb, static_cast<int>(a.M), lds, acc);
   if (lb.colsum) reduce_colsum<T, kDwBJ, V4>(lb, lds, dbias + 2 * off + j0);
 
   T* dwb = dw + static_cast<int64_t>(2) * off * H;  // [2I][H]
@@ -1128,14 +1128,19 @@ int launch_me_fwd(const void* x, const void* weight, const void* bias, const int
                                 &sc, &per_xcd)
                    ? per_xcd * kXcds
                    : grid.x);
-  if (a.vec4)
-    hipLaunchKernelGGL((me_fwd_kernel<T, true>), g, dim3(kGemmThreads), 0, stream, static_cast<const T*>(x),
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, g, dim3(kGemmThreads), 0, stream, static_cast<const T*>(x),
                        static_cast<const T*>(weight), static_cast<const T*>(bias), static_cast<T*>(pre),
                        static_cast<T*>(out), max_lchunks, xg, a, sc);
-  else
-    hipLaunchKernelGGL((me_fwd_kernel<T, false>), g, dim3(kGemmThreads), 0, stream, static_cast<const T*>(x),
-                       static_cast<const T*>(weight), static_cast<const T*>(bias), static_cast<T*>(pre),
-                       static_cast<T*>(out), max_lchunks, xg, a, sc);
+  };
+  constexpr bool kF32 = sizeof(T) == 4;
+  if (kF32 && split_macs(M, 2 * static_cast<int64_t>(hm.F), H)) {
+    if (a.vec4) go(me_fwd_kernel<T, true, kF32>);
+    else go(me_fwd_kernel<T, false, kF32>);
+  } else {
+    if (a.vec4) go(me_fwd_kernel<T, true>);
+    else go(me_fwd_kernel<T, false>);
+  }
   return check_launch("me_fwd_kernel");
 }
 
@@ -1162,6 +1167,11 @@ int launch_me_bwd(const void* gout, const void* x, const void* pre, const void* 
   a.vec4 = hm.vec4 && al(x, 4 * sizeof(T)) && al(weight, 4 * sizeof(T)) && al(pre, 4 * sizeof(T)) &&
            al(dx, 4 * sizeof(T)) && al(gout, 4 * sizeof(T)) && al(dw, 4 * sizeof(T));
   T* dpre = static_cast<T*>(workspace);
+  // fp32 dx and dW: the split where the widths are whole fours (62 bands, H = 768, 1032 rows: dx 267 against
+  // 216 us, dW 177 against 132); masked loads cost it what it gains (mono bands: dx 367 against 347, at 1896
+  // rows 614 each, dW 181 against 204; 32 odd widths, H = 2048: dx 473 against 514)
+  constexpr bool kF32 = sizeof(T) == 4;
+  const bool split = kF32 && a.vec4 && split_macs(M, 2 * static_cast<int64_t>(hm.F), H);
   if (M > 0) {
     const dim3 g1(static_cast<unsigned>((M + kDpreRows - 1) / kDpreRows), static_cast<unsigned>(hm.NB));
     const int64_t flat_threads = (M + kDpreFlatRows - 1) / kDpreFlatRows * (hm.F / 4);
@@ -1222,15 +1232,19 @@ int launch_me_bwd(const void* gout, const void* x, const void* pre, const void* 
       const int hchunks = static_cast<int>((H + kDxBH - 1) / kDxBH);
       const XcdGrid xg2{static_cast<uint32_t>(hm.NB * hchunks), static_cast<uint32_t>((M + kDxBM - 1) / kDxBM)};
       const dim3 g2(xg2.blocks());
-#define PMSST_MDX(TANH, V4)                                                                                    \
-  hipLaunchKernelGGL((me_bwd_dx_kernel<T, TANH, V4>), g2, dim3(kGemmThreads), 0, stream, dpre,                   \
-                     static_cast<const T*>(weight), static_cast<const T*>(x), static_cast<T*>(dx), hchunks, xg2, a)
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, g2, dim3(kGemmThreads), 0, stream, dpre, static_cast<const T*>(weight),
+                           static_cast<const T*>(x), static_cast<T*>(dx), hchunks, xg2, a);
+      };
       if (input_act == PMSST_ACT_TANH) {
-        if (a.vec4) PMSST_MDX(true, true); else PMSST_MDX(true, false);
+        if (split) go(me_bwd_dx_kernel<T, true, true, kF32>);
+        else if (a.vec4) go(me_bwd_dx_kernel<T, true, true>);
+        else go(me_bwd_dx_kernel<T, true, false>);
       } else {
-        if (a.vec4) PMSST_MDX(false, true); else PMSST_MDX(false, false);
+        if (split) go(me_bwd_dx_kernel<T, false, true, kF32>);
+        else if (a.vec4) go(me_bwd_dx_kernel<T, false, true>);
+        else go(me_bwd_dx_kernel<T, false, false>);
       }
-#undef PMSST_MDX
       rc = check_launch("me_bwd_dx_kernel");
       if (rc != PMSST_OK) return rc;
     }
@@ -1265,12 +1279,13 @@ int launch_me_bwd(const void* gout, const void* x, const void* pre, const void* 
                     &w3_per_xcd)
                     ? w3_per_xcd * kXcds
                     : xg3.blocks());
-  if (a.vec4)
-    hipLaunchKernelGGL((me_bwd_dw_kernel<T, true>), g3, dim3(kGemmThreads), 0, stream, dpre, static_cast<const T*>(x),
-                       static_cast<T*>(dw), static_cast<T*>(dbias), htiles, xg3, a, wsc3);
-  else
-    hipLaunchKernelGGL((me_bwd_dw_kernel<T, false>), g3, dim3(kGemmThreads), 0, stream, dpre,
-                       static_cast<const T*>(x), static_cast<T*>(dw), static_cast<T*>(dbias), htiles, xg3, a, wsc3);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, g3, dim3(kGemmThreads), 0, stream, dpre, static_cast<const T*>(x), static_cast<T*>(dw),
+                       static_cast<T*>(dbias), htiles, xg3, a, wsc3);
+  };
+  if (split) go(me_bwd_dw_kernel<T, true, kF32>);
+  else if (a.vec4) go(me_bwd_dw_kernel<T, true>);
+  else go(me_bwd_dw_kernel<T, false>);
   int rc = check_launch("me_bwd_dw_kernel");
   if (rc != PMSST_OK) return rc;
   // dbias was summed by the dW kernel (which also runs for M == 0 and then writes zeros)

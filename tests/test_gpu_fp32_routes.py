@@ -1,0 +1,111 @@
+"""fp32 products on both sides of the rule that splits large ones into bf16 parts (gemm.h).
+
+Below it a result is the chain of fused multiply-adds over k that the fp32 matrix cores compute, bit for
+bit: the tiny model's steps, whose L1 loss turns a change of 1e-7 in its estimate into one of 2e-3 in its
+gradients when an element passes its target, keep their outputs.  The chain is emulated in 64-bit
+significands (a product of two fp32 numbers is exact in 48 bits; rounding the sum to 64 bits first changes
+the fp32 result with a chance of 2^-40 an element).  Above it the error against 64 bits stays below
+sqrt(K) / 2 roundings of the fp32 sum.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.conftest import assert_parity, by_band, by_index, to_np
+from tests.test_gpu_band_split import BSR_WIDTHS, _check_ragged
+
+pytestmark = pytest.mark.gpu
+
+
+def _chain(a, b):
+    """``sum_k a[m, k] b[n, k]``, one fp32 rounding a term, in order of k."""
+    a, b = a.cpu().numpy().astype(np.longdouble), b.cpu().numpy().astype(np.longdouble)
+    acc = np.zeros((a.shape[0], b.shape[0]), np.float32)
+    for k in range(a.shape[1]):
+        acc = (acc + a[:, k, None] * b[None, :, k]).astype(np.float32)
+    return torch.from_numpy(acc)
+
+
+def _layer(m, groups, i, o, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(m, groups, i, generator=g)
+    w = torch.randn(groups, o, i, generator=g) / i**0.5
+    return x, w, torch.randn(m, groups, o, generator=g)
+
+
+@pytest.mark.parametrize("m,groups,i,o", [(1, 1, 1, 1), (33, 3, 7, 10), (65, 2, 36, 64), (130, 62, 64, 256),
+                                          (97, 62, 192, 256)])  # the last: 0.295 G multiply-adds, just below the rule
+def test_small_products_are_fused_chains(hip_ext, m, groups, i, o):
+    x, w, dy = _layer(m, groups, i, o, 5)
+    out = hip_ext.grouped_linear_forward(x.cuda(), w.cuda()).cpu()
+    dx, dw, _ = hip_ext.grouped_linear_backward(dy.cuda(), x.cuda(), w.cuda(), False)
+    for g in {0, groups - 1}:
+        assert torch.equal(out[:, g], _chain(x[:, g], w[g]))
+        assert torch.equal(dx[:, g].cpu(), _chain(dy[:, g], w[g].t()))
+        assert torch.equal(dw[g].cpu(), _chain(dy[:, g].t(), x[:, g].t()))
+
+
+def test_the_tiny_models_final_layer_is_a_fused_chain(hip_ext):
+    m, h = 130, 256  # 0.273 G multiply-adds, the tiny step's largest launch
+    g = torch.Generator().manual_seed(6)
+    x = torch.tanh(torch.randn(m, len(BSR_WIDTHS), h, generator=g))
+    ws = [torch.randn(2 * d, h, generator=g) / h**0.5 for d in BSR_WIDTHS]
+    bias = 0.1 * torch.randn(2 * sum(BSR_WIDTHS), generator=g)
+    wall = torch.cat([w.reshape(-1) for w in ws]).cuda()
+    _, pre = hip_ext.mask_estimator_final_forward_packed(x.cuda(), wall, bias.cuda(), BSR_WIDTHS)
+    at = 0
+    for b, d in enumerate(BSR_WIDTHS):
+        if b in (0, 44, 61):
+            cols = slice(2 * at, 2 * (at + d))
+            assert torch.equal(pre[:, cols].cpu(), _chain(x[:, b], ws[b]) + bias[cols])
+        at += d
+
+
+@pytest.mark.parametrize("m,groups,i,o", [
+    (99, 62, 192, 256),   # just above: the forward and dW split, dx (186 blocks of 128 rows) not
+    (130, 62, 192, 256),  # all three
+    (300, 62, 100, 260),  # columns, outputs and rows that end inside a tile, a partial K chunk each way
+    (700, 62, 101, 140),  # widths no vector load fits: the forward alone
+])
+def test_large_products_keep_the_error_of_fp32_sums(hip_ext, m, groups, i, o):
+    x, w, dy = (t.cuda() for t in _layer(m, groups, i, o, 7))
+    out = hip_ext.grouped_linear_forward(x, w)
+    dx, dw, db = hip_ext.grouped_linear_backward(dy, x, w, True)
+    xd, wd, dyd = x.double().transpose(0, 1).contiguous(), w.double(), dy.double().transpose(0, 1).contiguous()
+    wt, dyt = wd.transpose(1, 2).contiguous(), dyd.transpose(1, 2).contiguous()
+    exact = (torch.matmul(xd, wt).transpose(0, 1), torch.matmul(dyd, wd).transpose(0, 1), torch.matmul(dyt, xd))
+    for got, want, k in zip((out, dx, dw), exact, (i, o, m)):
+        rel = ((got.double() - want).norm() / want.norm()).item()
+        assert rel <= 2.0**-23.5 * (1 + k**0.5 / 2), (rel, k)
+    assert_parity(db, to_np(dyd.sum(1)), "f32", "db")
+
+
+@pytest.mark.parametrize("m,o", [(372, 192), (382, 192), (500, 260)])  # 0.293 G, 0.301 G, 0.53 G
+def test_band_split_across_the_rule(hip_ext, m, o):
+    _check_ragged(hip_ext, BSR_WIDTHS, m, o, torch.float32, 9)
+
+
+@pytest.mark.parametrize("m", [142, 144, 200])  # 62 bands, hidden 256: 0.298 G, 0.302 G, 0.42 G
+def test_mask_final_across_the_rule(hip_ext, m):
+    h, dims = 256, BSR_WIDTHS
+    g = torch.Generator().manual_seed(10)
+    x = torch.tanh(torch.randn(m, len(dims), h, generator=g)).cuda()
+    ws = [torch.randn(2 * d, h, generator=g) / h**0.5 for d in dims]
+    wall = torch.cat([w.reshape(-1) for w in ws]).cuda()
+    bias = (0.1 * torch.randn(2 * sum(dims), generator=g)).cuda()
+    gout = torch.randn(m, sum(dims), generator=g).cuda()
+    out, pre = hip_ext.mask_estimator_final_forward_packed(x, wall, bias, dims)
+    npw = [to_np(w) for w in ws]
+    r_out, r_pre = oracle.mask_estimator_final_forward(to_np(x), npw, to_np(bias), dims, "f32")[:2]
+    assert_parity(out, r_out, "f32", "out")
+    assert_parity(pre, r_pre, "f32", "pre")
+    dz, db, dw = hip_ext.mask_estimator_final_backward_packed(gout, x, pre, wall, dims, input_activation="tanh")
+    r_dz, r_db, r_dw = oracle.mask_estimator_final_backward(to_np(gout), to_np(x), to_np(pre), npw, dims, "f32",
+                                                            input_act="tanh", grad_pre_dt="f32")
+    assert_parity(dz, r_dz, "f32", "dz", by_index(1))
+    assert_parity(db, r_db, "f32", "dbias", by_band(0, [2 * d for d in dims]))
+    assert_parity(dw, np.concatenate([w.reshape(-1) for w in r_dw]), "f32", "dW")
