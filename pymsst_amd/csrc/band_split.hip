@@ -82,6 +82,7 @@ struct XGammaLoader {
   int rows_valid;
   int k_valid;
   mutable float ss[kQuads] = {0.f, 0.f};
+  mutable uint32_t least = ~0u;  // see note_least
   int64_t src_row[kQuads] = {};
   uint32_t off[kQuads] = {};
 
@@ -122,7 +123,8 @@ struct XGammaLoader {
       // plain grouped linear: no gamma, no sums of squares
 #pragma unroll
       for (int i = 0; i < kQuads; ++i)
-        commit_quad<T, kBM, SPLIT>(lds, tile_row(i), kq, masked ? mask_quad<T>(g.q[i], (g.ok >> i) & 1) : g.q[i]);
+        commit_quad<T, kBM, SPLIT>(lds, tile_row(i), kq, masked ? mask_quad<T>(g.q[i], (g.ok >> i) & 1) : g.q[i],
+                                   least);
       return;
     }
     float gm[4];
@@ -137,7 +139,7 @@ struct XGammaLoader {
         ss[i] += v[j] * v[j];
         pk.v[j] = from_f32<T>(v[j] * gm[j]);
       }
-      commit_quad<T, kBM, SPLIT>(lds, tile_row(i), kq, __builtin_bit_cast(quad_t<T>, pk));
+      commit_quad<T, kBM, SPLIT>(lds, tile_row(i), kq, __builtin_bit_cast(quad_t<T>, pk), least);
     }
   }
   template <bool SPLIT>

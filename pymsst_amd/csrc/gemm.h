@@ -15,15 +15,16 @@
 // fp32 tiles use a plain odd pitch and the fp32 MFMAs, whose sum of a result is the chain of fused
 // multiply-adds over k, bit for bit.  Large fp32 products (split_macs) take SPLIT instead: each value is
 // split on its way into LDS into three bf16 numbers, x = x1 + x2 + x3 (each the rest's round-to-nearest
-// bf16; 8 + 8 + 8 significant bits, so the sum is exact), and a product is the six bf16 MFMAs a1 b1, a1 b2,
-// a2 b1, a2 b2, a1 b3, a3 b1 with fp32 accumulation; the three left out are below 2^-25 of it.  bf16
-// products are exact in fp32, so the result's error stays that of the fp32 sums (measured against 64 bits:
-// no larger than with the fp32 MFMAs), at 6 x 16 matrix-core cycles per 16 x 16 x 32 instead of 8 x 32, and
-// 3 LDS reads of 16 bytes per fragment instead of 8 of 4.  A tile holds three planes, of 64-byte rows
-// (swz_k) or, from an MNLoader, of 32 K-rows as they are stored (swz_mn_p; read transposed).  A non-finite
-// accumulator (an infinity or a NaN among the inputs, or one above bf16's largest, whose split is not
-// finite; or an overflow) sends the block through the sum again on the fp32 MFMAs, which give such inputs
-// their usual results.
+// bf16), and a product is the six bf16 MFMAs a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1 with fp32
+// accumulation; the three left out come to at most 2^-24 of it, 2^-27.5 in the mean square.  The sum is
+// exact (8 + 8 + 8 significant bits) from 2^-110 on; below, x3's last bits fall under bf16's smallest
+// number, 2^-133.  bf16 products are exact in fp32, so the result's error stays that of the fp32 sums
+// (measured against 64 bits: no larger than with the fp32 MFMAs), at 6 x 16 matrix-core cycles per 16 x 16
+// x 32 instead of 8 x 32, and 3 LDS reads of 16 bytes per fragment instead of 8 of 4.  A tile holds three
+// planes, of 64-byte rows (swz_k) or, from an MNLoader, of 32 K-rows as they are stored (swz_mn_p; read
+// transposed).  A block that has met a number other than 0 below 2^-110, or has a non-finite accumulator
+// (an infinity or a NaN among the inputs, or one above bf16's largest, whose split is not finite; or an
+// overflow), goes through the sum again on the fp32 MFMAs, which give such inputs their usual results.
 //
 // Waves are laid out WR x WC over the tile; wave (wr, wc) owns rows
 // [wr * BR/WR, ...) and columns [wc * BC/WC, ...) as TR x TC 16x16 tiles.
@@ -148,6 +149,17 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&w)[3]) {
   }
 }
 
+// The least of 2 |x| - 1, as bits, over the numbers a thread has split (0 counts as the largest): below
+// kSplitLeast some number other than 0 is under 2^-110.
+constexpr uint32_t kSplitLeast = 2u * (17u << 23) - 1u;
+__device__ __forceinline__ void note_least(const float (&v)[4], uint32_t& least) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t b = 2u * __float_as_uint(v[j]) - 1u;
+    least = b < least ? b : least;
+  }
+}
+
 // Byte offset of element (r, k) inside plane 0 of a split tile; plane p is p * ROWS * 64 bytes on.
 __device__ __forceinline__ int split_offset(int r, int k) {
   return r * 64 + 16 * ((k >> 3) ^ swz_k(r & 15)) + 2 * (k & 7);
@@ -155,7 +167,8 @@ __device__ __forceinline__ int split_offset(int r, int k) {
 
 // 4 consecutive k (k % 4 == 0) of row r into the three planes.
 template <int ROWS>
-__device__ __forceinline__ void put_split(float* lds, int r, int k, const float (&v)[4]) {
+__device__ __forceinline__ void put_split(float* lds, int r, int k, const float (&v)[4], uint32_t& least) {
+  note_least(v, least);
   char* dst = reinterpret_cast<char*>(lds) + split_offset(r, k);
   uint32_t lo[3], hi[3];
   split_pair(v[0], v[1], lo);
@@ -166,7 +179,8 @@ __device__ __forceinline__ void put_split(float* lds, int r, int k, const float 
 
 // 4 consecutive rows mn (mn % 4 == 0) of K-row k into the three planes of a tile that keeps K-rows.
 template <int ROWS>
-__device__ __forceinline__ void put_split_mn(float* lds, int mn, int k, const float (&v)[4]) {
+__device__ __forceinline__ void put_split_mn(float* lds, int mn, int k, const float (&v)[4], uint32_t& least) {
+  note_least(v, least);
   char* dst = reinterpret_cast<char*>(lds) + k * 2 * ROWS + 16 * ((mn >> 3) ^ swz_mn_p<2 * ROWS>(k)) + 2 * (mn & 7);
   uint32_t lo[3], hi[3];
   split_pair(v[0], v[1], lo);
@@ -249,12 +263,14 @@ __device__ __forceinline__ void quad_to_f32(const quad_t<T>& q, float (&o)[4]) {
   }
 }
 
-// Stores a quad of consecutive k (kq % 4 == 0) of LDS row r (SPLIT: fp32 as three bf16 planes).
+// Stores a quad of consecutive k (kq % 4 == 0) of LDS row r (SPLIT: fp32 as three bf16 planes; `least` as
+// note_least keeps it).
 template <typename T, int ROWS, bool SPLIT>
-__device__ __forceinline__ void commit_quad(T* lds, int r, int kq, const quad_t<T>& q) {
+__device__ __forceinline__ void commit_quad(T* lds, int r, int kq, const quad_t<T>& q,
+                                            [[maybe_unused]] uint32_t& least) {
   if constexpr (SPLIT) {
     const float v[4] = {__uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z), __uint_as_float(q.w)};
-    put_split<ROWS>(lds, r, kq, v);
+    put_split<ROWS>(lds, r, kq, v, least);
   } else if constexpr (sizeof(T) == 2) {
     *reinterpret_cast<uint2*>(lds + lds_index<T>(r, kq)) = q;
   } else {
@@ -285,6 +301,7 @@ struct KRowLoader {
   int64_t src_row[kQuads] = {};  // source row of each of the thread's tile rows (clamped)
   uint32_t off[kQuads] = {};     // byte offset of (src_row, k = 4 (t % 8)) from base
   uint32_t rowok = 0;            // bit i: tile row i of this thread is a real row
+  mutable uint32_t least = ~0u;  // see note_least
 
   static __device__ __forceinline__ int tile_row(int i) {
     return (static_cast<int>(threadIdx.x) + i * kGemmThreads) / (kChunkK / 4);
@@ -320,7 +337,7 @@ struct KRowLoader {
   __device__ __forceinline__ void commit_edge(const Regs& g, T* lds) const {
 #pragma unroll
     for (int i = 0; i < kQuads; ++i)
-      commit_quad<T, ROWS, SPLIT>(lds, tile_row(i), lane_k(), mask_quad<T>(g.q[i], (g.ok >> i) & 1));
+      commit_quad<T, ROWS, SPLIT>(lds, tile_row(i), lane_k(), mask_quad<T>(g.q[i], (g.ok >> i) & 1), least);
   }
   __device__ __forceinline__ void fetch(int k0, Regs& g) const {
     if constexpr (V4) {
@@ -334,7 +351,7 @@ struct KRowLoader {
   __device__ __forceinline__ void commit(const Regs& g, T* lds) const {
     if constexpr (V4) {
 #pragma unroll
-      for (int i = 0; i < kQuads; ++i) commit_quad<T, ROWS, SPLIT>(lds, tile_row(i), lane_k(), g.q[i]);
+      for (int i = 0; i < kQuads; ++i) commit_quad<T, ROWS, SPLIT>(lds, tile_row(i), lane_k(), g.q[i], least);
     } else {
       commit_edge<SPLIT>(g, lds);
     }
@@ -374,6 +391,7 @@ struct MNLoader {
   mutable float csum[4] = {0.f, 0.f, 0.f, 0.f};
   int mn_src = 0;                          // this thread's (clamped) mn quad start
   uint32_t off[KB] = {};                   // byte offset of (kb + t, mn_src) from a chunk base
+  mutable uint32_t least = ~0u;            // see note_least
 
   static __device__ __forceinline__ int lane_mn() { return (threadIdx.x % kQuadsPerK) * 4; }
   static __device__ __forceinline__ int lane_kb() { return (threadIdx.x / kQuadsPerK) * KB; }
@@ -437,7 +455,7 @@ struct MNLoader {
     }
     if constexpr (SPLIT) {
 #pragma unroll
-      for (int t = 0; t < KB; ++t) put_split_mn<ROWS>(lds, mn, kb + t, v[t]);
+      for (int t = 0; t < KB; ++t) put_split_mn<ROWS>(lds, mn, kb + t, v[t], least);
       return;
     }
 #pragma unroll
@@ -710,7 +728,8 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
 // computed from the __shared__ base (no pointer tables), so every LDS access stays
 // a ds_* instruction and waits only on the LDS counter.
 //
-// SPLIT (fp32): gemm_f32_loop on the three bf16 planes, and again on the fp32 MFMAs if a sum is not finite.
+// SPLIT (fp32): gemm_f32_loop on the three bf16 planes, and again on the fp32 MFMAs if a sum is not finite
+// or a number too small for an exact split was among the operands.
 template <typename T, int BR, int BC, int WR, int WC, int DEPTH = 1, bool SPLIT = false, class LA, class LB>
 __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
                                               f32x4_t (&acc)[TileShape<BR, BC, WR, WC>::kTR]
@@ -723,14 +742,14 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
     const LA la0 = la;  // the loaders' row and column sums start again with a re-run
     const LB lb0 = lb;
     gemm_f32_loop<BR, BC, WR, WC, true>(la, lb, K, lds, acc);
-    bool finite = true;
+    bool good = (la.least < lb.least ? la.least : lb.least) >= kSplitLeast;
 #pragma unroll
     for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
       for (int j = 0; j < S::kTC; ++j)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) finite = finite && fabsf(acc[i][j][r]) <= 3.402823466e38f;
-    if (__syncthreads_or(!finite)) {
+        for (int r = 0; r < 4; ++r) good = good && fabsf(acc[i][j][r]) <= 3.402823466e38f;
+    if (__syncthreads_or(!good)) {
       la = la0;
       lb = lb0;
 #pragma unroll

@@ -5,7 +5,7 @@ bit: the tiny model's steps, whose L1 loss turns a change of 1e-7 in its estimat
 gradients when an element passes its target, keep their outputs.  The chain is emulated in 64-bit
 significands (a product of two fp32 numbers is exact in 48 bits; rounding the sum to 64 bits first changes
 the fp32 result with a chance of 2^-40 an element).  Above it the error against 64 bits stays below
-sqrt(K) / 2 roundings of the fp32 sum.
+sqrt(K) / 2 roundings of the fp32 sum, also for numbers that three bf16 parts cannot hold.
 """
 
 from __future__ import annotations
@@ -73,6 +73,11 @@ def test_the_tiny_models_final_layer_is_a_fused_chain(hip_ext):
 ])
 def test_large_products_keep_the_error_of_fp32_sums(hip_ext, m, groups, i, o):
     x, w, dy = (t.cuda() for t in _layer(m, groups, i, o, 7))
+    _check_against_64_bits(hip_ext, x, w, dy)
+
+
+def _check_against_64_bits(hip_ext, x, w, dy):
+    (m, _, i), o = x.shape, w.shape[1]
     out = hip_ext.grouped_linear_forward(x, w)
     dx, dw, db = hip_ext.grouped_linear_backward(dy, x, w, True)
     xd, wd, dyd = x.double().transpose(0, 1).contiguous(), w.double(), dy.double().transpose(0, 1).contiguous()
@@ -82,6 +87,27 @@ def test_large_products_keep_the_error_of_fp32_sums(hip_ext, m, groups, i, o):
         rel = ((got.double() - want).norm() / want.norm()).item()
         assert rel <= 2.0**-23.5 * (1 + k**0.5 / 2), (rel, k)
     assert_parity(db, to_np(dyd.sum(1)), "f32", "db")
+
+
+@pytest.mark.parametrize("exp", [-108, -112, -118, -124])
+def test_numbers_too_small_for_bf16_parts(hip_ext, exp):
+    """bf16 ends at 2^-133, so below 2^-110 three parts no longer hold 24 bits: 2^-118 lost 1e-5 of its
+    value, also where a large weight makes the result an ordinary number."""
+    x, w, dy = (t.cuda() for t in _layer(300, 62, 128, 260, 8))
+    _check_against_64_bits(hip_ext, torch.ldexp(x, torch.tensor(exp)), torch.ldexp(w, torch.tensor(100)), dy)
+
+
+def test_a_single_small_number(hip_ext):
+    x, w, _ = (t.cuda() for t in _layer(300, 62, 128, 260, 8))
+    clean = hip_ext.grouped_linear_forward(x, w)
+    x[5, 3] = 0.0
+    x[5, 3, 7] = 1.2345678 * 2.0**-121
+    w2 = w.clone()
+    w2[3, :, 7] *= 2.0**100
+    out = hip_ext.grouped_linear_forward(x, w2)
+    assert torch.equal(out[5, 3], x[5, 3, 7] * w2[3, :, 7])
+    others = torch.arange(62) != 3
+    assert torch.equal(out[:, others], clean[:, others])
 
 
 @pytest.mark.parametrize("m,o", [(372, 192), (382, 192), (500, 260)])  # 0.293 G, 0.301 G, 0.53 G
