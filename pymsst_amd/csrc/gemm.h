@@ -626,9 +626,14 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
     la.template commit<SPLIT>(ra, lds);
     lb.template commit<SPLIT>(rb, lds_b);
   }
-  // Where the registers allow, the products of the low parts have accumulators of their own, 2^-8 the
-  // size: the matrix cores cut a sum off one-sidedly (column sums of the result, over a thousand rows,
-  // showed it), and so the large accumulators are cut off once a chunk instead of six times.
+  // The matrix cores cut what a product adds below the accumulator's last place off one-sidedly, towards
+  // minus infinity.  The products of the high parts, 16 bits long, hardly reach below it; those of the low
+  // parts, 2^-8 and less of them, added to the same accumulator leave a mean error of -1.1e-8 of the
+  // result's RMS at K = 192 and -1.0e-7 at K = 2048, where the fp32 MFMAs' is within 1e-9.  So the low
+  // parts' products are summed apart: with 8 or fewer tiles a wave in accumulators of their own, added at
+  // the end, and with more, for want of registers, from zero in each chunk, added by a rounded addition:
+  // 7e-10 and 4e-10, and the error in the mean square from 1.9e-7 to 0.9e-7 and from 7.0e-7 to 3.1e-7, for
+  // 4 % of the forward's time (62 groups of 192 -> 768, 1032 rows: 212 -> 221 us).
   constexpr bool kLow = SPLIT && S::kTR * S::kTC <= 8;
   f32x4_t low[kLow ? S::kTR : 1][kLow ? S::kTC : 1];
 #pragma unroll
@@ -638,9 +643,15 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
   auto mma = [&]() {
     if constexpr (SPLIT) {
       constexpr int kP[6][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}, {0, 0}};  // small parts first
-      auto term = [&](int i, int j, int q, const bf16x8_t (&a)[3], const bf16x8_t (&b)[3]) {
-        f32x4_t& d = kLow && q < 5 ? low[kLow ? i : 0][kLow ? j : 0] : acc[i][j];
+      auto term = [&](int i, int j, int q, const bf16x8_t (&a)[3], const bf16x8_t (&b)[3], f32x4_t& chunk) {
+        f32x4_t& d = q == 5 ? acc[i][j] : kLow ? low[kLow ? i : 0][kLow ? j : 0] : chunk;
         d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kP[q][0]], b[kP[q][1]], d, 0, 0, 0);
+      };
+      auto add_chunk = [&](int i, int j, const f32x4_t& chunk) {
+        if constexpr (!kLow) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][j][r] += chunk[r];
+        }
       };
       auto frag = [&](auto tr, const float* tile, auto rows, int r, int t, bf16x8_t (&f)[3]) {
         constexpr int ROWS = decltype(rows)::value;
@@ -659,19 +670,29 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
       using RowsB = std::integral_constant<int, BC>;
       using TrA = std::integral_constant<bool, LA::kTransposed>;
       using TrB = std::integral_constant<bool, LB::kTransposed>;
-      // the operand with fewer tiles stays in registers, the other's tiles pass by
+      // The operand with fewer tiles stays in registers, the other's tiles pass by, with 4 x 4 tiles twice, once
+      // for each half of the first: all of its parts beside the chunk sums spill, and so do the sums of
+      // several passing tiles, which the scheduling barrier keeps apart.
       if constexpr (S::kTR <= S::kTC) {
-        bf16x8_t a[S::kTR][3];
+        constexpr int kHold = !kLow && S::kTR == 4 ? 2 : S::kTR;
 #pragma unroll
-        for (int i = 0; i < S::kTR; ++i) frag(TrA{}, lds, RowsA{}, r0, i, a[i]);
+        for (int h = 0; h < S::kTR; h += kHold) {
+          bf16x8_t a[kHold][3];
 #pragma unroll
-        for (int j = 0; j < S::kTC; ++j) {
-          bf16x8_t b[3];
-          frag(TrB{}, lds_b, RowsB{}, c0, j, b);
+          for (int i = 0; i < kHold; ++i) frag(TrA{}, lds, RowsA{}, r0, h + i, a[i]);
 #pragma unroll
-          for (int q = 0; q < 6; ++q)
+          for (int j = 0; j < S::kTC; ++j) {
+            bf16x8_t b[3];
+            frag(TrB{}, lds_b, RowsB{}, c0, j, b);
+            f32x4_t chunk[kHold] = {};
 #pragma unroll
-            for (int i = 0; i < S::kTR; ++i) term(i, j, q, a[i], b);
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+              for (int i = 0; i < kHold; ++i) term(h + i, j, q, a[i], b, chunk[i]);
+#pragma unroll
+            for (int i = 0; i < kHold; ++i) add_chunk(h + i, j, chunk[i]);
+            if constexpr (!kLow) __builtin_amdgcn_sched_barrier(0);
+          }
         }
       } else {
         bf16x8_t b[S::kTC][3];
@@ -681,10 +702,13 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
         for (int i = 0; i < S::kTR; ++i) {
           bf16x8_t a[3];
           frag(TrA{}, lds, RowsA{}, r0, i, a);
+          f32x4_t chunk[S::kTC] = {};
 #pragma unroll
           for (int q = 0; q < 6; ++q)
 #pragma unroll
-            for (int j = 0; j < S::kTC; ++j) term(i, j, q, a, b[j]);
+            for (int j = 0; j < S::kTC; ++j) term(i, j, q, a, b[j], chunk[j]);
+#pragma unroll
+          for (int j = 0; j < S::kTC; ++j) add_chunk(i, j, chunk[j]);
         }
       }
     } else {
@@ -692,7 +716,8 @@ __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
       for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
         for (int j = 0; j < S::kTC; ++j)
-          acc[i][j] = mfma_tile<float>(lds, r0 + i * 16 + (lane & 15), lds_b, c0 + j * 16 + (lane & 15), acc[i][j], lane);
+          acc[i][j] = mfma_tile<float>(lds, r0 + i * 16 + (lane & 15), lds_b, c0 + j * 16 + (lane & 15), acc[i][j],
+                                       lane);
     }
   };
   for (int kc = 0;;) {
