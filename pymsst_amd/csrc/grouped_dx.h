@@ -42,7 +42,7 @@ int launch_wide_dw(const void* dy, const void* x, void* dw, void* db, int64_t gr
                    int64_t out_features, int64_t rows, hipStream_t stream);
 
 // h[m, g, :] = tanh(x[m, g, :] W_g^T + bias_g), z rounded to the storage type before the tanh, on the same
-// file's forward tiles: 16-bit, in_features in whole 32s, out_features in whole eights, a bias.
+// file's forward tiles: 16-bit, in_features in whole 32s, out_features from 128 in whole eights, a bias.
 bool wide_tanh_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
                          const void* x, const void* w, const void* bias, const void* out);
 template <typename T>

@@ -411,7 +411,12 @@ int launch_wide_dw(const void* dy, const void* x, void* dw, void* db, int64_t gr
 
 bool wide_tanh_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
                          const void* x, const void* w, const void* bias, const void* out) {
-  return shape_ok(groups, in_features, out_features, rows, elem) && in_features % 32 == 0 && groups > 0 &&
+  // From 128 outputs: the tile is 192 or 256 wide.  64 outputs leave two thirds of it empty (62 groups of
+  // 192 -> 64: 31 rows 6.4 us against 9.2, 1896 rows 20 against 24; 64 -> 64: 15 against 19); at 128 the
+  // register-staged kernel takes 7.8 us at 31 rows and 28 at 1896 (62 groups of 64 -> 128), this one 7.7 and
+  // 20, and it stays ahead from one row and one group on (one group of 512 -> 2048, one row: 20 and 13 us;
+  // 62 groups of 192 -> 768, 31 rows: 15.5 and 11.0).
+  return out_features >= 128 && shape_ok(groups, in_features, out_features, rows, elem) && in_features % 32 == 0 && groups > 0 &&
          x != nullptr && w != nullptr && out != nullptr && in_features > 0 && out_features > 0 &&
          256 * in_features * 2 < (int64_t{1} << 31) && aligned16(x) && aligned16(w) && aligned16(out) &&
          bias != nullptr && reinterpret_cast<uintptr_t>(bias) % 8 == 0;
