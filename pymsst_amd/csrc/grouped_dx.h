@@ -28,8 +28,8 @@ int launch_uniform_dw(const void* dy, const void* x, void* dw, void* db, int64_t
                       int64_t out_features, int64_t rows, hipStream_t stream);
 
 // Whether the same two products run on grouped_gemm.hip's 256-wide tiles, which are taken first: 16-bit
-// layers of at least 192 inputs (dx at 192 and 256: where the grid fills its rounds), widths in whole
-// eights (dx: out_features in whole 32s), 16-byte aligned pointers.
+// layers of at least 192 inputs where the grid is large enough for the tiles (the rules stand at the
+// functions), widths in whole eights (dx: out_features in whole 32s), 16-byte aligned pointers.
 bool wide_dx_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
                        const void* dy, const void* w, const void* dx);
 template <typename T>

@@ -371,7 +371,18 @@ bool wide_dx_supported(int64_t groups, int64_t in_features, int64_t out_features
   if (!shape_ok(groups, in_features, out_features, rows, elem) || out_features % 32 != 0 || !aligned16(dy) ||
       !aligned16(w) || !aligned16(dx))
     return false;
-  if (in_features > 256) return true;  // glin_dx_kernel ends at 256; the register-staged kernel is the alternative
+  // Above 256, where glin_dx_kernel ends, the register-staged kernel with its 64 x 64 results a block is the
+  // alternative: it wins while it has fewer than 2.75 blocks' worth of results a CU, with few groups 4 (its
+  // blocks then walk a long K side by side where this kernel's tiles leave CUs idle).  62 groups of 512 ->
+  // 1024: 64 rows (1.9) 23.5 us against 26.4, 96 rows (2.9) 29 against 27, 130 rows 39 against 26; 384 ->
+  // 768: 80 rows (1.8) 18.9 against 19.3, 128 rows (2.9) 21.6 against 19.6; 30 groups of 512 -> 2048: 130
+  // rows (1.9) 38 against 43, 200 rows (2.9) 46 against 44; 16 of 768 -> 1536: 320 rows (3.75) 35.7 against
+  // 36.5, 600 rows (7) 69 against 39; 8 of 512 -> 2048: 600 rows (2.3) 38 against 45, 1032 rows (4) 58 against
+  // 47; one of 2048 -> 2048: 1500 rows (2.9) 40 against 45, 2760 rows (5.4) 68 against 47.
+  if (in_features > 256) {
+    const int64_t quarters = groups >= 24 ? 11 : 16;
+    return groups * rows * in_features >= quarters * 1024 * num_cus();
+  }
   // At 192 and 256 glin_dx_kernel's smaller blocks (two per CU) win unless whole rounds of one 256-row
   // block per CU are at least 80 % full: M = 1032, 62 groups of 192 -> 768: 310 blocks, 61 % of two
   // rounds, 53 us against 43; M = 2760, 60 groups: 660 blocks, 86 % of three, 89 us against 96.

@@ -42,3 +42,25 @@ def test_tanh_forward(hip_ext, m, groups, i, o, wide):
     out, names = launched(lambda: hip_ext.grouped_linear_forward_act(x, w, b, activation="tanh"))
     assert ("gg_kernel" in names) == wide and ("bs_fwd_kernel" in names) != wide
     assert_parity(out, oracle.grouped_linear_forward(to_np(x), to_np(w), to_np(b), "bf16", act="tanh"), "bf16", "tanh")
+
+
+def _check_backward(hip_ext, x, w, dy, dtype=torch.bfloat16):
+    (dx, dw, db), names = launched(lambda: hip_ext.grouped_linear_backward(dy, x, w, True))
+    dn = dt_name(dtype)
+    rdx, rdw, rdb = oracle.grouped_linear_backward(to_np(dy), to_np(x), to_np(w), True, dn)
+    assert_parity(dx, rdx, dn, "dx", by_index(1))
+    assert_parity(dw, rdw, dn, "dW", by_index(0))
+    assert_parity(db, rdb, dn, "db", by_index(0))
+    return names
+
+
+@pytest.mark.parametrize("m,groups,i,o,wide", [
+    (1, 3, 512, 32, False), (90, 62, 512, 64, False), (91, 62, 512, 64, True),   # 2.75 blocks a CU from 90.8 rows
+    (121, 62, 384, 64, False), (122, 62, 384, 96, True),                         # from 121.1 rows
+    (1023, 8, 512, 64, False), (1024, 8, 512, 64, True),                         # 4 blocks a CU
+    (129, 62, 320, 64, False), (146, 62, 320, 160, True), (173, 62, 264, 264, False),  # O no multiple of 32
+])
+def test_wide_input_gradient(hip_ext, m, groups, i, o, wide):
+    x, w, _, dy = _layer(m, groups, i, o)
+    names = _check_backward(hip_ext, x, w, dy)
+    assert ("bs_bwd_dx_kernel" in names) != wide
