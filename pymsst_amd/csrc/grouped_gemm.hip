@@ -402,15 +402,31 @@ bool wide_dw_supported(int64_t groups, int64_t in_features, int64_t out_features
   if (!shape_ok(groups, in_features, out_features, rows, elem) || in_features < 192 || rows < 32 || !aligned16(dy) ||
       !aligned16(x) || !aligned16(dw))
     return false;  // below 192 inputs columns of the tile stay empty
-  if (in_features > 256 || in_features % 64 != 0) return true;
-  // At 192 and 256 inputs me_bwd_dw_dma_kernel's smaller blocks win while the loop over the rows is short
-  // or the 256-row tiles leave CUs idle: 192 -> 768, 62 groups (186 blocks): 64 rows 8.8 us against 10.0,
-  // 320 rows 15.4 against 16.4, 600 rows 24.2 each, 1032 rows 37 against 36; 60 groups, 2760 rows 98
-  // against 90; 192 -> 384 (124 blocks): 162 rows 8.9 against 11.6, 600 rows 16.4 against 21.4.
-  const int64_t a_cols = in_features % 256 == 0 ? 256 : 192;
-  const int64_t blocks = groups * ((out_features + 255) / 256) * ((in_features + a_cols - 1) / a_cols);
-  const int64_t cus = num_cus(), rounds = (blocks + cus - 1) / cus;
-  return rows >= 1024 && 3 * blocks >= 2 * rounds * cus;
+  // Against the kernel that would run otherwise: how many rounds of its blocks, on the CUs it can use, stand
+  // against a round of this kernel's (one block per CU).  me_bwd_dw_dma_kernel (in_features in whole 64s; 64
+  // x 128 tiles) runs a group's blocks on one XCD; a round takes 18 us at 2760 rows, one of these tiles 92
+  // (256 inputs wide) or 73 (192).  Rounds against one, and the two times in us:
+  //   192 wide: 4.5 (62 groups of 192 -> 768): 320 rows 15.3, 15.9; 1032 rows 33.7, 32.7; 1400 rows 45.2, 41.8;
+  //     2760 rows 92, 77.  4.5 (62 of 384 -> 768): 1032 rows 60.8, 63.7; 1400 rows 80, 81; 1896 rows 109, 106.
+  //     6 (62 of 384 -> 1536): 128 rows 27.3, 29.5; 200 rows 36.8, 35.1; 1032 rows 120, 102.
+  //     3.1 (62 of 320 -> 640): 2760 rows 126, 144.
+  //   256 wide: 6 (62 of 256 -> 768): 64 rows 11.4, 10.7; 1032 rows 49, 38.  8 (62 of 512 -> 2048): 64 rows
+  //     38.7, 38.8; 1032 rows 225, 159.  4 (62 of 256 -> 512): 1032 rows 30.5, 37.2; 2760 rows 83, 84.  4.5
+  //     (16 of 768 -> 1536): 2760 rows 141, 145.  16 (one of 2048 -> 2048): 64 rows 18, 9.
+  const int64_t a_cols = in_features % 256 == 0 ? 256 : 192, cus = num_cus();
+  const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t rounds = cdiv(groups * cdiv(out_features, 256) * cdiv(in_features, a_cols), cus);
+  if (in_features % 64 == 0) {
+    const int64_t other = cdiv(groups, kXcds) * (in_features / 64) * cdiv(out_features, 128) * kXcds;  // blocks
+    if (a_cols == 256) return other >= 6 * rounds * cus && rows >= 64;
+    return (other >= 6 * rounds * cus && rows > 128) || (2 * other >= 9 * rounds * cus && rows >= 1400);
+  }
+  // Else the register-staged kernel, 64 x 64 tiles spread evenly: 6.8 (62 groups of 200 -> 400): 130 rows 12.6,
+  // 12.3, 320 rows 18.9, 15.4; 6.3 (62 of 200 -> 800): 200 rows 21.4, 22.8, 320 rows 28, 27; 5.5 (62 of 264 ->
+  // 528): 320 rows 24.6, 26.7, 600 rows 41.6, 39.4; 9.3 (62 of 520 -> 1040): 130 rows 38.7, 35.8; 1.6 (8 of
+  // 200 -> 800): 2760 rows 51, 64.
+  const int64_t other = groups * cdiv(in_features, 64) * cdiv(out_features, 64);
+  return other >= 5 * rounds * cus && rows * other >= 2000 * rounds * cus;
 }
 
 template <typename T>

@@ -47,10 +47,10 @@ def test_tanh_forward(hip_ext, m, groups, i, o, wide):
 def _check_backward(hip_ext, x, w, dy, dtype=torch.bfloat16):
     (dx, dw, db), names = launched(lambda: hip_ext.grouped_linear_backward(dy, x, w, True))
     dn = dt_name(dtype)
-    rdx, rdw, rdb = oracle.grouped_linear_backward(to_np(dy), to_np(x), to_np(w), True, dn)
-    assert_parity(dx, rdx, dn, "dx", by_index(1))
-    assert_parity(dw, rdw, dn, "dW", by_index(0))
-    assert_parity(db, rdb, dn, "db", by_index(0))
+    xd, dyd = (t.double().transpose(0, 1).contiguous() for t in (x, dy))
+    assert_parity(dx, torch.matmul(dyd, w.double()).transpose(0, 1), dn, "dx", by_index(1))
+    assert_parity(dw, torch.matmul(dyd.transpose(1, 2).contiguous(), xd), dn, "dW", by_index(0))
+    assert_parity(db, dyd.sum(1), dn, "db", by_index(0))
     return names
 
 
@@ -64,3 +64,33 @@ def test_wide_input_gradient(hip_ext, m, groups, i, o, wide):
     x, w, _, dy = _layer(m, groups, i, o)
     names = _check_backward(hip_ext, x, w, dy)
     assert ("bs_bwd_dx_kernel" in names) != wide
+
+
+@pytest.mark.parametrize("m,groups,i,o,wide", [
+    (63, 62, 256, 768, False), (64, 62, 256, 768, True),       # 256-wide tiles, 6 rounds against one
+    (97, 60, 256, 640, False),                                 # 5
+    (128, 62, 384, 1536, False), (129, 62, 384, 1416, True),   # 192-wide, 6; an output tile that ends after 136
+    (1399, 62, 192, 768, False), (1400, 62, 192, 768, True),   # 192-wide, 4.5
+    (1500, 62, 192, 384, False),                               # 2.25
+    (318, 62, 200, 800, True), (317, 62, 200, 800, False),     # no whole 64s: rows x 6.3 from 2000
+    (800, 62, 200, 200, False), (700, 8, 200, 200, False),     # 3.9, 0.5
+    (65, 2, 2048, 1024, True),                                 # few groups on few XCDs: 8
+])
+def test_wide_weight_gradient(hip_ext, m, groups, i, o, wide):
+    x, w, _, dy = _layer(m, groups, i, o)
+    names = _check_backward(hip_ext, x, w, dy)
+    assert ("me_bwd_dw_dma_kernel" in names or "bs_bwd_dw_kernel" in names) != wide
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,groups,i,o", [
+    (91, 62, 512, 32),      # dx: one K chunk
+    (257, 62, 264, 1056),   # dx: a tile of one row, one of 8 columns; dW not wide
+    (64, 62, 512, 1024),    # dW: two whole K chunks
+    (65, 60, 768, 1032),    # dW: three 256-wide tiles, an output tile of 8, a first chunk of one row
+    (161, 62, 384, 1536),   # dW: 192-wide tiles; dx: 48 K chunks
+    (416, 62, 264, 1056),   # both at a width in whole eights only
+])
+def test_wide_tiles_at_their_edges(hip_ext, dtype, m, groups, i, o):
+    x, w, _, dy = _layer(m, groups, i, o, dtype)
+    assert "gg_kernel" in _check_backward(hip_ext, x, w, dy, dtype)
