@@ -584,14 +584,19 @@ int launch_mlp_fwd(const void* x, const void* w1, const void* b1, const void* w2
 
 // Whether a hidden-layer and a final-layer kernel beat the one pass when the hidden layer is stored anyway.
 // The one pass recomputes GEMM1 for every 64 GLU outputs past a band's first, and from dim 384 on its
-// x fragments leave it 4 waves of 32 rows; the two kernels read the hidden layer once more.  Forward
-// with the hidden layer stored: dim 512, 62 bands, 1896 rows 770 -> 600 us; 60 mel bands (2.5 passes a
-// band), dim 192, 2760 rows 375 -> 346 us; 62 bands (1.6 passes), dim 192, 1032 rows 99 -> 131 us, so
-// there the one pass stays.
-bool two_kernels_better(int64_t dim, const int64_t* dim_inputs, int64_t band_count) {
+// x fragments leave it 4 waves of 32 rows; the two kernels read the hidden layer once more.  Forward with the
+// hidden layer stored, one pass and two kernels in us:
+//   62 bands (1.6 passes a band): dim 192, 1032 rows 99, 131.  dim 384 -> 768: 16 rows 31, 28; 130 rows 36.1,
+//     35.9; 1896 rows 253, 206.  dim 512 -> 2048: 31 rows 89, 53; 1896 rows 665, 536.
+//   60 mel bands (2.5 passes): dim 256 -> 1024: 16 rows 58, 29; 1896 rows 375, 284.  Below, the one pass wins
+//     while a single row tile of 256 holds the rows, and at dim 64 up to three: dim 192 -> 384: 31 rows 16,
+//     19; 256 rows 28, 31; 257 rows 46, 33; 513 rows 50, 46; 1896 rows 129, 112.  dim 128 -> 256: 256 rows 24,
+//     29; 257 rows 38, 29.  dim 64 -> 128: 256 rows 18, 22; 600 rows 32, 35; 800 rows 43, 41; 1896 rows 78, 60.
+bool two_kernels_better(int64_t rows, int64_t dim, const int64_t* dim_inputs, int64_t band_count) {
+  if (dim >= 384) return true;
   int64_t passes = 0;
   for (int64_t b = 0; b < band_count; ++b) passes += (dim_inputs[b] + kMlpJ - 1) / kMlpJ;
-  return dim >= 384 || passes > 2 * band_count;
+  return passes > 2 * band_count && (dim >= 256 || rows > (dim <= 64 ? 768 : 256));
 }
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
@@ -622,7 +627,7 @@ int mask_mlp_forward_impl(const char* op, const void* x, const void* w1, const v
   int64_t total = 0;
   for (int64_t b = 0; b < band_count; ++b) total += dim_inputs[b];
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (hidden_out != nullptr && two_kernels_better(dim, dim_inputs, band_count) &&
+  if (hidden_out != nullptr && two_kernels_better(rows, dim, dim_inputs, band_count) &&
       wide_tanh_supported(band_count, dim, hidden, rows, 2, x, w1, b1, hidden_out) &&
       mask_final_supported(dim_inputs, band_count, hidden)) {
     auto two = [&](auto tag) {

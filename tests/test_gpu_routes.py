@@ -94,3 +94,27 @@ def test_wide_weight_gradient(hip_ext, m, groups, i, o, wide):
 def test_wide_tiles_at_their_edges(hip_ext, dtype, m, groups, i, o):
     x, w, _, dy = _layer(m, groups, i, o, dtype)
     assert "gg_kernel" in _check_backward(hip_ext, x, w, dy, dtype)
+
+
+@pytest.mark.parametrize("m,dim,dims,two", [
+    (256, 192, (260, 200, 196, 140), False), (257, 192, (260, 200, 196, 140), True),
+    (256, 128, (260, 200, 196, 140), False), (257, 128, (260, 200, 196, 140), True),
+    (768, 64, (260, 200, 196, 140), False), (769, 64, (260, 200, 196, 140), True),
+    (3, 256, (260, 200, 196, 140), True), (3, 256, (8, 64, 132), False), (3, 384, (8, 64, 132), True),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_mask_mlp_forward(hip_ext, dtype, m, dim, dims, two):
+    """Both forms give the same bits: the call without the stored hidden layer always runs the one pass."""
+    hidden, nb = 160, len(dims)
+    g = torch.Generator().manual_seed(62)
+    x = torch.randn(m, nb, dim, generator=g).to(dtype).cuda()
+    w1 = (torch.randn(nb, hidden, dim, generator=g) / dim**0.5).to(dtype).cuda()
+    b1 = (0.1 * torch.randn(nb, hidden, generator=g)).to(dtype).cuda()
+    w2 = torch.cat([(torch.randn(2 * d, hidden, generator=g) / hidden**0.5).reshape(-1) for d in dims]).to(dtype).cuda()
+    b2 = (0.1 * torch.randn(2 * sum(dims), generator=g)).to(dtype).cuda()
+    (out, pre, hid), names = launched(lambda: hip_ext.mask_mlp_forward(x, w1, b1, w2, b2, dims, save_hidden=True))
+    assert ("gg_kernel" in names) == two and ("mlp_fwd_kernel" in names) != two
+    out1, pre1, _ = hip_ext.mask_mlp_forward(x, w1, b1, w2, b2, dims)
+    assert torch.equal(out, out1) and torch.equal(pre, pre1)
+    assert_parity(hid, oracle.mask_mlp_hidden(to_np(x), to_np(w1), to_np(b1), dt_name(dtype)), dt_name(dtype), "hidden",
+                  by_index(1))
