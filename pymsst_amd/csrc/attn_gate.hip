@@ -26,8 +26,8 @@
 // issue order).  The grids hold as many blocks as fit on the device at once, so a block's staging of
 // W is spread over as many tokens as possible.
 //
-// 16-bit, dim a multiple of 64 up to 512: the three products run on the matrix cores (gate_mfma_*_kernel
-// below), on the same 16-bit operands.
+// 16-bit, dim a multiple of 64 up to 512, where the products or the tokens are many (gate_mfma_*_pays): the
+// three products run on the matrix cores (gate_mfma_*_kernel below), on the same 16-bit operands.
 //
 // Any other shape runs the generic kernels (one wave per token, one head at a time).
 #include <algorithm>
@@ -761,6 +761,25 @@ inline bool gate_mfma_ok(const GateShape& s, size_t esz, const void* x, const vo
   return esz == 2 && al && s.dim % 64 == 0 && (nt <= 4 || nt == 6 || nt == 8) && s.rows() < (int64_t{1} << 30);
 }
 
+// Whether they pay, by the products a token needs (heads x dim) and the tokens.  The forward's blocks hold 64
+// tokens and load all of them before the first product, so a small grid waits where the vector kernels'
+// blocks, of fewer tokens, are done; 256 CUs have a block each from 16384 tokens.  us, vector and matrix
+// cores: heads 8 x dim 512: 31 tokens 7.0, 5.7; 2000 tokens 7.8, 7.8; 8060 tokens 15.7, 9.5.  8 x 192: 31
+// tokens 4.3, 4.7; 2000 tokens 5.1, 6.2; 8060 tokens 9.2, 7.3.  8 x 128: 8060 tokens 8.0, 6.9.  4 x 192: 8060
+// tokens 5.8, 6.2; 16120 tokens 8.7, 6.8.  4 x 64: 8060 tokens 4.8, 5.0; 16120 tokens 6.8, 5.3.
+inline bool gate_mfma_fwd_pays(const GateShape& s) {
+  const int64_t work = s.heads * s.dim, rows = s.rows();
+  return work >= 4096 || rows >= 16384 || (rows >= 8192 && work >= 1024);
+}
+// The backward's two transposes of gpre and its barrier a group cost as much as the products at narrow dims.
+// 8 x 192: 31 tokens 12.7, 10.8; 63984 tokens 67, 53.  8 x 128: 500 tokens 11.8, 12.9; 2000 tokens 13.8, 12.5;
+// 63984 tokens 54, 50.  4 x 192: 31 tokens 10.5, 10.5; 32000 tokens 28.4, 27.5; 117552 tokens 64.3, 66.8.  4 x
+// 64: 31 tokens 9.2, 11.3; 117552 tokens 37, 52.
+inline bool gate_mfma_bwd_pays(const GateShape& s) {
+  const int64_t work = s.heads * s.dim;
+  return work >= 1536 || (work >= 1024 && s.rows() >= 2000);
+}
+
 // f(E, NT) as integral constants.
 template <class F>
 void gate_mfma_dispatch(int e, int64_t dim, F&& f) {
@@ -808,7 +827,7 @@ int launch_gate_fwd(const void* attn, const int64_t* attn_strides, const void* x
     return check_launch("gate_fwd_generic_kernel");
   }
   if constexpr (sizeof(T) == 2) {
-    if (gate_mfma_ok(s, sizeof(T), x, weight, nullptr)) {
+    if (gate_mfma_ok(s, sizeof(T), x, weight, nullptr) && gate_mfma_fwd_pays(s)) {
       const dim3 grid(static_cast<unsigned>((rows + 16 * kGateWaves - 1) / (16 * kGateWaves)));
       gate_mfma_dispatch(e, s.dim, [&](auto ec, auto nt) {
         hipLaunchKernelGGL((gate_mfma_fwd_kernel<T, decltype(ec)::value, decltype(nt)::value>), grid,
@@ -912,7 +931,7 @@ int launch_gate_bwd(const void* grad_out, const void* attn, const int64_t* attn_
                          stream, gpre, px, pw, pbias, rows, heads, dim, static_cast<int>(gate_dw_chunk_rows(rows)));
       rc = check_launch("gate_dw_generic_kernel");
       if (rc != PMSST_OK) return rc;
-    } else if (gate_mfma_ok(s, sizeof(T), x, weight, grad_x)) {
+    } else if (gate_mfma_ok(s, sizeof(T), x, weight, grad_x) && gate_mfma_bwd_pays(s)) {
       if constexpr (sizeof(T) == 2) {
         // the groups of 32 tokens in equal turns of at most two blocks per CU
         const int64_t groups = (rows + 31) / 32;

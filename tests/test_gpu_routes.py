@@ -3,6 +3,7 @@ they measured slower than the kernels they replace (the figures stand at each ru
 
 from __future__ import annotations
 
+import numpy as np
 import pytest
 import torch
 
@@ -118,3 +119,33 @@ def test_mask_mlp_forward(hip_ext, dtype, m, dim, dims, two):
     assert torch.equal(out, out1) and torch.equal(pre, pre1)
     assert_parity(hid, oracle.mask_mlp_hidden(to_np(x), to_np(w1), to_np(b1), dt_name(dtype)), dt_name(dtype), "hidden",
                   by_index(1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("m,heads,dh,dim,fwd,bwd", [
+    (1, 8, 64, 512, True, True), (33, 16, 32, 256, True, True), (31, 16, 16, 384, True, False),  # 16 x 384: generic
+    (47, 8, 64, 384, False, True), (8193, 8, 64, 256, True, True), (8191, 8, 64, 256, False, True),
+    (8192, 4, 32, 192, False, False), (16384, 4, 32, 192, True, False), (1999, 8, 16, 128, False, False),
+    (2000, 8, 16, 128, False, True), (15, 8, 64, 192, False, True), (65, 16, 16, 128, False, True),
+    (16421, 2, 64, 64, True, False), (3001, 16, 8, 64, False, True), (16400, 4, 64, 128, True, False),
+])
+def test_attention_gate(hip_ext, dtype, m, heads, dh, dim, fwd, bwd):
+    """The matrix-core gate on both sides of its rules, at groups of 64 and 32 tokens that end anywhere and at
+    each dim it is built for."""
+    dn = dt_name(dtype)
+    g = torch.Generator().manual_seed(63)
+    attn = torch.randn(m, heads, dh, generator=g).to(dtype).cuda()
+    x = torch.randn(m, dim, generator=g).to(dtype).cuda()
+    w = (torch.randn(heads, dim, generator=g) / dim**0.5).to(dtype).cuda()
+    b = (0.1 * torch.randn(heads, generator=g)).to(dtype).cuda()
+    gout = torch.randn(m, heads * dh, generator=g).to(dtype).cuda()
+    (out, gate, *_), names = launched(lambda: hip_ext.attention_gate_forward(attn, x, w, b))
+    assert ("gate_mfma_fwd_kernel" in names) == fwd
+    r_out, r_gate = oracle.attention_gate_forward(to_np(attn), to_np(x), to_np(w), to_np(b), dn)[:2]
+    assert_parity(out, r_out.reshape(m, -1), dn, "out")
+    assert_parity(gate, r_gate, dn, "gate")
+    (ga, gx, gw, gb), names = launched(lambda: hip_ext.attention_gate_backward(gout, attn, x, w, gate))
+    assert ("gate_mfma_bwd_kernel" in names) == bwd
+    refs = oracle.attention_gate_backward(to_np(gout), to_np(attn), to_np(x), to_np(w), to_np(gate), dn)
+    for got, want, what in zip((ga, gx, gw, gb), refs, ("grad_attn", "grad_x", "grad_W", "grad_b")):
+        assert_parity(got, np.asarray(want).reshape(got.shape), dn, what)
