@@ -630,6 +630,14 @@ int mask_mlp_forward_impl(const char* op, const void* x, const void* w1, const v
   if (hidden_out != nullptr && two_kernels_better(rows, dim, dim_inputs, band_count) &&
       wide_tanh_supported(band_count, dim, hidden, rows, 2, x, w1, b1, hidden_out) &&
       mask_final_supported(dim_inputs, band_count, hidden)) {
+    // The one pass's tables are uploaded here too, as by every eager call: a later call under capture may need
+    // them (without the hidden layer, or with fewer rows) and could not upload them.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
+      const uint16_t* tabs = nullptr;
+      const int rc = tanh_tables(s, &tabs);
+      if (rc != PMSST_OK) return rc;
+    }
     auto two = [&](auto tag) {
       using T = decltype(tag);
       const int rc = launch_wide_tanh<T>(x, w1, b1, hidden_out, band_count, dim, hidden, rows, s);

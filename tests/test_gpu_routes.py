@@ -3,6 +3,10 @@ they measured slower than the kernels they replace (the figures stand at each ru
 
 from __future__ import annotations
 
+import subprocess
+import sys
+from pathlib import Path
+
 import numpy as np
 import pytest
 import torch
@@ -149,3 +153,35 @@ def test_attention_gate(hip_ext, dtype, m, heads, dh, dim, fwd, bwd):
     refs = oracle.attention_gate_backward(to_np(gout), to_np(attn), to_np(x), to_np(w), to_np(gate), dn)
     for got, want, what in zip((ga, gx, gw, gb), refs, ("grad_attn", "grad_x", "grad_W", "grad_b")):
         assert_parity(got, np.asarray(want).reshape(got.shape), dn, what)
+
+
+_CAPTURE_AFTER_WARM_UP = """
+import torch
+from pymsst_amd.fused_extension import load_fused_band_split_extension
+ext = load_fused_band_split_extension()
+dims, dim, hidden, m = (8, 64, 132), 384, 160, 70
+g = torch.Generator().manual_seed(64)
+x = torch.randn(m, len(dims), dim, generator=g).bfloat16().cuda()
+w1 = (torch.randn(len(dims), hidden, dim, generator=g) / dim**0.5).bfloat16().cuda()
+b1 = torch.randn(len(dims), hidden, generator=g).bfloat16().cuda()
+w2 = (torch.randn(2 * sum(dims) * hidden, generator=g) / hidden**0.5).bfloat16().cuda()
+b2 = torch.randn(2 * sum(dims), generator=g).bfloat16().cuda()
+want = ext.mask_mlp_forward(x, w1, b1, w2, b2, dims, save_hidden=True)
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+with torch.cuda.graph(graph):
+    got = ext.mask_mlp_forward(x, w1, b1, w2, b2, dims)
+for _ in range(3):
+    got[0].zero_()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+print("captured")
+"""
+
+
+def test_capture_of_the_one_pass_after_a_two_kernel_warm_up(hip_ext):
+    """A process of its own: the device's tanh tables are uploaded once."""
+    run = subprocess.run([sys.executable, "-c", _CAPTURE_AFTER_WARM_UP], cwd=Path(__file__).resolve().parents[1],
+                         capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and "captured" in run.stdout, run.stderr[-2000:]
