@@ -86,6 +86,7 @@ struct XGammaLoader {
   int64_t src_row[kQuads] = {};
   uint32_t off[kQuads] = {};
 
+  __device__ __forceinline__ void forget() { asm volatile("" : "+v"(rows_valid)); }
   static __device__ __forceinline__ int tile_row(int i) {
     return (static_cast<int>(threadIdx.x) + i * kGemmThreads) / (kChunkK / 4);
   }

@@ -303,6 +303,9 @@ struct KRowLoader {
   uint32_t rowok = 0;            // bit i: tile row i of this thread is a real row
   mutable uint32_t least = ~0u;  // see note_least
 
+  // For a second run of the K loop: what it derives from its rows is derived again, not kept in registers
+  // through the first run.
+  __device__ __forceinline__ void forget() { asm volatile("" : "+v"(rows_valid)); }
   static __device__ __forceinline__ int tile_row(int i) {
     return (static_cast<int>(threadIdx.x) + i * kGemmThreads) / (kChunkK / 4);
   }
@@ -393,6 +396,7 @@ struct MNLoader {
   uint32_t off[KB] = {};                   // byte offset of (kb + t, mn_src) from a chunk base
   mutable uint32_t least = ~0u;            // see note_least
 
+  __device__ __forceinline__ void forget() { asm volatile("" : "+v"(mn_valid)); }
   static __device__ __forceinline__ int lane_mn() { return (threadIdx.x % kQuadsPerK) * 4; }
   static __device__ __forceinline__ int lane_kb() { return (threadIdx.x / kQuadsPerK) * KB; }
 
@@ -777,6 +781,8 @@ __device__ __forceinline__ void gemm_mainloop(LA& la, LB& lb, int K, T* lds,
     if (__syncthreads_or(!good)) {
       la = la0;
       lb = lb0;
+      la.forget();
+      lb.forget();
 #pragma unroll
       for (int i = 0; i < S::kTR; ++i)
 #pragma unroll
