@@ -44,7 +44,7 @@ if str(REPO) not in sys.path:
 
 HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0
-FP32_PEAK_TFLOPS = 157.3
+FP32_PEAK_TFLOPS = BF16_PEAK_TFLOPS / 6  # an fp32 product of this size is six bf16 products (csrc/gemm.h)
 METRIC = "fused-layer fwd+bwd HBM GB/s (% peak) + BSR train samples/s, 1 MI355X"
 BSR_WIDTHS = tuple([8] * 24 + [16] * 12 + [48] * 8 + [96] * 8 + [192] * 8 + [512, 516])
 # ops of the step that are one kernel launched n times per op call: the roofline candidates

@@ -36,7 +36,6 @@ struct GgArgs {
   void* db;        // dw: bias gradient or null; fwd: bias
   int64_t M;
   int G, O, I;
-  int a_tiles;     // tiles of AR along the A rows
 };
 
 // One 16-byte-per-lane global -> LDS DMA from a uniform base plus a 32-bit byte offset per lane (see
@@ -339,13 +338,12 @@ int launch(const GgArgs& a, hipStream_t stream) {
   BandSched sc;
   uint32_t per_xcd = 0;
   constexpr int AR = 16 * TA * WA;
-  GgArgs ar = a;
   constexpr int BR = 16 * 4 * gg_waves(OP) / WA;
-  ar.a_tiles = ((OP == kGgFwd ? a.O : a.I) + AR - 1) / AR;
+  const int64_t a_tiles = ((OP == kGgFwd ? a.O : a.I) + AR - 1) / AR;  // tiles of AR along the A rows
   const int64_t b_rows = OP == kGgDw ? a.O : a.M;
-  if (!build_even_sched(a.G, (b_rows + BR - 1) / BR, [&](int) { return static_cast<int64_t>(ar.a_tiles); }, &sc, &per_xcd))
+  if (!build_even_sched(a.G, (b_rows + BR - 1) / BR, [&](int) { return a_tiles; }, &sc, &per_xcd))
     return fail(PMSST_EINVAL, "grouped linear: too many groups or rows for the block schedule");
-  hipLaunchKernelGGL((gg_kernel<T, OP, TA, WA>), dim3(per_xcd * kXcds), dim3(64 * gg_waves(OP)), 0, stream, ar, sc);
+  hipLaunchKernelGGL((gg_kernel<T, OP, TA, WA>), dim3(per_xcd * kXcds), dim3(64 * gg_waves(OP)), 0, stream, a, sc);
   return check_launch("gg_kernel");
 }
 
@@ -394,7 +392,7 @@ template <typename T>
 int launch_wide_dx(const void* dy, const void* w, void* dx, int64_t groups, int64_t in_features, int64_t out_features,
                    int64_t rows, hipStream_t stream) {
   return launch_op<T, kGgDx>(GgArgs{w, dy, dx, nullptr, rows, static_cast<int>(groups), static_cast<int>(out_features),
-                                    static_cast<int>(in_features), 0}, stream);
+                                    static_cast<int>(in_features)}, stream);
 }
 
 bool wide_dw_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
@@ -433,7 +431,7 @@ template <typename T>
 int launch_wide_dw(const void* dy, const void* x, void* dw, void* db, int64_t groups, int64_t in_features,
                    int64_t out_features, int64_t rows, hipStream_t stream) {
   return launch_op<T, kGgDw>(GgArgs{x, dy, dw, db, rows, static_cast<int>(groups), static_cast<int>(out_features),
-                                    static_cast<int>(in_features), 0}, stream);
+                                    static_cast<int>(in_features)}, stream);
 }
 
 bool wide_tanh_supported(int64_t groups, int64_t in_features, int64_t out_features, int64_t rows, size_t elem,
@@ -453,7 +451,7 @@ template <typename T>
 int launch_wide_tanh(const void* x, const void* w, const void* bias, void* out, int64_t groups, int64_t in_features,
                      int64_t out_features, int64_t rows, hipStream_t stream) {
   return launch_op<T, kGgFwd>(GgArgs{w, x, out, const_cast<void*>(bias), rows, static_cast<int>(groups),
-                                     static_cast<int>(out_features), static_cast<int>(in_features), 0}, stream);
+                                     static_cast<int>(out_features), static_cast<int>(in_features)}, stream);
 }
 
 #define PMSST_GG(T)                                                                                                  \

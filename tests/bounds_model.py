@@ -73,18 +73,18 @@ def cdiv(a: int, b: int) -> int:
 # ----------------------------------------------------------------------------- device helpers
 
 
-def swz_k(r):  # dma_gemm.h
+def swz_k(r):  # gemm.h
     return -(r >> 2) & 3
 
 
-def swz_mn_p(pitch: int, k):  # dma_gemm.h swz_mn_p<PITCH>
+def swz_mn_p(pitch: int, k):  # gemm.h swz_mn_p<PITCH>
     assert pitch % 128 == 0
     if pitch % 256 == 0:
         return 2 * ((k & 3) | (((k >> 3) & 1) << 2))
     return 2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1))
 
 
-def frag_mn_addr(region, c0, pitch, lane):  # dma_gemm.h frag_mn_addr_p
+def frag_mn_addr(region, c0, pitch, lane):  # gemm.h frag_mn_addr_p
     j, g = lane & 15, lane >> 4
     k = 8 * g + (j >> 2)
     col = c0 + 4 * (j & 3)
@@ -287,8 +287,64 @@ def mn_loader(bnd, buf, esz, base_el, kstride, mn_valid, k_valid, rows, v4, kbeg
                     bnd.touch(buf, np.where(ok, base_el + kc * kstride + mn + j, base_el) * esz, esz)
 
 
-def gemm_lds_bytes(esz, br, bc):
+SPLIT_ROW = 48  # gemm.h kSplitRow: LDS floats per tile row of a split fp32 tile
+
+
+def gemm_lds_bytes(esz, br, bc, split=False):  # gemm.h gemm_lds_elems
+    if split:
+        return (br + bc) * SPLIT_ROW * 4
     return 2 * (br + bc) * (LDS_PITCH16 if esz == 2 else LDS_PITCH32) * esz
+
+
+CUS = 256                 # num_cus() of the device the dispatch rules are replayed for
+SPLIT_MACS = 300_000_000  # gemm.h kSplitMacs
+
+
+def split_macs(rows, in_features, out_features):  # gemm.h
+    return rows * in_features >= cdiv(SPLIT_MACS, out_features)
+
+
+def split_dw(widths, M, O, norm):  # band_split.hip
+    otiles = cdiv(O, 64 if norm else 128)
+    return split_macs(M, sum(widths), O) and sum(cdiv(w, 64) for w in widths) * otiles >= CUS
+
+
+def split_tile_lds(bnd, br, bc, wr_n, tr_a, tr_b):
+    """gemm.h gemm_f32_loop on one block's LDS tile: operand A's planes, then B's; the commits (rows, or
+    the K-rows of an MNLoader where ``tr``), the fragment reads of WR x WC waves, and the fp32 tile of a
+    second run in the same place.  Each operand has its region, which no access may leave."""
+    tid = np.arange(GEMM_THREADS)
+    lane, wave = tid & 63, tid >> 6
+    wc_n = 4 // wr_n
+    split_offset = lambda r, k: r * 64 + 16 * ((k >> 3) ^ swz_k(r & 15)) + 2 * (k & 7)  # noqa: E731
+    for name, rows, first, tiles, tr in (("lds_split_a", br, (wave // wc_n) * (br // wr_n), br // wr_n // 16, tr_a),
+                                         ("lds_split_b", bc, (wave % wc_n) * (bc // wc_n), bc // wc_n // 16, tr_b)):
+        bnd.sizes[name] = rows * SPLIT_ROW * 4
+        if tr:
+            mn, kb = (tid % (rows // 4)) * 4, (tid // (rows // 4)) * (rows // 32)
+            if np.any(kb + rows // 32 > CHUNK_K):
+                bnd.fail("split tile: a K-row past the chunk")
+        else:
+            r, k = krow_rows(tid, rows), (tid[:, None] % 8) * 4
+        for plane in range(3):
+            at = plane * rows * 64
+            if tr:
+                for t in range(rows // 32):
+                    bnd.touch(name, at + (kb + t) * 2 * rows + 16 * ((mn >> 3) ^ swz_mn_p(2 * rows, kb + t)) + 2 * (mn & 7), 8)
+            else:
+                bnd.touch(name, at + split_offset(r, k), 8)
+            for t in range(tiles):
+                if tr:
+                    a = np.array([frag_mn_addr(0, int(f) + 16 * t, 2 * rows, int(l)) for f, l in zip(first, lane)])
+                    if np.any(a % (2 * rows) + 8 > 2 * rows):
+                        bnd.fail("split tile: a transposed read leaves its K-row")
+                    bnd.touch(name, at + a, 8)
+                    bnd.touch(name, at + a + 4 * 2 * rows, 8)
+                else:
+                    bnd.touch(name, at + split_offset(first + 16 * t + (lane & 15), 8 * (lane >> 4)), 16)
+        for t in range(tiles):  # the second run: rows of LDS_PITCH32 floats
+            bnd.touch(name, ((first + 16 * t + (lane & 15)) * LDS_PITCH32 + (lane >> 4) + CHUNK_K - 4) * 4, 4)
+        bnd.touch(name, ((rows - 1) * LDS_PITCH32 + CHUNK_K - 4) * 4, 16)
 
 
 # ----------------------------------------------------------------------------- band split
@@ -303,8 +359,12 @@ def tile_capacity(o):
 
 
 def replay_band_split_forward(widths, M, O, esz, *, norm=True, x_stride=None, has_bias=True, act_tanh=False):
-    """band_split.hip launch_fwd + bs_fwd_kernel (also the grouped linear forward when norm=False)."""
+    """band_split.hip launch_fwd + bs_fwd_kernel (also the grouped linear forward when norm=False, whose
+    16-bit tanh form runs grouped_gemm.hip where it is supported)."""
     nb, F = len(widths), int(sum(widths))
+    if act_tanh and has_bias and not norm and len(set(widths)) == 1 and x_stride in (None, F) \
+            and wide_tanh_supported(nb, widths[0], O, M, esz):
+        return replay_gg("fwd", nb, widths[0], O, M)
     x_stride = F if x_stride is None else x_stride
     offs = _offs(widths)
     sizes = {"x": ((M - 1) * x_stride + F) * esz, "gamma": F * esz, "weight": O * F * esz,
@@ -317,7 +377,10 @@ def replay_band_split_forward(widths, M, O, esz, *, norm=True, x_stride=None, ha
     TO = tile_capacity(O) if vec4 else 4
     OT = 64 * TO
     cap = 64 * tile_capacity(O)
-    sizes["lds"] = gemm_lds_bytes(esz, OT, 64) + 64 * 4
+    split = esz == 4 and split_macs(M if vec4 else M // 2, F, O)
+    sizes["lds"] = gemm_lds_bytes(esz, OT, 64, split) + 64 * 4
+    if split:
+        split_tile_lds(bnd, OT, 64, 4, False, False)
     mtiles, oz = cdiv(M, 64), cdiv(O, cap)
     tid = np.arange(GEMM_THREADS)
     lane, wave = tid & 63, tid >> 6
@@ -406,36 +469,52 @@ def replay_band_split_backward(widths, M, O, esz, *, has_bias=True, grouped=Fals
     tid = np.arange(GEMM_THREADS)
     lane, wave = tid & 63, tid >> 6
     norm = not grouped
-    # -- dx of the grouped linear on grouped_dx.hip (16-bit, uniform supported widths)
-    if grouped and esz == 2 and M > 0 and len(set(widths)) == 1 and widths[0] in GDX_TILES and O % 32 == 0 \
-            and O >= 64:
+    uniform = grouped and len(set(widths)) == 1 and not even_dx  # even_dx: the mixed band split's g
+    # -- dx of the grouped linear on grouped_gemm.hip or grouped_dx.hip (16-bit, uniform supported widths)
+    if uniform and wide_dx_supported(nb, widths[0], O, M, esz):
+        replay_gg("dx", nb, widths[0], O, M, bnd=bnd)
+        M_dx = 0
+    elif uniform and esz == 2 and M > 0 and widths[0] in GDX_TILES and O % 32 == 0 and O >= 64:
         _replay_glin_dx(bnd, nb, widths[0], O, M)
         M_dx = 0  # the register-path dx kernel below does not run
     else:
         M_dx = M
-    # -- dx (one block per (band, 64-wide input chunk, 64 rows))
+    # -- dx (one block per (band, 64-wide input chunk, BM rows): 64, 128 in the split grouped linear and in
+    # the mixed band split's g on large grids)
     max_ich = cdiv(max(widths), 64)
-    sizes["lds"] = gemm_lds_bytes(esz, 64, 64) + 64 * 4 + 4 * 64 * 4
+    v4 = vec4 and ovec4
+    split_dx = esz == 4 and v4 and split_macs(M, F, O)
+    BM = 64
+    if grouped and not even_dx:
+        split_dx = split_dx and M > 64 and 5 * nb * max_ich * cdiv(M, 128) >= 6 * CUS
+        BM = 128 if split_dx else 64
+    elif even_dx and cdiv(M, 64) * sum(cdiv(w, 64) for w in widths) >= 2 * 7 * CUS:
+        BM = 128
+    WR = 4 if BM == 64 else 2
+    WC = 4 // WR
+    dx_tiles = cdiv(M, BM)
+    sizes["lds"] = gemm_lds_bytes(esz, 64, BM, split_dx) + BM * 4 + 4 * BM * 4
+    if M_dx > 0 and split_dx:
+        split_tile_lds(bnd, 64, BM, WR, True, False)
     if M_dx > 0:
         # norm: the even schedule over the existing (band, row tile, chunk) blocks (the XcdGrid of
         # NB * max_ichunks groups past 256 bands); grouped: the XcdGrid (all groups one width)
-        sc = build_even_sched(nb, m_tiles, lambda b: cdiv(widths[b], 64)) if norm or even_dx else None
+        sc = build_even_sched(nb, dx_tiles, lambda b: cdiv(widths[b], 64)) if norm or even_dx else None
         if sc is not None:
             sched_decode(sc, nb, lambda b: cdiv(widths[b], 64), True, bnd, "bs_bwd_dx")
         else:
-            grp, mt, valid = xcd_decode(nb * max_ich, m_tiles)
-            if np.any(mt[valid] >= m_tiles):
+            grp, mt, valid = xcd_decode(nb * max_ich, dx_tiles)
+            if np.any(mt[valid] >= dx_tiles):
                 bnd.fail("dx: member out of range")
-        v4 = vec4 and ovec4
         for band in range(nb):
             off, I = int(offs[band]), int(widths[band])
             for ich in range(max_ich):
                 i0 = ich * 64
                 if i0 >= I:
                     continue
-                for mtile in sorted({0, m_tiles - 1}):
-                    m0 = mtile * 64
-                    rv = min(M - m0, 64)
+                for mtile in sorted({0, dx_tiles - 1}):
+                    m0 = mtile * BM
+                    rv = min(M - m0, BM)
                     r64 = np.arange(64)
                     if norm:
                         bnd.touch("inv_norm", ((m0 + r64) * nb + band) * 4, 4, r64 < rv)
@@ -444,34 +523,35 @@ def replay_band_split_backward(widths, M, O, esz, *, has_bias=True, grouped=Fals
                     nk = cdiv(O, CHUNK_K)
                     kbeg = O - nk * CHUNK_K
                     mn_loader(bnd, "weight", esz, O * off + i0, I, I - i0, O, 64, v4, kbeg, nk, tid)
-                    krow_loader(bnd, "dy", esz, (m0 * nb + band) * O, nb * O, rv, O, 64, v4, kbeg, nk, tid)
-                    il = i0 + wave * 16 + 4 * (lane >> 4)
-                    for j in range(4):
-                        m = j * 16 + (lane & 15)
-                        ok = (m < rv) & (il < I)
+                    krow_loader(bnd, "dy", esz, (m0 * nb + band) * O, nb * O, rv, O, BM, v4, kbeg, nk, tid)
+                    for it in range(64 // WR // 16):
+                        il = i0 + (wave // WC) * (64 // WR) + 16 * it + 4 * (lane >> 4)
+                        for j in range(BM // WC // 16):
+                            m = (wave % WC) * (BM // WC) + j * 16 + (lane & 15)
+                            ok = (m < rv) & (il < I)
+                            if norm:
+                                for r in range(4):
+                                    gi = np.where(il + r < I, off + il + r, off)
+                                    bnd.touch("gamma", gi * esz, esz, il + r < I)
+                            e = (m0 + m) * F + off + il
+                            if vec4:
+                                if norm:
+                                    bnd.touch("x", e * esz, 4 * esz, ok)
+                                    bnd.touch("workspace", dgp + pdb + e * 4, 16, ok)
+                                else:
+                                    bnd.touch("dx", e * esz, 4 * esz, ok)
+                            else:
+                                for r in range(4):
+                                    okr = ok & (il + r < I)
+                                    if norm:
+                                        bnd.touch("x", (e + r) * esz, esz, okr)
+                                        bnd.touch("workspace", dgp + pdb + (e + r) * 4, 4, okr)
+                                    else:
+                                        bnd.touch("dx", (e + r) * esz, esz, okr)
                         if norm:
                             for r in range(4):
-                                gi = np.where(il + r < I, off + il + r, off)
-                                bnd.touch("gamma", gi * esz, esz, il + r < I)
-                        e = (m0 + m) * F + off + il
-                        if vec4:
-                            if norm:
-                                bnd.touch("x", e * esz, 4 * esz, ok)
-                                bnd.touch("workspace", dgp + pdb + e * 4, 16, ok)
-                            else:
-                                bnd.touch("dx", e * esz, 4 * esz, ok)
-                        else:
-                            for r in range(4):
-                                okr = ok & (il + r < I)
-                                if norm:
-                                    bnd.touch("x", (e + r) * esz, esz, okr)
-                                    bnd.touch("workspace", dgp + pdb + (e + r) * 4, 4, okr)
-                                else:
-                                    bnd.touch("dx", (e + r) * esz, esz, okr)
-                    if norm:
-                        for r in range(4):
-                            bnd.touch("workspace", (mtile * F + off + il + r) * 4, 4,
-                                      ((lane & 15) == 0) & (il + r < I))
+                                bnd.touch("workspace", (mtile * F + off + il + r) * 4, 4,
+                                          ((lane & 15) == 0) & (il + r < I))
         # -- finish: the dx kernel's blocks (band, 64-wide chunk, 64 rows); with the DMA dW kernel and the
         # dx schedule they are that kernel's tail blocks, decoded at blockIdx.x minus its scheduled
         # blocks (a multiple of 8): the same decode and addresses
@@ -521,6 +601,8 @@ def replay_band_split_backward(widths, M, O, esz, *, has_bias=True, grouped=Fals
         and O % 8 == 0
     if dma:
         _replay_bs_dw_dma(bnd, widths, offs, M, O, esz, has_bias)
+    elif uniform and wide_dw_supported(nb, widths[0], O, M, esz):
+        replay_gg("dw", nb, widths[0], O, M, bnd=bnd, has_bias=has_bias)
     elif uniform_dw:  # the mask-estimator DMA dW kernel with HT = 64 on bands of width 2 I_b = O
         _replay_me_dw_dma(bnd, [O // 2] * nb, _offs([O // 2] * nb), M, widths[0], esz, 64, "dy", "x", "dw",
                           "db" if has_bias else None, "lds_dw", JT=dw_jt(nb, widths[0], O))
@@ -669,6 +751,149 @@ def replay_band_split_mixed(widths, M, O, *, x_stride=None):
     # g = T(dy W) on the norm-free dx kernel (dx = g here, x = the features) and dW / dbias on the DMA dW
     # kernel, or where that does not fit on the norm-free register dW kernel
     yield "band_split_mixed_bwd_gemm", replay_band_split_backward(widths, M, O, 2, grouped=True, even_dx=True)
+
+
+# ----------------------------------------------------------------------------- grouped_gemm.hip
+
+
+def _gg_shape_ok(groups, I, O, rows, esz):  # shape_ok (aligned pointers)
+    return (esz == 2 and rows > 0 and groups <= 256 and I % 8 == 0 and O % 8 == 0
+            and 256 * groups * O * 2 < 1 << 31 and 256 * groups * I * 2 < 1 << 31)
+
+
+def wide_dx_supported(groups, I, O, rows, esz):
+    if not _gg_shape_ok(groups, I, O, rows, esz) or O % 32:
+        return False
+    if I > 256:
+        return groups * rows * I >= (11 if groups >= 24 else 16) * 1024 * CUS
+    blocks = groups * cdiv(rows, 256)
+    return I in (192, 256) and 5 * blocks >= 4 * cdiv(blocks, CUS) * CUS
+
+
+def wide_dw_supported(groups, I, O, rows, esz):
+    if not _gg_shape_ok(groups, I, O, rows, esz) or I < 192 or rows < 32:
+        return False
+    a_cols = 256 if I % 256 == 0 else 192
+    rounds = cdiv(groups * cdiv(O, 256) * cdiv(I, a_cols), CUS)
+    if I % 64 == 0:
+        other = cdiv(groups, XCDS) * (I // 64) * cdiv(O, 128) * XCDS
+        if a_cols == 256:
+            return other >= 6 * rounds * CUS and rows >= 64
+        return (other >= 6 * rounds * CUS and rows > 128) or (2 * other >= 9 * rounds * CUS and rows >= 1400)
+    other = groups * cdiv(I, 64) * cdiv(O, 64)
+    return other >= 5 * rounds * CUS and rows * other >= 2000 * rounds * CUS
+
+
+def wide_tanh_supported(groups, I, O, rows, esz):
+    return O >= 128 and _gg_shape_ok(groups, I, O, rows, esz) and I % 32 == 0 and 256 * I * 2 < 1 << 31
+
+
+def gg_tile(op, I, O):
+    """launch_op / gg_kernel: (waves, stages, TA, A columns, B rows) of an operation."""
+    nw = 4 if op == "fwd" else 8
+    ta = 8 if (O if op == "fwd" else I) % 256 == 0 else 6
+    return nw, 4 if nw == 8 else 3, ta, 32 * ta, 16 * 4 * nw // 2
+
+
+def replay_gg(op, G, I, O, M, *, bnd=None, has_bias=True, names=None):
+    """grouped_gemm.hip gg_kernel: ``op`` "fwd" (h = tanh(x W^T + b)), "dx" (dy W) or "dw" (dy^T x, db).  The
+    DMA pieces of both operands (columns and rows past the tile clamped, dW's K rows before row 0 read
+    from row 0), the fragment reads inside a stage, the bias, db and the result staged through LDS."""
+    if bnd is None:
+        bnd = Bounds({"x": M * G * I * 2, "weight": G * O * I * 2, "bias": G * O * 2, "out": M * G * O * 2})
+    names = names or {}
+    a_buf, b_buf, d_buf = {"fwd": ("weight", "x", "out"), "dx": ("weight", "dy", "dx"), "dw": ("x", "dy", "dw")}[op]
+    a_buf, b_buf, d_buf = (names.get(n, n) for n in (a_buf, b_buf, d_buf))
+    bias_buf = names.get("bias", "bias")
+    NW, S, TA, AR, BR = gg_tile(op, I, O)
+    WA, TB = 2, 4
+    kA = AR * 64
+    kStage = kA + BR * 64
+    kPA, kPT = kA // 1024, kStage // 1024
+    PW = cdiv(kPT, NW)
+    kOP = AR + 8
+    lds = f"lds_gg_{op}"
+    bnd.sizes[lds] = max(S * kStage, BR * kOP * 2)
+    bnd.sizes[lds + "_a"], bnd.sizes[lds + "_b"] = kA, BR * 64
+    if bnd.sizes[lds] > 160 * 1024:
+        bnd.fail("gg: more than 160 KB of LDS")
+    K = {"dx": O, "dw": M, "fwd": I}[op]
+    nk = cdiv(K, 32)
+    kbeg = K - 32 * nk
+    if op != "dw" and kbeg:
+        bnd.fail("gg: a partial K chunk where only dW has one")
+    a_all, b_all = (O if op == "fwd" else I), (O if op == "dw" else M)
+    a_tiles, b_tiles = cdiv(a_all, AR), cdiv(b_all, BR)
+    units = lambda b: a_tiles  # noqa: E731
+    sc = build_even_sched(G, b_tiles, units)
+    decoded = sched_decode(sc, G, units, False, bnd, "gg")
+    lane = np.arange(64)
+    gq, rr = lane >> 4, lane & 15
+    dyrow, xrow = G * O, G * I
+    astride = xrow if op == "dw" else I
+    bstride = xrow if op == "fwd" else dyrow
+    a_kc, b_kc = op == "fwd", op != "dw"
+    for g, tb, ta in sorted({(b, m, u) for b, m, u in decoded if b in (0, G - 1) and m in (0, b_tiles - 1)}):
+        a0, b0 = ta * AR, tb * BR
+        av, bv = min(a_all - a0, AR), min(b_all - b0, BR)
+        abase = {"dx": g * O * I + a0, "dw": g * I + a0, "fwd": g * O * I + a0 * I}[op]
+        bbase = g * (I if op == "fwd" else O) + (b0 if op == "dw" else b0 * bstride)
+        for wave in range(NW):
+            for q in range(PW):
+                k = wave + NW * q
+                k = k if k < kPT else wave
+                isa = k < kPA
+                kc, stride, valid = (a_kc, astride, av) if isa else (b_kc, bstride, bv)
+                cols = AR if isa else BR
+                if not kc:
+                    U = 64 * (k if isa else k - kPA) + lane
+                    kr = U // (cols // 8)
+                    u = (U % (cols // 8)) ^ swz_mn_p(2 * cols, kr)
+                    if np.any(u >= cols // 8) or np.any(kr >= 32):
+                        bnd.fail("gg: a swizzled unit leaves its K-row")
+                    off = kr * stride + np.where(8 * u < valid, 8 * u, valid - 8)
+                else:
+                    r = 16 * (k if isa else k - kPA) + (lane >> 2)
+                    kr = np.zeros(64, dtype=np.int64)
+                    off = np.minimum(r, valid - 1) * stride + 8 * ((lane & 3) ^ swz_k(lane >> 2))
+                if np.any(2 * off >= 1 << 32):
+                    bnd.fail("gg: 32-bit DMA offset overflows")
+                base = abase if isa else bbase
+                for c in steps(nk):
+                    if op == "dw":
+                        row0 = kbeg + 32 * c
+                        over = np.where((c == 0) & (kbeg + kr < 0), -(kbeg + kr), 0)
+                        at = base + row0 * stride + off + over * stride
+                    else:
+                        at = base + off + (32 * c if kc else 32 * c * stride)
+                    bnd.touch(a_buf if isa else b_buf, at * 2, 16)
+                    bnd.touch(lds, (c % S) * kStage + k * 1024 + lane * 16, 16)
+                bnd.touch(lds, (S - 1) * kStage + k * 1024 + lane * 16, 16)
+            wa, wb = wave % WA, wave // WA
+            for name, tiles, first, kc, cols in ((lds + "_a", TA, TA * wa, a_kc, AR), (lds + "_b", TB, TB * wb, b_kc, BR)):
+                for t in range(tiles):
+                    if kc:
+                        bnd.touch(name, frag_k_addr(0, 16 * (first + t), lane), 16)
+                    else:
+                        f = frag_mn_addr(0, 16 * (first + t), 2 * cols, lane)
+                        bnd.touch(name, f, 8)
+                        bnd.touch(name, f + 4 * 2 * cols, 8)
+                    if op == "fwd" and name.endswith("_a"):
+                        o = 16 * (first + t) + 4 * gq
+                        bnd.touch(bias_buf, (g * O + a0 + np.where(o < av, o, av - 4)) * 2, 8)
+            for j in range(TB):
+                r = 16 * (TB * wb + j) + rr
+                if op == "dw" and has_bias and ta == 0 and wa == 0:
+                    bnd.touch("db", (g * O + b0 + r) * 2, 2, (lane < 16) & (r < bv))
+                for i in range(TA):
+                    bnd.touch(lds, (r * kOP + 16 * (TA * wa + i) + 4 * gq) * 2, 8)
+        q = np.arange(BR * (AR // 8))
+        r, u = q // (AR // 8), q % (AR // 8)
+        ok = (r < bv) & (u < av // 8)
+        drow, d0 = {"dx": (xrow, g * I), "dw": (I, g * O * I), "fwd": (dyrow, g * O)}[op]
+        bnd.touch(lds, (r * kOP + 8 * u) * 2, 16, ok)
+        bnd.touch(d_buf, (d0 + (b0 + r) * drow + a0 + 8 * u) * 2, 16, ok)
+    return bnd
 
 
 GDX_TILES = {64: (4, 4, 4), 128: (8, 4, 4), 192: (12, 2, 4), 256: (16, 2, 4)}  # grouped_dx.hip launch_grouped_dx: DT, NT, stages
@@ -869,12 +1094,17 @@ def _replay_bs_dw_dma(bnd, widths, offs, M, O, esz, has_bias):
 
 
 def _replay_bs_dw_reg(bnd, widths, offs, M, O, esz, has_bias, norm, v4):
-    """band_split.hip bs_bwd_dw_kernel (register-staged main loop; also the grouped linear's dW)."""
+    """band_split.hip bs_bwd_dw_kernel (register-staged main loop; also the grouped linear's dW): 64-wide
+    output tiles, 128 in the split grouped linear."""
     nb, F = len(widths), int(sum(widths))
     max_it = cdiv(max(widths), 64)
+    split = esz == 4 and v4 and split_dw(widths, M, O, norm)
+    BO = 128 if split and not norm else 64
+    if split:
+        split_tile_lds(bnd, 64, BO, 2, True, True)
     # the even schedule over the existing (band, input tile, output tile) blocks (sub = input tile x
     # output tiles + output tile); the XcdGrid past 256 bands
-    otiles = cdiv(O, 64)
+    otiles = cdiv(O, BO)
     units = lambda b: cdiv(widths[b], 64) * otiles
     sc = build_even_sched(nb, 1, units)
     if sc is not None:
@@ -887,24 +1117,24 @@ def _replay_bs_dw_reg(bnd, widths, offs, M, O, esz, has_bias, norm, v4):
     lane, wave = tid & 63, tid >> 6
     nk = cdiv(M, CHUNK_K)
     kbeg = M - nk * CHUNK_K
-    bnd.sizes["lds"] = max(bnd.sizes["lds"], gemm_lds_bytes(esz, 64, 64))
+    bnd.sizes["lds"] = max(bnd.sizes["lds"], gemm_lds_bytes(esz, 64, BO, split))
     for g_, o_ in blocks:
         band, i0 = int(g_) // max_it, (int(g_) % max_it) * 64
-        o0 = int(o_) * 64
+        o0 = int(o_) * BO
         off, I = int(offs[band]), int(widths[band])
         if i0 >= I or M == 0:
             continue
         mn_loader(bnd, "x", esz, off + i0, F, I - i0, M, 64, v4, kbeg, nk, tid)
         if norm:
             bnd.touch("inv_norm", (np.arange(M) * nb + band) * 4, 4)
-        mn_loader(bnd, "dy", esz, band * O + o0, nb * O, O - o0, M, 64, v4, kbeg, nk, tid)
+        mn_loader(bnd, "dy", esz, band * O + o0, nb * O, O - o0, M, BO, v4, kbeg, nk, tid)
         if has_bias and i0 == 0:
             t64 = np.arange(GEMM_THREADS)
-            bnd.touch("db", (band * O + o0 + t64) * esz, esz, (t64 < 64) & (t64 < O - o0))
-        ir, oc = (wave >> 1) * 32, (wave & 1) * 32
+            bnd.touch("db", (band * O + o0 + t64) * esz, esz, (t64 < BO) & (t64 < O - o0))
+        ir, oc = (wave >> 1) * 32, (wave & 1) * (BO // 2)
         for u in range(2):
             i = i0 + ir + u * 16 + 4 * (lane >> 4)
-            for v in range(2):
+            for v in range(BO // 32):
                 o = o0 + oc + v * 16 + (lane & 15)
                 ok = (i < I) & (o < O)
                 if v4:
@@ -917,13 +1147,17 @@ def _replay_bs_dw_reg(bnd, widths, offs, M, O, esz, has_bias, norm, v4):
 # ----------------------------------------------------------------------------- mask estimator
 
 
-def replay_mask_final_forward(widths, M, H, esz):
-    """mask_estimator.hip launch_me_fwd: me_fwd_dma_kernel on the band schedule (16-bit, aligned), else
-    me_fwd_kernel."""
+def replay_mask_final_forward(widths, M, H, esz, *, apply=None):
+    """mask_estimator.hip launch_me_fwd: me_fwd_dma_kernel on the band schedule (16-bit, aligned; with
+    ``apply`` the masked spectrum in the place of ``out``), else me_fwd_kernel."""
     nb, F = len(widths), int(sum(widths))
     offs = _offs(widths)
     sizes = {"x": M * nb * H * esz, "weight": 2 * F * H * esz, "bias": 2 * F * esz, "pre": M * 2 * F * esz,
              "out": M * F * esz, "offsets": (nb + 1) * 8, "lds": 4 * 16384}
+    if apply is not None:
+        bsz = M // apply["frames"]
+        sizes["spec"] = bsz * (F // 2) * apply["frames"] * 8
+        sizes["est"] = bsz * apply["stems"] * (F // 2) * apply["frames"] * 8
     bnd = Bounds(sizes)
     vec4 = all(w % 4 == 0 for w in widths) and H % 4 == 0
     mtiles = cdiv(M, 128)
@@ -989,13 +1223,24 @@ def replay_mask_final_forward(widths, M, H, esz):
                 m = 64 * wc + 16 * j + rr
                 for base in (0, 128 * kop, 2 * 128 * kop):
                     bnd.touch("lds", (base + m * kop + lt) * esz, 4 * esz, active)
+                if apply is not None:
+                    fr, ch, ns, st = apply["frames"], apply["channels"], apply["stems"], apply["stem"]
+                    fbins = F // (2 * ch)
+                    ok = okl & (m < rv)
+                    bb, tt = (m0 + m) // fr, (m0 + m) % fr
+                    for q in range(2):
+                        r = (off + l) // 2 + q
+                        f, c = r // ch, r % ch
+                        bnd.touch("spec", ((bb * fbins * ch + r) * fr + tt) * 8, 8, ok)
+                        bnd.touch("est", ((((bb * ns + st) * ch + c) * fbins + f) * fr + tt) * 8, 8, ok)
         c4 = (tid & 15) * 4
         for p in range(8):
             m = (tid >> 4) + 16 * p
             ok = (l0 + c4 < I) & (m < rv)
             bnd.touch("pre", ((m0 + m) * 2 * F + 2 * off + l0 + c4) * esz, 8, ok)
             bnd.touch("pre", ((m0 + m) * 2 * F + 2 * off + l0 + c4 + I) * esz, 8, ok)
-            bnd.touch("out", ((m0 + m) * F + off + l0 + c4) * esz, 8, ok)
+            if apply is None:
+                bnd.touch("out", ((m0 + m) * F + off + l0 + c4) * esz, 8, ok)
     bnd.touch("offsets", np.arange(nb + 1) * 8, 8)
     return bnd
 
@@ -1315,6 +1560,24 @@ def mlp_row_tile(M, NT, WV):
     return full
 
 
+def two_kernels_better(rows, dim, widths):
+    """mask_mlp.hip: whether the forward with the hidden layer stored runs a hidden and a final kernel."""
+    if dim >= 384:
+        return True
+    return sum(cdiv(w, 64) for w in widths) > 2 * len(widths) and (dim >= 256 or rows > (768 if dim <= 64 else 256))
+
+
+def replay_mask_mlp_saved(widths, M, D, H, esz, *, apply=None):
+    """mask_mlp.hip mask_mlp_forward_impl with the hidden layer stored: yields (label, Bounds) of the one
+    pass, or of the hidden layer (grouped_gemm.hip) and the final layer (mask_estimator.hip)."""
+    tag = "_apply" if apply else ""
+    if not (two_kernels_better(M, D, widths) and wide_tanh_supported(len(widths), D, H, M, esz) and H % 8 == 0 and H > 32):
+        yield "mask_mlp_fwd" + tag, replay_mask_mlp_forward(widths, M, D, H, esz, apply=apply)
+        return
+    yield "mask_mlp_fwd_hidden" + tag, replay_gg("fwd", len(widths), D, H, M)
+    yield "mask_mlp_fwd_final" + tag, replay_mask_final_forward(widths, M, H, esz, apply=apply)
+
+
 def replay_mask_mlp_forward(widths, M, D, H, esz, *, write_h=True, wv=None, apply=None, rb=None):
     """mask_mlp.hip mlp_fwd_kernel (whole depth-2 mask MLP, 16-bit) on its band schedule: the b1 fill,
     the x fragments, the W1 / W2 DMA ring, the LDS fragment reads, the hidden stores and the GLU
@@ -1479,7 +1742,10 @@ def _replay_me_fwd_reg(bnd, widths, offs, M, H, esz, vec4):
     nb, F = len(widths), int(sum(widths))
     max_l = cdiv(max(widths), 64)
     mtiles = cdiv(M, 128)
-    bnd.sizes["lds"] = gemm_lds_bytes(esz, 128, 128)
+    split = esz == 4 and split_macs(M, 2 * F, H)
+    bnd.sizes["lds"] = gemm_lds_bytes(esz, 128, 128, split)
+    if split:
+        split_tile_lds(bnd, 128, 128, 1, False, False)
     tid = np.arange(GEMM_THREADS)
     lane, wave = tid & 63, tid >> 6
     nk = cdiv(H, CHUNK_K)
@@ -1530,7 +1796,10 @@ def _replay_me_dx_reg(bnd, widths, offs, M, H, esz, tanh_in):
     hch = cdiv(H, 128)
     mtiles = cdiv(M, 64)
     grp, mt, valid = xcd_decode(nb * hch, mtiles)
-    bnd.sizes["lds"] = max(bnd.sizes["lds"], gemm_lds_bytes(esz, 128, 64))
+    split = esz == 4 and split_macs(M, 2 * F, H)
+    bnd.sizes["lds"] = max(bnd.sizes["lds"], gemm_lds_bytes(esz, 128, 64, split))
+    if split:
+        split_tile_lds(bnd, 128, 64, 2, True, False)
     tid = np.arange(GEMM_THREADS)
     lane, wave = tid & 63, tid >> 6
     v4 = True
@@ -1563,6 +1832,8 @@ def _replay_me_dw_reg(bnd, widths, offs, M, H, esz):
     nb, F = len(widths), int(sum(widths))
     ht = cdiv(H, 128)
     maxj = cdiv(2 * max(widths), 64)
+    if esz == 4 and split_macs(M, 2 * F, H):
+        split_tile_lds(bnd, 128, 64, 2, True, True)
     tid = np.arange(GEMM_THREADS)
     lane, wave = tid & 63, tid >> 6
     nk = cdiv(M, CHUNK_K)
@@ -1715,8 +1986,118 @@ def replay_rotary_qkv(B: int, N: int, H: int, D: int, esz: int, backward: bool):
     return bnd
 
 
+def _replay_gate_mfma_fwd(bnd, rows, N, H, E, dim, strides):
+    """attn_gate.hip gate_mfma_fwd_kernel: 16 tokens a wave, W as A fragments in LDS, the gates by token."""
+    sb, sn, sh = strides
+    KS = dim // 32
+    bnd.sizes.update({"lds_w": KS * 1024, "lds_gates": 4 * 16 * 17 * 4})
+    lane = np.arange(64)
+    gq, rr = lane >> 4, lane & 15
+    lph = WAVE // H
+    head, sub = lane // lph, lane % lph
+    q = np.arange(KS * 64)
+    h = q & 15
+    bnd.touch("weight", (h * dim + 32 * (q >> 6) + 8 * ((q & 63) >> 4)) * 2, 16, h < H)
+    bnd.touch("lds_w", q * 16, 16)
+    blocks = cdiv(rows, 64)
+    for blk in sorted({0, blocks - 1}):
+        for wave in range(4):
+            m0 = (blk * 4 + wave) * 16
+            if m0 >= rows:
+                continue
+            mx = np.minimum(m0 + rr, rows - 1)
+            for k in range(KS):
+                bnd.touch("x", (mx * dim + 32 * k + 8 * gq) * 2, 16)
+                bnd.touch("lds_w", k * 1024 + lane * 16, 16)
+            for r in range(4):
+                h = 4 * gq + r
+                bnd.touch("bias", h * 2, 2, h < H)
+                bnd.touch("lds_gates", ((wave * 16 + rr) * 17 + h) * 4, 4)
+                bnd.touch("gate", ((m0 + rr) * H + h) * 2, 2, (h < H) & (m0 + rr < rows))
+            for t in range(16):
+                m = min(m0 + t, rows - 1)
+                bnd.touch("attn", ((m // N) * sb + (m % N) * sn + head * sh + sub * E) * 2, 2 * E)
+                bnd.touch("lds_gates", ((wave * 16 + t) * 17 + head) * 4, 4)
+                if m0 + t < rows:
+                    bnd.touch("out", ((m0 + t) * 64 * E + lane * E) * 2, 2 * E)
+
+
+def _replay_gate_mfma_bwd(bnd, rows, N, H, E, dim, strides, ws_gpre, ws_pw):
+    """attn_gate.hip gate_mfma_bwd_kernel: 32-token groups in equal turns, the x tile by DMA into two
+    buffers, gpre by token and by head in LDS; returns the number of partials."""
+    sb, sn, sh = strides
+    NT = dim // 64
+    pitch = 2 * dim
+    tile = 32 * pitch
+    bnd.sizes.update({"lds_x": 2 * tile, "lds_tok": 2 * 32 * 16 * 2, "lds_head": 2 * 16 * 32 * 2, "lds_red": 4 * 16 * 4})
+    if 2 * tile + 2 * 2048 + 256 > 160 * 1024:
+        bnd.fail("gate: more than 160 KB of LDS")
+    lane = np.arange(64)
+    gq, rr = lane >> 4, lane & 15
+    lph = WAVE // H
+    head, sub = lane // lph, lane % lph
+    groups = cdiv(rows, 32)
+    slots = min(2 * CUS, 1024)
+    turns = cdiv(groups, slots)
+    parts = cdiv(groups, turns)
+    if parts > slots:
+        bnd.fail("gate: more blocks than slots")
+    for blk in sorted({0, parts - 1, (groups - 1) % parts}):
+        mine = list(range(blk, groups, parts))
+        for it, grp in ((i, g) for i, g in enumerate(mine) if i in (0, 1, len(mine) - 1)):
+            buf = it & 1
+            for wave in range(4):
+                for q in range(NT):
+                    p = wave + 4 * q
+                    U = 64 * p + lane
+                    kr = U // (dim // 8)
+                    u = (U % (dim // 8)) ^ swz_mn_p(pitch, kr)
+                    if np.any(u >= dim // 8) or np.any(kr >= 32):
+                        bnd.fail("gate: a swizzled unit leaves its row")
+                    m = np.minimum(grp * 32 + kr, rows - 1)
+                    bnd.touch("x", (m * dim + 8 * u) * 2, 16)
+                    bnd.touch("lds_x", buf * tile + p * 1024 + lane * 16, 16)
+                    bnd.touch("lds_x", buf * tile + U * 16, 16)
+                for t in range(8):
+                    tok = wave * 8 + t
+                    m = min(grp * 32 + tok, rows - 1)
+                    at = (m // N) * sb + (m % N) * sn + head * sh + sub * E
+                    bnd.touch("grad_out", (m * 64 * E + lane * E) * 2, 2 * E)
+                    bnd.touch("attn", at * 2, 2 * E)
+                    bnd.touch("gate", (m * H + head) * 2, 2)
+                    if grp * 32 + tok < rows:
+                        bnd.touch("grad_attn", at * 2, 2 * E)
+                    bnd.touch("lds_tok", ((buf * 32 + tok) * 16 + head) * 2, 2, sub == 0)
+                    bnd.touch("lds_head", ((buf * 16 + head) * 32 + tok) * 2, 2, sub == 0)
+                i0 = 16 * NT * wave
+                for n in range(2):
+                    bnd.touch("lds_tok", ((buf * 32 + 16 * n + rr) * 16 + 8 * gq) * 2, 16, gq < 2)
+                    m = grp * 32 + 16 * n + rr
+                    for t in range(0, NT - 1, 2):
+                        bnd.touch("grad_x", (m * dim + i0 + 16 * t + 8 * gq) * 2, 16, m < rows)
+                    if NT % 2:
+                        bnd.touch("grad_x", (m * dim + i0 + 16 * (NT - 1) + 4 * gq) * 2, 8, m < rows)
+                bnd.touch("lds_head", ((buf * 16 + rr) * 32 + 8 * gq) * 2, 16)
+                for t in range(NT):
+                    f = frag_mn_addr(0, i0 + 16 * t, pitch, lane)
+                    if np.any(f % pitch + 8 > pitch):
+                        bnd.fail("gate: a transposed read leaves its row")
+                    bnd.touch("lds_x", buf * tile + f, 8)
+                    bnd.touch("lds_x", buf * tile + f + 4 * pitch, 8)
+        for wave in range(4):
+            i0 = 16 * NT * wave
+            for t in range(NT):
+                col = np.where(t < NT // 2 * 2, 32 * (t // 2) + 8 * (rr >> 2) + 4 * (t & 1) + (rr & 3), 16 * t + rr)
+                for e in range(8):
+                    bnd.touch("weight", ((8 * gq + e) * dim + i0 + col) * 2, 2, 8 * gq + e < H)
+                bnd.touch("workspace", ws_gpre + (blk * H * dim + rr * dim + i0 + 4 * gq + 16 * t) * 4, 16, rr < H)
+            bnd.touch("lds_red", (wave * 16 + head) * 4, 4, sub == 0)
+        bnd.touch("workspace", ws_gpre + ws_pw + (blk * H + np.arange(H)) * 4, 4)
+    return parts
+
+
 def replay_attention_gate(B: int, N: int, H: int, Dh: int, dim: int, esz: int):
-    """attn_gate.hip gate_fwd_kernel / gate_bwd_kernel (fast path) with attn and grad_attn the
+    """attn_gate.hip gate_fwd_kernel / gate_bwd_kernel (fast path), or the matrix-core kernels, with attn and grad_attn the
     [B, N, H, Dh] views of dense [B, H, N, Dh] SDPA buffers, col_sum of the partials."""
     rows = B * N
     HD = H * Dh
@@ -1749,9 +2130,23 @@ def replay_attention_gate(B: int, N: int, H: int, Dh: int, dim: int, esz: int):
     k = np.arange(H * dim)
     bnd.touch("weight", k * esz, esz)
     bnd.touch("lds", ((k % dim) * H + k // dim) * 4, 4)
+    mfma = set()
+    if esz == 2 and dim % 64 == 0 and dim // 64 in (1, 2, 3, 4, 6, 8):
+        if H * dim >= 4096 or rows >= 16384 or (rows >= 8192 and H * dim >= 1024):  # gate_mfma_fwd_pays
+            _replay_gate_mfma_fwd(bnd, rows, N, H, E, dim, (sb, sn, sh))
+            mfma.add("fwd")
+        if H * dim >= 1536 or (H * dim >= 1024 and rows >= 2000):  # gate_mfma_bwd_pays
+            parts = _replay_gate_mfma_bwd(bnd, rows, N, H, E, dim, (sb, sn, sh), ws_gpre, ws_pw)
+            if parts > parts_ws:
+                bnd.fail("gate: more partials than the workspace holds")
+            _replay_col_sum(bnd, "workspace", parts, H * dim, "grad_weight", esz, poff=ws_gpre)
+            _replay_col_sum(bnd, "workspace", parts, H, "grad_bias", esz, poff=ws_gpre + ws_pw)
+            mfma.add("bwd")
     # the grids: up to 4096 / 1024 blocks, fewer where fewer fit on the device at once (any count works:
     # the loops stride over the grid); both ends are replayed
     for kind, maxb in (("fwd", 4096), ("fwd", 1792), ("bwd", 1024), ("bwd", 768)):
+        if kind in mfma:
+            continue
         nblk = min(cdiv(rows, 4 * 2), maxb)
         for blk in sorted({0, nblk - 1}):
             # a wave's rows: m0 = (block * 4 + wave) * 2 + trip * (grid * 8) while m0 < rows; the
@@ -1835,11 +2230,12 @@ def all_replays(name: str, esz: int):
     yield "mask_final_fwd", replay_mask_final_forward(widths, M, hidden, esz)
     yield "mask_final_bwd", replay_mask_final_backward(widths, M, hidden, esz, tanh_in=True)
     if esz == 2:
-        yield "mask_mlp_fwd", replay_mask_mlp_forward(widths, M, dim, hidden, esz)
+        yield from replay_mask_mlp_saved(widths, M, dim, hidden, esz)
+        yield "mask_mlp_fwd_unsaved", replay_mask_mlp_forward(widths, M, dim, hidden, esz, write_h=False)
         if name in ("configs1", "configs4"):  # BS-RoFormer: stereo, bins x 2 channels x (re, im)
             frames = {"configs1": 258, "configs4": 948}[name]
             stems = {"configs1": 4, "configs4": 1}[name]
-            yield "mask_mlp_fwd_apply", replay_mask_mlp_forward(
+            yield from replay_mask_mlp_saved(
                 widths, M, dim, hidden, esz, apply={"frames": frames, "channels": 2, "stems": stems, "stem": stems - 1})
     yield "rms_norm", replay_rms_norm(M * nb, dim, esz)
     for shape in qk:

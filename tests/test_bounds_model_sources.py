@@ -109,3 +109,53 @@ def test_a_planted_mismatch_is_caught(monkeypatch, mistake):
         monkeypatch.setattr(bm, "CHUNK_K", 64)
         with pytest.raises(AssertionError):
             test_shared_constants()
+
+
+def test_fp32_split_rules_and_tiles():
+    """gemm.h kSplitRow, kSplitMacs, gemm_lds_elems; the launchers' rules in band_split.hip and
+    mask_estimator.hip."""
+    assert _const("kSplitRow", "gemm.h") == bm.SPLIT_ROW
+    m = _one(r"constexpr int64_t kSplitMacs = ([\d']+);", _src("gemm.h"), "kSplitMacs")
+    assert int(m.group(1).replace("'", "")) == bm.SPLIT_MACS
+    _one(r"return SPLIT \? \(BR \+ BC\) \* kSplitRow : 2 \* \(BR \+ BC\) \* LdsPitch<T>::value;", _src("gemm.h"), "LDS")
+    s = _src("band_split.hip")
+    _one(r"constexpr int dw_cols\(bool norm, bool split\) \{ return split && !norm \? 128 : 64; \}", s, "dW columns")
+    _one(r"return split_macs\(M, hb\.F, O\) && blocks >= num_cus\(\);", s, "dW rule")
+    _one(r"if \(split_macs\(a\.vec4 \? M : M / 2, hb\.F, O\)\) launch\(std::true_type\{\}\);", s, "forward rule")
+    _one(r"kF32 && v4 && split_macs\(M, hb\.F, O\) && M > 64 && 5 \* split_blocks >= int64_t\{6\} \* num_cus\(\);", s,
+         "grouped dx rule")
+    _one(r"const bool split = kF32 && v4 && split_macs\(M, hb\.F, O\);", s, "band split dx rule")
+    _one(r"\(M \+ 63\) / 64 \* chunks >= int64_t\{2\} \* 7 \* num_cus\(\)", s, "mixed 128-row rule")
+    s = _src("mask_estimator.hip")
+    _one(r"kF32 && a\.vec4 && split_macs\(M, 2 \* static_cast<int64_t>\(hm\.F\), H\);", s, "mask backward rule")
+    _one(r"if \(kF32 && split_macs\(M, 2 \* static_cast<int64_t>\(hm\.F\), H\)\) \{", s, "mask forward rule")
+
+
+def test_wide_grouped_tiles_and_rules():
+    """grouped_gemm.hip: waves, stages, tiles and the dispatch rules; mask_mlp.hip's choice of form."""
+    s = _src("grouped_gemm.hip")
+    _one(r"return op == kGgFwd \? 4 : 8; \}", s, "waves")
+    _one(r"constexpr int NW = gg_waves\(OP\), S = NW == 8 \? 4 : 3;", s, "stages")
+    _one(r"constexpr int WB = NW / WA, TB = 4;", s, "B tiles")
+    _one(r"% 256 == 0\) return launch<T, OP, 8, 2>\(a, stream\);\s+return launch<T, OP, 6, 2>\(a, stream\);", s, "tiles")
+    assert bm.gg_tile("dx", 512, 64) == (8, 4, 8, 256, 256) and bm.gg_tile("fwd", 64, 192) == (4, 3, 6, 192, 128)
+    _one(r"const int64_t quarters = groups >= 24 \? 11 : 16;", s, "dx rule")
+    _one(r"return groups \* rows \* in_features >= quarters \* 1024 \* num_cus\(\);", s, "dx rule")
+    _one(r"\(in_features == 192 \|\| in_features == 256\) && 5 \* blocks >= 4 \* rounds \* cus;", s, "dx rule at 192, 256")
+    _one(r"if \(a_cols == 256\) return other >= 6 \* rounds \* cus && rows >= 64;", s, "dW rule, 256 wide")
+    _one(r"\(other >= 6 \* rounds \* cus && rows > 128\) \|\| \(2 \* other >= 9 \* rounds \* cus && rows >= 1400\);", s,
+         "dW rule, 192 wide")
+    _one(r"return other >= 5 \* rounds \* cus && rows \* other >= 2000 \* rounds \* cus;", s, "dW rule, no whole 64s")
+    _one(r"return out_features >= 128 && shape_ok\(", s, "tanh rule")
+    s = _src("mask_mlp.hip")
+    _one(r"if \(dim >= 384\) return true;", s, "two kernels")
+    _one(r"return passes > 2 \* band_count && \(dim >= 256 \|\| rows > \(dim <= 64 \? 768 : 256\)\);", s, "two kernels")
+
+
+def test_matrix_core_gate_rules():
+    s = _src("attn_gate.hip")
+    _one(r"return work >= 4096 \|\| rows >= 16384 \|\| \(rows >= 8192 && work >= 1024\);", s, "forward rule")
+    _one(r"return work >= 1536 \|\| \(work >= 1024 && s\.rows\(\) >= 2000\);", s, "backward rule")
+    _one(r"\(nt <= 4 \|\| nt == 6 \|\| nt == 8\)", s, "dims")
+    assert _const("kGateBwdMaxBlocks", "attn_gate.hip") == 1024
+    _one(r"std::min<int64_t>\(2 \* static_cast<int64_t>\(num_cus\(\)\), kGateBwdMaxBlocks\)", s, "backward blocks")

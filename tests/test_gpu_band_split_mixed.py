@@ -94,6 +94,11 @@ def test_mixed_dw_row_steps(hip_ext, m):
     _case(hip_ext, (8, 124), m, 8, torch.float16, 200 + m)
 
 
+def test_mixed_128_row_tiles(hip_ext):
+    # the input-gradient product on 128-row tiles (from 3584 blocks of 64 rows), the last of 3 rows
+    _case(hip_ext, BSR_WIDTHS, 2307, 64, torch.float16, 35)
+
+
 def test_mixed_empty_batch(hip_ext):
     dims = (8, 16)
     x = torch.empty(0, 24, device="cuda")

@@ -158,3 +158,52 @@ def test_the_final_layers_errors_have_no_sign(hip_ext):
     _, pre = hip_ext.mask_estimator_final_forward_packed(x, torch.cat([w.reshape(-1) for w in ws]), bias, dims)
     want = torch.cat([x[:, b].double() @ w.double().t().contiguous() for b, w in enumerate(ws)], 1)
     assert abs((pre.double() - want).mean().item()) <= 2.0**-28 * want.pow(2).mean().sqrt().item()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan"), 3.4e38])
+def test_values_no_bf16_part_can_hold(hip_ext, bad):
+    """3.4e38 rounds to infinity in bf16.  Row 5 of group 3 holds the value alone: the results are those of an
+    fp32 product, other groups' are untouched, and the block that sums again counts every row of db once."""
+    x, w, dy = (t.cuda() for t in _layer(300, 62, 128, 260, 13))
+    clean = hip_ext.grouped_linear_forward(x, w)
+    dx, dw, db = hip_ext.grouped_linear_backward(dy, x, w, True)
+    x2 = x.clone()
+    x2[5, 3] = 0.0
+    x2[5, 3, 7] = bad
+    out = hip_ext.grouped_linear_forward(x2, w)
+    want = bad * w[3, :, 7]
+    assert torch.equal(torch.isnan(out[5, 3]), torch.isnan(want))
+    assert torch.equal(out[5, 3][~torch.isnan(want)], want[~torch.isnan(want)])
+    others = torch.arange(62) != 3
+    assert torch.equal(out[:, others], clean[:, others])
+    rows = torch.arange(300) != 5
+    assert torch.allclose(out[rows][:, 3], clean[rows][:, 3], rtol=1e-5, atol=1e-5)
+    dy2 = dy.clone()
+    dy2[5, 3, 11] = bad
+    dx2, dw2, db2 = hip_ext.grouped_linear_backward(dy2, x, w, True)
+    cols = torch.arange(260) != 11
+    assert torch.equal(dx2[:, others], dx[:, others]) and torch.equal(dw2[others], dw[others])
+    assert torch.equal(db2[3][cols], db[3][cols]) and torch.equal(db2[others], db[others])
+    assert torch.allclose(dw2[3][cols], dw[3][cols], rtol=1e-4, atol=1e-4)
+    assert bad == 3.4e38 or not torch.isfinite(db2[3, 11])
+
+
+@pytest.mark.parametrize("bad", [float("inf"), 2.0**-125])
+def test_row_norms_of_a_block_that_sums_again(hip_ext, bad):
+    """The band split's forward gathers the rows' squares in its K loop: a weight that sends the block
+    through it twice leaves inv_norm as it was."""
+    m, o, dims = 400, 192, BSR_WIDTHS
+    g = torch.Generator().manual_seed(14)
+    x = torch.randn(m, sum(dims), generator=g).cuda()
+    gamma = (1 + 0.1 * torch.randn(sum(dims), generator=g)).cuda()
+    w = torch.cat([(torch.randn(o, d, generator=g) / d**0.5).reshape(-1) for d in dims]).cuda()
+    b = torch.zeros(len(dims) * o, device="cuda")
+    out, _, inv = hip_ext.band_split_ragged_forward_packed(x, gamma, w, b, dims, write_normed=False)
+    w2 = w.clone()
+    w2[o * sum(dims[:61]) + 3 * dims[61] + 100] = bad  # band 61, output 3
+    out2, _, inv2 = hip_ext.band_split_ragged_forward_packed(x, gamma, w2, b, dims, write_normed=False)
+    assert torch.equal(inv, inv2)
+    assert torch.equal(out[:, :61], out2[:, :61])
+    cols = torch.arange(o) != 3
+    assert torch.allclose(out[:, 61][:, cols], out2[:, 61][:, cols], rtol=1e-4, atol=1e-5)
+    assert bad < 1 or not torch.isfinite(out2[:, 61, 3]).any()

@@ -1,10 +1,13 @@
-"""fp32 products from bf16 parts (gemm.h): as exact as the fp32 sums, and unchanged for what bf16 parts
-cannot hold.
+"""fp32 products (gemm.h): as exact as the fp32 sums, also for what three bf16 parts cannot hold.
+
+Most of these sizes are below gemm.h's rule for the split into bf16 parts and run the fp32 matrix
+instructions, whose results the split has to match; test_gpu_fp32_routes.py asks the same of sizes that
+are split.
 
 * Error against 64 bits, at the sizes where the K loop can go wrong (one partial chunk, several), no
   larger than sqrt(K) / 2 rounding errors of the fp32 sum: 2^-24 (1 + sqrt(K) / 2) of the result's RMS
-  times sqrt(2), measured 0.3 of it.
-* Values over the whole range of an fp32 exponent: the parts follow the exponent.
+  times sqrt(2), measured 0.8 of it (0.3 split).
+* Exponents from -60 to 60 (test_gpu_fp32_routes.py: from 2^-124).
 * An infinity, a NaN, a value above bf16's largest, an overflow: the results of a plain fp32 product.
 """
 

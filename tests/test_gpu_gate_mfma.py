@@ -1,6 +1,8 @@
-"""GPU parity of the 16-bit attention gate on the matrix cores (dim a multiple of 64): groups of 16 and 32
-tokens that end anywhere, every head count and pack width of the fast path, every dim it is built for, and
-more groups than blocks (several turns of the double-buffered backward, the last one partial)."""
+"""GPU parity of the 16-bit attention gate at dims that are a multiple of 64: groups of 16 and 32 tokens that
+end anywhere, every head count and pack width of the fast path, every dim the matrix-core kernels are built
+for, and more groups than blocks (several turns of the double-buffered backward, the last one partial).
+Which of them run the matrix cores, each way, is decided by heads x dim and tokens; test_gpu_routes.py has
+the cases on both sides."""
 
 from __future__ import annotations
 
@@ -42,3 +44,19 @@ def test_infinities_stay_in_their_token(hip_ext):
     keep = torch.ones(d, dtype=torch.bool)
     keep[5] = False
     assert torch.equal(gw1[:, keep], gw2[:, keep]) and torch.isinf(gw2[:, 5]).all()
+
+
+def test_infinities_stay_in_their_token_at_many_products(hip_ext):
+    """The same at heads x dim of 4096, where the forward runs the matrix cores at any number of tokens."""
+    m, h, dh, d = 70, 8, 64, 512
+    g = torch.Generator().manual_seed(64)
+    attn = torch.randn(m, h, dh, generator=g).to(torch.bfloat16).cuda()
+    x = torch.randn(m, d, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(h, d, generator=g) / d**0.5).to(torch.bfloat16).cuda()
+    b = torch.zeros(h, dtype=torch.bfloat16, device="cuda")
+    x2 = x.clone()
+    x2[69, 5] = float("inf")
+    o1, g1, *_ = hip_ext.attention_gate_forward(attn, x, w, b)
+    o2, g2, *_ = hip_ext.attention_gate_forward(attn, x2, w, b)
+    assert torch.equal(o1[:69], o2[:69]) and torch.equal(g1[:69], g2[:69])
+    assert torch.equal(g2[69], (w[:, 5] > 0).to(torch.bfloat16))

@@ -1,6 +1,9 @@
-"""GPU parity: the grouped linear's backward products on the 256-wide tiles of grouped_gemm.hip, at the
-edges of its tiles: one and several K chunks (the ring is 4 deep, the loop unrolled by two), rows and
-widths that end inside a tile, a row count that is no multiple of 32 (dW's first K chunk is partial)."""
+"""GPU parity: the grouped linear's backward products at more than 192 inputs and its tanh forward.
+
+The backward cases are small grids, which the dispatch gives to the kernels with narrower blocks (all but
+the dx of the case with 60 groups); the 256-wide tiles of grouped_gemm.hip are taken from the grid sizes
+of test_gpu_routes.py, which holds the cases at their edges.  The tanh forward and the two-kernel mask MLP
+run grouped_gemm.hip here."""
 
 from __future__ import annotations
 
@@ -16,12 +19,12 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,groups,i,o", [
     (1, 3, 512, 32),       # one row, one K chunk
-    (31, 2, 512, 64),      # dW below its 32 rows: the register-staged kernel
+    (31, 2, 512, 64),      # dW below 32 rows: the register-staged kernel
     (32, 5, 384, 96),      # one dW K chunk
-    (63, 2, 320, 160),     # a second tile of 128 of its 192 columns; dW chunk 0 with one row
-    (257, 3, 264, 264),    # a tile of 8 columns, a tile of one row; O no multiple of 32: dx elsewhere
-    (150, 2, 768, 2048),   # three 256-wide tiles, 64 K chunks
-    (513, 62, 192, 256),   # dW from 192 inputs on
+    (63, 2, 320, 160),     # dW chunk 0 with one row
+    (257, 3, 264, 264),    # widths in whole eights, a tile of one row
+    (150, 2, 768, 2048),   # a long K
+    (513, 62, 192, 256),   # glin_dx and the DMA dW at 192 inputs
     (129, 4, 256, 512),
 ])
 def test_wide_grouped_backward(hip_ext, dtype, m, groups, i, o):
@@ -80,7 +83,7 @@ def test_tanh_of_every_pattern(hip_ext, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("m,groups,i,o", [
-    (1, 3, 32, 8),         # one row, one K chunk, one unit of outputs
+    (1, 3, 32, 8),         # one row, one K chunk, one unit of outputs: the register-staged kernel
     (127, 2, 64, 256),     # two chunks
     (129, 5, 96, 384),     # a second row tile of one row; 192-wide output tiles
     (260, 3, 160, 264),    # five chunks, an output tile that ends after 72 of 192

@@ -185,3 +185,31 @@ def test_capture_of_the_one_pass_after_a_two_kernel_warm_up(hip_ext):
     run = subprocess.run([sys.executable, "-c", _CAPTURE_AFTER_WARM_UP], cwd=Path(__file__).resolve().parents[1],
                          capture_output=True, text=True, timeout=100)
     assert run.returncode == 0 and "captured" in run.stdout, run.stderr[-2000:]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [384, 512])
+def test_one_pass_with_the_hidden_layer_at_wide_dims(hip_ext, dtype, dim):
+    """A first bias that is not 8-byte aligned keeps dims 384 and 512 on the one pass, with the hidden layer
+    stored and with the mask product: the bits of the aligned call."""
+    dims, hidden, batch, frames, stems, channels = (8, 64, 132), 160, 2, 35, 2, 2
+    m, nb, total = batch * frames, len(dims), sum(dims)
+    g = torch.Generator().manual_seed(65)
+    x = torch.randn(m, nb, dim, generator=g).to(dtype).cuda()
+    w1 = (torch.randn(nb, hidden, dim, generator=g) / dim**0.5).to(dtype).cuda()
+    b1 = (0.1 * torch.randn(nb * hidden + 1, generator=g)).to(dtype).cuda()[1:].view(nb, hidden)
+    w2 = (torch.randn(2 * total * hidden, generator=g) / hidden**0.5).to(dtype).cuda()
+    b2 = (0.1 * torch.randn(2 * total, generator=g)).to(dtype).cuda()
+    spec = torch.view_as_complex(torch.randn(batch, total // 2, frames, 2, generator=g)).cuda()
+
+    def apply(bias):
+        est = torch.zeros(batch * stems * channels, total // 2 // channels, frames, dtype=torch.complex64, device="cuda")
+        pre, hid = hip_ext.mask_mlp_forward_apply(x, w1, bias, w2, b2, dims, spec, est, 1, channels, save_hidden=True)
+        return pre, hid, torch.view_as_real(est)
+
+    for call in (lambda b: hip_ext.mask_mlp_forward(x, w1, b, w2, b2, dims, save_hidden=True), apply):
+        one, names = launched(lambda: call(b1))
+        assert "mlp_fwd_kernel" in names and "gg_kernel" not in names
+        two, names = launched(lambda: call(b1.clone()))
+        assert "gg_kernel" in names
+        assert all(torch.equal(a, b) for a, b in zip(one, two))

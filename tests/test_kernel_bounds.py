@@ -136,3 +136,87 @@ def test_grouped_dx_row_tiles_stay_in_bounds():
     for rb in range(16, 193, 16):
         assert not replay(1032, 62, rb), rb
     assert replay(1032, 62, 200) and replay(1032, 62, 208)
+
+
+@pytest.mark.parametrize("op,G,I,O,M", [
+    ("dx", 62, 512, 32, 91), ("dx", 62, 264, 1056, 257), ("dx", 60, 192, 96, 2601), ("dx", 62, 768, 96, 61),
+    ("dw", 62, 512, 1024, 64), ("dw", 60, 768, 1032, 65), ("dw", 62, 384, 1536, 161), ("dw", 62, 264, 1056, 416),
+    ("fwd", 1, 96, 264, 1), ("fwd", 5, 64, 128, 300), ("fwd", 62, 512, 2048, 129),
+])
+def test_wide_grouped_products_stay_in_bounds(op, G, I, O, M):
+    """gg_kernel at the edges of its tiles; each product writes its result to the last byte."""
+    assert {"dx": bm.wide_dx_supported, "dw": bm.wide_dw_supported, "fwd": bm.wide_tanh_supported}[op](G, I, O, M, 2)
+    b = bm.Bounds({"x": M * G * I * 2, "weight": G * O * I * 2, "dy": M * G * O * 2, "dx": M * G * I * 2,
+                   "dw": G * O * I * 2, "db": G * O * 2, "out": M * G * O * 2, "bias": G * O * 2})
+    bm.replay_gg(op, G, I, O, M, bnd=b)
+    assert not b.violations(), b.violations()
+    out = {"dx": "dx", "dw": "dw", "fwd": "out"}[op]
+    assert b.lo[out] == 0 and b.hi[out] == b.sizes[out]
+    for short in (out, "dy" if op != "fwd" else "x", "weight" if op != "dw" else "x"):
+        b.sizes[short] -= 2
+        assert any(v.startswith(short + ":") for v in b.violations()), short
+        b.sizes[short] += 2
+
+
+def test_replay_flags_a_wrong_transposed_swizzle(monkeypatch):
+    """A swizzle that leaves its aligned group of units is caught in each kernel that reads transposed."""
+    monkeypatch.setattr(bm, "swz_mn_p", lambda pitch, k: 64 * (k & 1))
+    assert bm.replay_band_split_backward([512] * 62, 1896, 2048, 2, grouped=True).violations()
+    assert bm.replay_band_split_backward([192] * 62, 1032, 768, 4, grouped=True).violations()
+    assert bm.replay_attention_gate(124, 948, 8, 64, 512, 2).violations()
+
+
+@pytest.mark.parametrize("br,bc,wr,tr_a,tr_b", [
+    (64, 64, 4, False, False), (128, 64, 4, False, False), (192, 64, 4, False, False), (256, 64, 4, False, False),
+    (64, 64, 4, True, False), (64, 128, 2, True, False), (64, 64, 2, True, True), (64, 128, 2, True, True),
+    (128, 128, 1, False, False), (128, 64, 2, True, False), (128, 64, 2, True, True),
+])
+def test_split_fp32_tiles_stay_in_their_regions(monkeypatch, br, bc, wr, tr_a, tr_b):
+    """Every tile of the split fp32 kernels: three planes an operand, and the second run's fp32 rows."""
+    b = bm.Bounds({})
+    bm.split_tile_lds(b, br, bc, wr, tr_a, tr_b)
+    assert not b.violations(), b.violations()
+    assert b.hi["lds_split_a"] == 3 * br * 64 and b.hi["lds_split_b"] == 3 * bc * 64
+    monkeypatch.setattr(bm, "SPLIT_ROW", 47)  # a float a row less than three planes need
+    b = bm.Bounds({})
+    bm.split_tile_lds(b, br, bc, wr, tr_a, tr_b)
+    assert b.violations()
+
+
+def test_fp32_split_is_replayed_on_both_sides_of_its_rules():
+    """The split's larger tiles (128-row dx, 128-column dW) and LDS are replayed where the rules choose
+    them, the plain fp32 tiles elsewhere."""
+    lds = lambda M, I, O, G: bm.replay_band_split_backward([I] * G, M, O, 4, grouped=True)  # noqa: E731
+    large, small = lds(1032, 192, 768, 62), lds(130, 64, 256, 62)
+    assert not large.violations() and not small.violations()
+    assert "lds_split_a" in large.sizes and "lds_split_a" not in small.sizes
+    assert large.sizes["lds"] == (64 + 128) * 48 * 4 + 5 * 128 * 4 and small.sizes["lds"] == 2 * 128 * 33 * 4 + 5 * 64 * 4
+    fwd = bm.replay_band_split_forward([192] * 62, 1032, 768, 4, norm=False)
+    assert fwd.sizes["lds"] == (256 + 64) * 48 * 4 + 256 and not fwd.violations()
+    for M in (98, 99, 130, 131):  # either side of 0.3 G multiply-adds, and of dx's full 128-row tiles
+        assert not lds(M, 192, 256, 62).violations(), M
+        assert not bm.replay_band_split_backward(bm.BSR_WIDTHS, 4 * M, 192, 4).violations(), M
+        assert not bm.replay_mask_final_backward(bm.BSR_WIDTHS, M, 256, 4).violations(), M
+
+
+def test_mixed_band_split_128_row_tiles_stay_in_bounds():
+    for M in (2240, 2304, 2307):  # 62 bands: 101 chunks; from two rounds of seven 64-row blocks a CU
+        reps = dict(bm.replay_band_split_mixed(bm.BSR_WIDTHS, M, 64))
+        assert not reps["band_split_mixed_bwd_gemm"].violations(), M
+        assert reps["band_split_mixed_bwd_gemm"].hi["dx"] == M * 4100 * 2
+
+
+@pytest.mark.parametrize("B,N,H,Dh,dim", [
+    (1, 1, 8, 64, 512), (1, 33, 16, 32, 256), (47, 1, 8, 64, 384), (3, 2731, 8, 64, 256), (1, 16421, 2, 64, 64),
+    (5, 401, 8, 16, 128), (1, 15, 8, 64, 192), (124, 948, 8, 64, 512),
+])
+def test_matrix_core_gate_stays_in_bounds(B, N, H, Dh, dim):
+    b = bm.replay_attention_gate(B, N, H, Dh, dim, 2)
+    assert not b.violations(), b.violations()
+    forward, backward = "lds_w" in b.sizes, "lds_x" in b.sizes
+    assert forward or backward
+    for buf in ("out", "gate") * forward + ("grad_x", "grad_attn", "x") * backward:
+        assert b.hi[buf] == b.sizes[buf], buf
+        b.sizes[buf] -= 2
+        assert any(v.startswith(buf + ":") for v in b.violations()), buf
+        b.sizes[buf] += 2
