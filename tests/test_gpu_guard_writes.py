@@ -246,3 +246,28 @@ def test_train_path_ops_write_inside_their_outputs(hip_ext, guarded, dtype):
     hip_ext.band_rows_scatter(yr.float(), plan)
     hip_ext.band_rows_scatter(yr.float(), plan, mean=True)
     assert not guarded.damaged(), "mel band rows"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("shape", [(161, 62, 384, 1536), (65, 60, 768, 1032), (416, 62, 264, 1056), (130, 62, 192, 256),
+                                   (300, 62, 100, 260)])
+def test_large_grouped_linear_writes_inside_its_outputs(hip_ext, guarded, dtype, shape):
+    """The sizes that run the wide tiles (16 bits) and the split products (fp32), with tiles, K chunks and
+    columns that end early."""
+    test_grouped_linear_writes_inside_its_outputs(hip_ext, guarded, dtype, shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,heads,dh,dim", [(33, 16, 32, 256), (8193, 8, 64, 256), (16421, 2, 64, 64), (2001, 8, 16, 128)])
+def test_matrix_core_gate_writes_inside_its_outputs(hip_ext, guarded, m, heads, dh, dim):
+    g = torch.Generator().manual_seed(6)
+    attn = torch.randn(m, heads, dh, generator=g).bfloat16().cuda()
+    x, w = torch.randn(m, dim, generator=g).bfloat16().cuda(), torch.randn(heads, dim, generator=g).bfloat16().cuda()
+    b = torch.randn(heads, generator=g).bfloat16().cuda()
+    gout = torch.randn(m, heads * dh, generator=g).bfloat16().cuda()
+    print(f"[guard] matrix-core gate {m} {heads} {dh} {dim}", flush=True)
+    _, gate, sa, sx = hip_ext.attention_gate_forward(attn, x, w, b)
+    assert not guarded.damaged(), "attention_gate_forward"
+    hip_ext.attention_gate_backward(gout, sa, sx, w, gate)
+    assert not guarded.damaged(), "attention_gate_backward"
