@@ -600,9 +600,9 @@ inline bool split_macs(int64_t rows, int64_t in_features, int64_t out_features) 
   return rows * in_features >= (kSplitMacs + out_features - 1) / out_features;
 }
 
-// The K loop of a SPLIT kernel: one LDS tile, the next chunk's loads in registers while this one is multiplied (the
-// blocks of a CU, two to six of them, cover each other's splits and barriers).  SPLIT: three bf16 planes
-// and six products; else the fp32 MFMAs.
+// The K loop of a SPLIT kernel: one LDS tile, the next chunk's loads in registers while this one is
+// multiplied (the blocks of a CU, two to six of them, cover each other's splits and barriers).  SPLIT:
+// three bf16 planes and six products; else the fp32 MFMAs.
 template <int BR, int BC, int WR, int WC, bool SPLIT, class LA, class LB>
 __device__ __forceinline__ void gemm_f32_loop(LA& la, LB& lb, int K, float* lds,
                                               f32x4_t (&acc)[TileShape<BR, BC, WR, WC>::kTR]

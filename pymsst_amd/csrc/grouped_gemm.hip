@@ -441,7 +441,8 @@ bool wide_tanh_supported(int64_t groups, int64_t in_features, int64_t out_featur
   // register-staged kernel takes 7.8 us at 31 rows and 28 at 1896 (62 groups of 64 -> 128), this one 7.7 and
   // 20, and it stays ahead from one row and one group on (one group of 512 -> 2048, one row: 20 and 13 us;
   // 62 groups of 192 -> 768, 31 rows: 15.5 and 11.0).
-  return out_features >= 128 && shape_ok(groups, in_features, out_features, rows, elem) && in_features % 32 == 0 && groups > 0 &&
+  return out_features >= 128 && shape_ok(groups, in_features, out_features, rows, elem) &&
+         in_features % 32 == 0 && groups > 0 &&
          x != nullptr && w != nullptr && out != nullptr && in_features > 0 && out_features > 0 &&
          256 * in_features * 2 < (int64_t{1} << 31) && aligned16(x) && aligned16(w) && aligned16(out) &&
          bias != nullptr && reinterpret_cast<uintptr_t>(bias) % 8 == 0;
